@@ -84,6 +84,11 @@ constexpr int kPicGMax = 64;        // cells per push/count group (LDS tables; t
 constexpr int kPushWaves = 4;
 constexpr int kXMove = 8;           // move_block threads per push/count block boundary
 constexpr int kBatch = 2;           // chunks of 64 particles fetched per memory round trip
+// pic_push_group: waves per group, and chunks of 64 particles each holds in
+// registers across the group's counts.  8 x 3 chunks hold 1,536 particles,
+// half as many again as a group aims at.
+constexpr int kMcWaves = 8;
+constexpr int kMcHold = 3;
 // pic_push_cell's LDS rows (dynamic shared memory): one pushed 64-particle
 // chunk each (id, move and rank, frac, ux, uy, uz), xr rows for each of a
 // wave's two cells; at most 8 in FP32, 4 in FP64 (about 96 KiB per workgroup)

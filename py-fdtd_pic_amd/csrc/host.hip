@@ -32,7 +32,7 @@ template <typename R>
 hipError_t launch_energy(const EnergyJob<R>* jobs, int n, hipStream_t st);
 template <typename R>
 hipError_t launch_push(const SimDev<R>* sims, const BeamDev<R>* beams, const int2* cell_items, int ncell,
-                       const int2* group_items, int ngroup, long long launch_idx, int xr, int single, hipStream_t st,
+                       const int2* group_items, int ngroup, bool coop, long long launch_idx, int xr, int single, hipStream_t st,
                        hipEvent_t e0, hipEvent_t e1);
 template <typename R>
 hipError_t launch_scatter(const SimDev<R>* sims, const BeamDev<R>* beams, const int2* scatter_blocks,
@@ -616,17 +616,22 @@ static int attach_t(fdtd_ctx* c, int id, SimHost& s, const fdtd_beam_desc_t* bd)
     // live range (cells of the particles; all live at attach)
     b->range0[0] = b->cell0.front();
     b->range0[1] = b->cell0.back();
-    // cells per push/count group; a wave loops over groups of the live range
-    // in a grid stride.  Dense beams (>= 96 particles per occupied cell) take
-    // one-cell groups (the scalar-carry path); sparser ones groups of about
-    // 1,024 particles, which amortise the per-group work of the multi-cell
-    // path (measured on config 4's 2,048 beams: push/count 1.17 ms per step
-    // at ~96 particles per group, 0.85 ms with this rule; config 3, 100 per
-    // cell: 13.0 us at one cell per group, 16.9 us at four)
+    // Cells per push/count group; the kernels loop over the groups of the live
+    // range in a grid stride.  G fixes the order of the deposit's sums, so it
+    // depends on the beam alone.  Dense beams take one-cell groups (the
+    // scalar-carry path), sparser ones groups of about 1,024 particles, which
+    // amortise the per-group work of the multi-cell path (config 4's 2,048
+    // beams: push/count 1.17 ms per step at ~96 particles per group, 0.85 ms
+    // with this rule).  FP32 from 96 particles per occupied cell (config 3,
+    // 100 per cell: 13.0 us at one cell per group, 16.9 us at four).  FP64 from
+    // 40: us per step, one cell per group against groups of 1,024, 45 per cell:
+    // 1 beam 10.8 / 16, 24 beams 38 / 57, 200 beams 328 / 286; 57 per cell: 1
+    // beam 11.2 / 16, 64 beams 70 / 88, 200 beams 233 / 234; below 40 it loses
+    // from 24 beams on (27 per cell 48.5 / 47).
     int G = bd->group;
     if (G <= 0) {
         const double per_cell = occupied ? (double)n / occupied : 1.0;
-        G = per_cell >= 96.0 ? 1 : (int)std::lround(1024.0 / per_cell);
+        G = per_cell >= kOneCellDensity<R> ? 1 : (int)std::lround(1024.0 / per_cell);
     }
     b->G = std::min(std::max(G, 1), kPicGMax);
     const int span = b->range0[1] - b->range0[0] + 3;
@@ -745,6 +750,9 @@ static int rebuild_t(fdtd_ctx* c) {
         // for the staged movers and the parked particles
         for (int k = 0; k < bh->nnode + bh->nmove; ++k) pblocks.push_back(make_int2(bi, -(k + 1)));
     }
+    // small launches of multi-cell beams give each group a workgroup (the
+    // results are the same bits either way)
+    c->mc_coop = (long long)pitems.size() <= kCoopGroupsPerCu<R> * std::max(c->cu_count, 1);
     while (pitems.size() % kPushWaves) pitems.push_back(make_int2(-1, 0));   // whole push/count workgroups
     c->has_pic = !bdev.empty();
     c->npnode = (int)pblocks.size();
@@ -1056,10 +1064,10 @@ int fdtd_run(fdtd_ctx* c, int64_t nsteps) {
                                                  std::to_string(c->launch_idx) + ": " + hipGetErrorString(stale));
             hipError_t e = c->prec == FDTD_F64
                 ? launch_push<double>((const SimDev<double>*)c->d_sims, (const BeamDev<double>*)c->d_beams,
-                                      c->d_pitems + c->npitems, c->npcell, c->d_pitems, c->npitems,
+                                      c->d_pitems + c->npitems, c->npcell, c->d_pitems, c->npitems, c->mc_coop,
                                       c->launch_idx, c->pc_xr, c->pc_single, c->st, e0, e1)
                 : launch_push<float>((const SimDev<float>*)c->d_sims, (const BeamDev<float>*)c->d_beams,
-                                     c->d_pitems + c->npitems, c->npcell, c->d_pitems, c->npitems,
+                                     c->d_pitems + c->npitems, c->npcell, c->d_pitems, c->npitems, c->mc_coop,
                                      c->launch_idx, c->pc_xr, c->pc_single, c->st, e0, e1);
             if (e != hipSuccess)
                 return fdtd_fail(FDTD_E_HIP, std::string("push/count launch ") + std::to_string(c->launch_idx) +

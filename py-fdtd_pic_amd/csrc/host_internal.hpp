@@ -100,6 +100,7 @@ struct fdtd_ctx {
     size_t d_pitems_cap = 0;                 // index), then npcell one-cell workgroups (beam, workgroup)
     int npblocks = 0, npitems = 0, npcell = 0;
     int npnode = 0;                          // scatter blocks: npnode node blocks, then particle blocks
+    bool mc_coop = false;                    // the multi-cell items run one workgroup each (pic_push_group)
     bool has_pic = false;                    // some active simulation carries a beam
     bool fuse_pic = true;                    // scatter in the same launch as the last tile group's field step
     // bound on queued work: an event every kThrottleEvery launches; the host
@@ -126,6 +127,21 @@ struct fdtd_ctx {
 };
 
 int fdtd_fail(int code, const std::string& msg);
+
+// Particles per occupied cell from which a beam takes one-cell groups (see
+// attach_t).
+template <typename R>
+constexpr double kOneCellDensity = sizeof(R) == 4 ? 96.0 : 40.0;
+
+// Groups per CU up to which a launch's multi-cell beams take pic_push_group
+// (a workgroup per group) rather than pic_push_count (a wave per group): two
+// workgroups of it fit on a CU in FP32, one in FP64.  us per step, group
+// against wave, beams of 40,000 particles over 1,500 cells (39 groups each):
+// FP32 1 beam 14.2 / 35.9, 24 beams 29.6 / 41.2, 32 beams 38.1 / 47.9, and at
+// 200 beams 231 / 203; FP64 1 beam 16.1 / 43.1, 16 beams 41.0 / 48.5, 24 beams
+// 46.9 / 49.7, 200 beams 431 / 288.
+template <typename R>
+constexpr long long kCoopGroupsPerCu = sizeof(R) == 4 ? 6 : 4;
 
 // Largest field launch (tiles) that takes the particle scatter into its grid.
 constexpr int kFuseMaxTiles = 2048;

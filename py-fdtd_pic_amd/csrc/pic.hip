@@ -13,14 +13,14 @@ namespace fdtd {
 //
 // Push/count of one step: the one-cell beams' kernel (one item per
 // workgroup) and the multi-cell beams' kernel (one item per wave, padded to
-// whole workgroups), e0 at the start of the first launch, e1 at the end of
+// whole workgroups; coop: one workgroup per item, pic_push_group), e0 at the start of the first launch, e1 at the end of
 // the last.
 // xr: LDS rows per cell of the one-cell kernel (1 .. kPushCellMaxRows);
 // single: the one-cell items' beam when they all belong to one (items
 // (single, 0 .. ncell-1)), else -1.
 template <typename R>
 hipError_t launch_push(const SimDev<R>* sims, const BeamDev<R>* beams, const int2* cell_items, int ncell,
-                       const int2* group_items, int ngroup, long long launch_idx, int xr, int single, hipStream_t st,
+                       const int2* group_items, int ngroup, bool coop, long long launch_idx, int xr, int single, hipStream_t st,
                        hipEvent_t e0, hipEvent_t e1) {
     const bool ev = e0 || e1;
     if (ncell > 0) {
@@ -50,7 +50,13 @@ hipError_t launch_push(const SimDev<R>* sims, const BeamDev<R>* beams, const int
     if (ngroup > 0) {
         const int nb = (ngroup + kPushWaves - 1) / kPushWaves;    // items are padded to whole blocks
         hipEvent_t a0 = ncell > 0 ? nullptr : e0, a1 = e1;
-        if (ev)
+        if (coop && ev)
+            hipExtLaunchKernelGGL((pic_push_group<R>), dim3(ngroup), dim3(64 * kMcWaves), 0, st, a0, a1, 0, sims,
+                                  beams, group_items, launch_idx);
+        else if (coop)
+            hipLaunchKernelGGL((pic_push_group<R>), dim3(ngroup), dim3(64 * kMcWaves), 0, st, sims, beams,
+                               group_items, launch_idx);
+        else if (ev)
             hipExtLaunchKernelGGL((pic_push_count<R>), dim3(nb), dim3(64 * kPushWaves), 0, st, a0, a1, 0, sims,
                                   beams, group_items, launch_idx);
         else
@@ -78,9 +84,10 @@ hipError_t launch_scatter(const SimDev<R>* sims, const BeamDev<R>* beams, const 
 }
 
 template hipError_t launch_push<double>(const SimDev<double>*, const BeamDev<double>*, const int2*, int,
-                                        const int2*, int, long long, int, int, hipStream_t, hipEvent_t, hipEvent_t);
+                                        const int2*, int, bool, long long, int, int, hipStream_t, hipEvent_t,
+                                        hipEvent_t);
 template hipError_t launch_push<float>(const SimDev<float>*, const BeamDev<float>*, const int2*, int, const int2*,
-                                       int, long long, int, int, hipStream_t, hipEvent_t, hipEvent_t);
+                                       int, bool, long long, int, int, hipStream_t, hipEvent_t, hipEvent_t);
 template hipError_t launch_scatter<double>(const SimDev<double>*, const BeamDev<double>*, const int2*, int,
                                            long long, hipStream_t, hipEvent_t, hipEvent_t);
 template hipError_t launch_scatter<float>(const SimDev<float>*, const BeamDev<float>*, const int2*, int, long long,

@@ -719,6 +719,281 @@ __global__ __launch_bounds__(64 * kPushWaves) void pic_push_count(const SimDev<R
     }
 }
 
+// ---- multi-cell groups, one workgroup each ----
+
+// One chunk of a multi-cell group in registers.
+template <typename R>
+struct McChunk {
+    int c, id;
+    R f, ux, uy, uz;
+};
+template <typename R>
+__device__ __forceinline__ void mc_load(gptr<const int32_t> cell, gptr<const int32_t> pid, gptr<const R> pf,
+                                        gptr<const R> px, gptr<const R> py, gptr<const R> pz, int base, int np,
+                                        int lane, McChunk<R>& m) {
+    const unsigned i = (unsigned)min(base + lane, np - 1);
+    m.c = ldo(cell, i);
+    m.id = ldo(pid, i);
+    m.f = ldo(pf, i); m.ux = ldo(px, i); m.uy = ldo(py, i); m.uz = ldo(pz, i);
+}
+
+// One pushed particle of a one-pass group, waiting in registers for the
+// group's totals: its state, new cell, group cell (-1: none), move and rank.
+template <typename R>
+struct McHeld {
+    Pushed<R> s;
+    int c, k, d, r;
+};
+
+// Counting pass over one chunk of a group's run (particles base ..
+// base+63, those below phi): the moves, the counts and
+// the CIC sums; HOLD keeps the pushed particle and its rank, and puts the
+// sums of the run's first cell (group cell first) into Sf, chunk by chunk.
+template <typename R, bool HOLD>
+__device__ __forceinline__ void grp_count(const PushArgs<R>& pa, const R* Et, const R* Ht, int g0,
+                                          const McChunk<R>& cb, int base, int phi, int lane,
+                                          int (&cnt)[kPicGMax + 1][3], double (&Sl)[kPicGMax + 1][4], int first,
+                                          double (&Sf)[4], McHeld<R>& h) {
+    const int i = base + lane;
+    const int c_old = i < phi ? cb.c : 0x7fffffff;
+    const Chunk k = chunk_info(c_old, i, phi, lane);
+    int c = c_old, d = 0, off = 1;
+    R f = cb.f, ux = cb.ux, uy = cb.uy, uz = cb.uz;
+    R a0 = R(0), a1 = R(0);
+    if (k.valid) push_tab<R>(pa, Et, Ht, g0, c, f, ux, uy, uz, d, off, a0, a1);
+    const unsigned long long seg = lanes_le(lane) & ~lanes_lt(k.fl);
+    const unsigned long long bd0 = __ballot(k.valid && d == -1);
+    const unsigned long long bd1 = __ballot(k.valid && d == 0);
+    const unsigned long long bd2 = __ballot(k.valid && d == 1);
+    if (HOLD && k.valid) {
+        const unsigned long long mine = d < 0 ? bd0 : (d == 0 ? bd1 : bd2);
+        h.k = c_old - g0;
+        h.d = d;
+        h.r = cnt[h.k][d + 1] + __popcll(mine & lanes_lt(lane) & ~lanes_lt(k.fl));
+        h.c = c;
+        h.s.id = cb.id;
+        h.s.f = f; h.s.ux = ux; h.s.uy = uy; h.s.uz = uz;
+    }
+    // the chunk's segment sums of the weights onto nodes c-1+off,
+    // c+off, in R (FP32: at most 64 weights, then added into the
+    // FP64 cell sums in a fixed order)
+    R v[4];
+    v[0] = off == 0 ? a0 : R(0);
+    v[1] = off == 0 ? a1 : (off == 1 ? a0 : R(0));
+    v[2] = off == 1 ? a1 : (off == 2 ? a0 : R(0));
+    v[3] = off == 2 ? a1 : R(0);
+    seg_scan4<R>(v, lane, k.fl);
+    const int lk = k.valid ? c_old - g0 : -1;
+    if (k.valid && k.last) {
+        cnt[lk][0] += __popcll(bd0 & seg);
+        cnt[lk][1] += __popcll(bd1 & seg);
+        cnt[lk][2] += __popcll(bd2 & seg);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            if (HOLD && lk == first) Sf[w] = (double)v[w];
+            else Sl[lk][w] += (double)v[w];
+        }
+    }
+    wave_sync();
+}
+
+// Push, counts, CIC sums and the new state of the multi-cell beams of a small
+// launch: one workgroup of kMcWaves waves per group of G cells (grid-stride).
+//
+// Bound: the dependent chain of one group (its loads, then its chunks one
+// after the other).  The group's chunks of 64 particles are dealt out in
+// contiguous runs, one run per wave, and each wave holds its pushed particles
+// in registers until the group's totals are known, so a particle is pushed
+// once and a group of ~1,024 particles is 2 chunks deep instead of the 2 x 16
+// of pic_push_count.  A step of a lone beam of 40,000 particles over 1,500
+// cells took 35.9 us in FP32 and 43.1 us in FP64 with pic_push_count and takes
+// 14.2 and 16.1 us with this kernel; 8 x 3 chunks per group leave FP32 four
+// waves per SIMD and FP64 three.
+//
+// Counts, ranks and sums: each wave keeps tables of its own run (LDS); after
+// the barrier the threads add the waves' counts into the group's totals and
+// leave in each wave's table the counts of the waves before it, which the
+// wave adds to its ranks.  The sums are added in the order of the chunks, as
+// one wave going through the group adds them: a cell that begins in a run is
+// summed there from zero; the run's first cell, which earlier runs may have
+// begun, keeps each chunk's part to itself (Sf) to be added after theirs.  So
+// the results are those of pic_push_count bit for bit, and the choice between
+// the two may follow the load of the launch.
+// A group of more than kMcWaves * kMcHold chunks (a group size given by the
+// caller, or a beam that bunched) is done by one wave in two passes: a
+// counting pass, then the same pushes again with the ranks.  It is one wave
+// because the second pass reads the old buffer while it stages movers there.
+template <typename R>
+constexpr int kMcOcc = sizeof(R) == 4 ? 4 : 3;      // waves per SIMD asked of the register allocator
+template <typename R>
+__global__ __launch_bounds__(64 * kMcWaves, kMcOcc<R>) void pic_push_group(const SimDev<R>* __restrict__ sims,
+                                                                           const BeamDev<R>* __restrict__ beams,
+                                                                           const int2* __restrict__ items,
+                                                                           long long launch_idx) {
+    __shared__ int cnt_all[kMcWaves][kPicGMax + 1][3];     // per wave: down, stay, up per group cell (rank carry)
+    __shared__ double S_all[kMcWaves][kPicGMax + 1][4];    // per wave: J' sums onto nodes c-1 .. c+2
+    __shared__ double Sf_all[kMcWaves][kMcHold][4];        // per wave and chunk: the sums of the run's first cell
+    __shared__ int first_all[kMcWaves];                    // per wave: the run's first group cell (-1: none)
+    __shared__ int tot[kPicGMax + 1][3];                   // the group's totals
+    __shared__ int stl[kPicGMax + 2];                      // start[] of the group's cells g0 .. g1
+    __shared__ R Et[kPicGMax + 3], Ht[kPicGMax + 3];       // the group's E and averaged H (stage_fields)
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int (&cnt)[kPicGMax + 1][3] = cnt_all[wv];
+    double (&Sl)[kPicGMax + 1][4] = S_all[wv];
+    // wave-uniform by construction: the item and the descriptors come in
+    // through scalar loads
+    const int2 it = items[blockIdx.x];
+    if (it.x < 0) return;
+    const cref<BeamDev<R>> b = ((cptr<BeamDev<R>>)beams)[it.x];
+    const cref<SimDev<R>> sd = ((cptr<SimDev<R>>)sims)[b.sim];
+    const int par = (int)((launch_idx - b.launch_begin) & 1);
+    const int po = par ^ 1;
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int N = b.N, np = b.np, nwg = b.nwaves;
+    const int G = max(2, min(b.G, kPicGMax));
+    const PushArgs<R> pa{gp((const R*)sd.E[par]), gp((const R*)sd.H[par]), gp((const R*)sd.H[par ^ 1]),
+                         b.a, b.jscale, b.Sc, N};
+    const gptr<const int32_t> rng_p = gp((const int32_t*)b.range[par]);
+    const gptr<const int32_t> st = gp((const int32_t*)b.start[par]);
+    const gptr<const int32_t> cell = gp((const int32_t*)b.cell[par]), pid = gp((const int32_t*)b.id[par]);
+    const gptr<const R> pf = gp((const R*)b.frac[par]), px = gp((const R*)b.ux[par]);
+    const gptr<const R> py = gp((const R*)b.uy[par]), pz = gp((const R*)b.uz[par]);
+    const int cmin = rng_p[0], cmax = rng_p[1];
+    if (it.y == 0 && tid == 0) begin_step<R>(beams[it.x], par, N);
+    if (cmin > cmax) return;
+    const int lo_cell = max(cmin - 1, 0), hi_cell = min(cmax + 1, N);   // counts cover the range +-1
+    const int ngroups = mc_groups(lo_cell, hi_cell, G);
+    for (int gi = it.y; gi < ngroups; gi += nwg) {
+        const int2 gb = mc_group(lo_cell, hi_cell, G, ngroups, gi);
+        const int g0 = gb.x, g1 = gb.y, n = g1 - g0;
+        // live cells only (the graveyard cells 1 and N-2 are skipped); both
+        // bounds come in with one load (lane 0 and lane 1), read back with readlane
+        const int sb = ldo(st, (unsigned)(lane == 0 ? max(g0, 2) : min(g1, N - 2)));
+        for (int k = lane; k < n; k += 64) {
+            cnt[k][0] = cnt[k][1] = cnt[k][2] = 0;
+            Sl[k][0] = Sl[k][1] = Sl[k][2] = Sl[k][3] = 0.0;
+        }
+        if (wv == kMcWaves - 1)
+            for (int k = lane; k <= n; k += 64) stl[k] = ldo(st, (unsigned)min(g0 + k, N + 1));
+        if (wv == 0) stage_fields<R>(pa, Et, Ht, g0, n, lane);
+        const int plo = min(max(__builtin_amdgcn_readlane(sb, 0), 0), np);
+        const int phi = max(plo, min(max(__builtin_amdgcn_readlane(sb, 1), 0), np));
+        // this wave's run of chunks [w0, w1) in particle indices
+        const int nch = (phi - plo + 63) / 64;
+        const int per = (nch + kMcWaves - 1) / kMcWaves;
+        const bool one = per <= kMcHold;
+        const int w0 = one ? min(phi, plo + 64 * per * wv) : (wv == 0 ? plo : phi);
+        const int w1 = one ? min(phi, w0 + 64 * per) : phi;
+        if (lane < 4 * kMcHold) Sf_all[wv][lane >> 2][lane & 3] = 0.0;
+        int first = -1;
+        McHeld<R> held[kMcHold];
+#pragma unroll
+        for (int q = 0; q < kMcHold; ++q) held[q].k = -1;      // -1: no particle held
+        McChunk<R> nb;
+        if (one) {
+            // every chunk's loads in flight before the fields' barrier
+            McChunk<R> hb[kMcHold];
+#pragma unroll
+            for (int q = 0; q < kMcHold; ++q)
+                if (w0 + 64 * q < w1) mc_load<R>(cell, pid, pf, px, py, pz, w0 + 64 * q, np, lane, hb[q]);
+            if (w0 < w1) first = __builtin_amdgcn_readfirstlane(hb[0].c) - g0;
+            if (lane == 0) first_all[wv] = first;
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < kMcHold; ++q)
+                if (w0 + 64 * q < w1)
+                    grp_count<R, true>(pa, Et, Ht, g0, hb[q], w0 + 64 * q, w1, lane, cnt, Sl, first, Sf_all[wv][q],
+                                       held[q]);
+        } else {
+            // Pass 1 of the two-pass form: the next chunk's loads in flight
+            // while one is processed.
+            if (lane == 0) first_all[wv] = -1;
+            if (wv == 0) mc_load<R>(cell, pid, pf, px, py, pz, plo, np, lane, nb);
+            __syncthreads();
+            for (int bb = w0; bb < w1; bb += 64) {
+                McChunk<R> cb = nb;
+                if (bb + 64 < w1) mc_load<R>(cell, pid, pf, px, py, pz, bb + 64, np, lane, nb);
+                grp_count<R, false>(pa, Et, Ht, g0, cb, bb, w1, lane, cnt, Sl, -1, Sf_all[0][0], held[0]);
+            }
+        }
+        __syncthreads();
+        // the group's totals and sums: out to the node blocks, and kept for the ranks
+        const gptr<int32_t> cup = gp(b.cup), cdown = gp(b.cdown);
+        const gptr<double> Sg = gp(b.S);
+        for (int k = tid; k < n * 4; k += 64 * kMcWaves) {
+            const int kc = k >> 2, w = k & 3;
+            double t = 0.0;
+#pragma unroll
+            for (int v = 0; v < kMcWaves; ++v) {
+                t += S_all[v][kc][w];
+                if (first_all[v] == kc) {
+#pragma unroll
+                    for (int q = 0; q < kMcHold; ++q) t += Sf_all[v][q][w];
+                }
+            }
+            Sg[4 * (size_t)(g0 + kc) + w] = t;
+            if (w < 3) {
+                int c = 0;
+#pragma unroll
+                for (int v = 0; v < kMcWaves; ++v) {
+                    const int x = cnt_all[v][kc][w];
+                    cnt_all[v][kc][w] = one ? c : 0;
+                    c += x;
+                }
+                tot[kc][w] = c;
+                if (w == 0) cdown[g0 + kc] = c;
+                if (w == 2) cup[g0 + kc] = c;
+            }
+        }
+        __syncthreads();
+        // The new state (mc_put): from registers, or pass 2 (bitwise the same
+        // moves; the particles come back from L2/MALL) with the ranks.
+        const StateOut<R> nxt{gp(b.id[po]), gp(b.frac[po]), gp(b.ux[po]), gp(b.uy[po]), gp(b.uz[po])};
+        const StateOut<R> stg{gp(b.id[par]), gp(b.frac[par]), gp(b.ux[par]), gp(b.uy[par]), gp(b.uz[par])};
+        const gptr<int32_t> cello = gp(b.cell[po]), cellp = gp(b.cell[par]);
+        const gptr<int32_t> err = gp(b.err);
+        if (one) {
+#pragma unroll
+            for (int q = 0; q < kMcHold; ++q)
+                if (held[q].k >= 0)
+                    mc_put<R>(nxt, stg, cello, cellp, stl, tot, n, held[q].k, held[q].d,
+                              held[q].r + cnt[held[q].k][held[q].d + 1], held[q].c, held[q].s, np, err);
+        } else {
+            if (w0 < w1) mc_load<R>(cell, pid, pf, px, py, pz, w0, np, lane, nb);
+            for (int bb = w0; bb < w1; bb += 64) {
+                McChunk<R> cb = nb;
+                if (bb + 64 < w1) mc_load<R>(cell, pid, pf, px, py, pz, bb + 64, np, lane, nb);
+                const int i = bb + lane;
+                const int c_old = i < phi ? cb.c : 0x7fffffff;
+                const Chunk k = chunk_info(c_old, i, phi, lane);
+                Pushed<R> s;
+                s.id = cb.id;
+                s.f = cb.f; s.ux = cb.ux; s.uy = cb.uy; s.uz = cb.uz;
+                int c = c_old, d = 0, off = 1;
+                R a0 = R(0), a1 = R(0);
+                if (k.valid) push_tab<R>(pa, Et, Ht, g0, c, s.f, s.ux, s.uy, s.uz, d, off, a0, a1);
+                const unsigned long long seg = lanes_le(lane) & ~lanes_lt(k.fl);
+                const unsigned long long bd0 = __ballot(k.valid && d == -1);
+                const unsigned long long bd1 = __ballot(k.valid && d == 0);
+                const unsigned long long bd2 = __ballot(k.valid && d == 1);
+                const unsigned long long mine = d < 0 ? bd0 : (d == 0 ? bd1 : bd2);
+                const int lk = k.valid ? c_old - g0 : 0;
+                int r = 0;
+                if (k.valid) r = cnt[lk][d + 1] + __popcll(mine & lanes_lt(lane) & ~lanes_lt(k.fl));
+                wave_sync();
+                if (k.valid && k.last) {
+                    cnt[lk][0] += __popcll(bd0 & seg);
+                    cnt[lk][1] += __popcll(bd1 & seg);
+                    cnt[lk][2] += __popcll(bd2 & seg);
+                }
+                if (k.valid) mc_put<R>(nxt, stg, cello, cellp, stl, tot, n, lk, d, r, c, s, np, err);
+                wave_sync();
+            }
+        }
+        __syncthreads();      // the tables are written again by the next group
+    }
+}
+
 // The pair's eight FP64 CIC sums (a: cell A onto nodes c-1 .. c+2, b: cell
 // B) over the wave's 64 lanes, in a fixed order, through the wave's own LDS
 // rows red[0..8]: lane l adds the eight values of sum l/8 held by lanes

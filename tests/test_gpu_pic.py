@@ -248,3 +248,42 @@ def test_config3_full_size_invariants():
     for k in ("E", "H", "J", "x", "u"):
         assert np.array_equal(a[k], b[k]), k
 
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("per_cell,group", [(3, 0), (30, 0), (30, 64), (70, 13), (90, 11), (25, 2)])
+def test_group_per_workgroup_equals_group_per_wave(prec, per_cell, group):
+    """A small launch gives each multi-cell group a workgroup, a large one a
+    wave.  A beam alone (a workgroup per group) and beside a beam of thousands
+    of two-cell groups (a wave per group) must agree bit for bit: fields, J',
+    particles.  Densities put cells over one to three 64-particle chunks;
+    64 cells of 30 particles exceed what a workgroup holds (its two-pass
+    form)."""
+    from fdtd_pic_amd import configs, engine
+    steps, n_cells = 60, 150
+    rng = np.random.default_rng(11)
+
+    def spec(N):
+        p = configs.base(N, steps, slab_start=60, slab_stop=90, src_cell=200, probes=[150, N - 60], src_t0=5e-15,
+                         src_tau=2e-15, src_amp=1e6)
+        return engine.physical_spec(p)
+
+    def beam(lo, cells, n, g):
+        x = lo + rng.uniform(0.0, cells, n)
+        u = rng.normal(0.0, 0.15, (n, 3))
+        return engine.Beam(x, u, -configs.E_CHARGE, configs.M_ELECTRON, 1e9, configs.DT, configs.DZ, group=g)
+
+    mine = beam(250, n_cells, per_cell * n_cells, group)
+    filler = beam(300, 4000, 8000, 2)
+    outs = []
+    for with_filler in (False, True):
+        with engine.Context(prec, K=1, S=1) as c:
+            s = c.add(spec(700), beam=mine)
+            if with_filler:
+                c.add(spec(5000), beam=filler)
+            c.run(steps)
+            x, u, alive = s.particles()
+            outs.append({"E": s.read("E"), "H": s.read("H"), "J": s.read("J"), "x": x, "u": u, "alive": alive})
+    assert np.abs(outs[0]["J"]).max() > 0
+    for k in outs[0]:
+        assert np.array_equal(outs[0][k], outs[1][k]), k
