@@ -145,20 +145,30 @@ int fdtd_set_pic_fusion(fdtd_ctx *ctx, int on);
  * in the reference (which has no particles). */
 int fdtd_set_pic_lds_rows(fdtd_ctx *ctx, int rows);
 
-/* Persistent field launches (on = 1): when the context's tiles all fit on
- * the device at once (one slab kind, uniform tiles, S <= 64K - 2S, no beam),
- * one launch runs up to 4,096 blocks of S steps.  Each tile keeps its window
- * in registers for the whole launch; between blocks it writes its interior,
- * publishes a per-tile flag, waits for its two neighbour tiles to reach the
- * same block, and reloads only its halo cells.  The waits are bounded (2 s);
- * one that times out makes fdtd_sync and the reads fail with FDTD_E_STATE.
- * Otherwise, and for the steps left over, launches run one block each.
- * Results are bitwise those of one-block launches of the same (K, S).  No
- * counterpart in the reference; it replaces the per-S-steps relaunch of this
- * library's own loop (the `for counts in range(P.timeSteps)` bodies of
- * Solver_Engine.py:167,236,294). */
+/* Resident field launches (on = 1, the default; 0: one launch per S steps):
+ * when the context's tiles all fit on the device at once (no beam, no energy
+ * recording, one kind of Lorentz/Kerr slab), fdtd_run is one launch.  Each
+ * tile keeps its window in registers for the whole run; between blocks of
+ * steps it hands its edge cells to the tiles beside it through a mailbox in
+ * device memory.  The tiles' widths and the block length are chosen by the
+ * library (FP32: blocks of the S of fdtd_set_tiling, whose rounding depends on
+ * it).  Results are bitwise those of one launch per S steps.  A wait for a
+ * neighbour is bounded (max_wait_us; 0: 50 ms): a launch that passes the bound
+ * because something else holds the device leaves its starting state as it
+ * was, and the next call on the context runs its steps again with one launch
+ * per S steps.  No counterpart in the reference; it replaces the per-S-steps
+ * relaunch of this library's own loop (the `for counts in range(P.timeSteps)`
+ * bodies of Solver_Engine.py:167,236,294). */
+int fdtd_set_resident(fdtd_ctx *ctx, int on, int64_t max_wait_us);
+/* *active = 1 when the next fdtd_run uses resident launches. */
+int fdtd_resident_active(fdtd_ctx *ctx, int *active);
+/* Request for persistent launches (on = 1) under the conditions of uniform
+ * tiles with S <= 64K - 2S, one slab kind and no beam: fdtd_persistent_active
+ * tells whether the next fdtd_run keeps its tiles on the device between
+ * blocks of S steps under them.  Resident launches do so with or without
+ * this request; the results are the same bits. */
 int fdtd_set_persistent(fdtd_ctx *ctx, int on);
-/* *active = 1 when the next fdtd_run uses persistent launches. */
+/* *active = 1 when the request holds for the next fdtd_run. */
 int fdtd_persistent_active(fdtd_ctx *ctx, int *active);
 /* Workgroup halo exchange (h > 0; 0 turns it off, the default): the four
  * waves of a field workgroup take adjacent windows of one simulation that

@@ -50,25 +50,50 @@ struct EnergyJob {
 
 enum SlabKind { SLAB_NONE = 0, SLAB_DIEL = 1, SLAB_LINEAR = 2, SLAB_KERR_REF = 3, SLAB_KERR_E = 4 };
 
-// A field launch that runs nblocks blocks of S steps instead of one.  Every
-// tile stays resident for the whole launch with its window in registers:
-// after a block it writes its interior (as a one-block launch does) and
-// publishes flags[tile] = the global index of the block it finished; before
-// the next block it waits until both neighbour tiles (nbr: left, right; -1
-// none) have finished the same block, then reloads only its halo cells, which
-// lie in their interiors (the host guarantees S <= U, uniform tiles, and no
-// more tiles than the device holds at once).  A wait that passes
-// spin_ticks of the 100 MHz real-time counter sets *err and ends the tile
-// (a bounded wait: the launch always drains).  nblocks = 1 and flags = null
-// is the plain one-block launch.
+// Halo option of a one-block field launch.
 struct PersistArgs {
-    int nblocks;
-    unsigned long long* flags;
-    const int2* nbr;
-    int32_t* err;
-    long long spin_ticks;
     int halo;        // > 0: the workgroup halo-exchange instance, exchange period (cells = steps)
 };
+
+// A resident field launch: nsteps steps of every simulation in one launch, in
+// blocks of S.  Every tile is one wave that keeps its window in registers for
+// the whole launch; after a block it hands its edge cells to the tiles whose
+// halos they are, through the mailbox, and takes its own halo cells from
+// there.  The host launches no more tiles than the device holds at once.
+//
+// Mailbox: u64 words [set 2][slot 3][value kResValues][cell].  A word holds
+// the value itself (FP64) or a pair of values (FP32: a field and its Kahan
+// compensation), and kResEmpty, a signalling NaN pattern that no arithmetic
+// produces, while nothing is there, so one load brings a value and tells that
+// it has come.  Hand-off q of a launch uses slot q % 3; a tile empties the
+// words of hand-off q - 1 once it has received hand-off q (its readers sent q
+// after they had read q - 1), two blocks before they are written again, and
+// waits for those stores before its next sends.  Launches alternate the sets:
+// each empties what the launch before it left in the other one.
+//
+// A wait of more than max_polls loads of the halo (each goes to memory and
+// back, about 0.5 us; the tiles are not all resident: something else holds the
+// device) sets *err and *herr to the launch's ordinal and ends the tile; the other tiles end the same way
+// and a later launch that finds *err set returns at once.  The launch reads
+// the buffers of its parity and writes only the other ones, so the host runs
+// the steps again from there with one-block launches.
+struct ResArgs {
+    unsigned long long* box;     // this launch's set
+    unsigned long long* other;   // the other set
+    int stride;                  // cells of the mailbox (all simulations, with one spare)
+    int nsteps, S;
+    int ordinal;
+    int32_t* err;                // device
+    int32_t* herr;               // host memory
+    int max_polls;
+};
+// Tile of a resident launch: x = simulation | flags, y, z = first owned cell
+// and the one after the last, w = the simulation's first cell in the mailbox.
+constexpr int kResK2 = 1 << 24, kResK4 = 1 << 25;   // cells per lane: 1, 2 or 4
+constexpr int kResPlain = 1 << 26;                  // no D-form slab cell in its window: the plain bodies
+constexpr unsigned long long kResEmpty = 0x7ff45ea17fb45ea1ull;
+template <typename R>
+constexpr int kResValues = sizeof(R) == 8 ? 7 : 6;   // FP64 E H D P Pm psiE psiH; FP32 pairs E H D P, Pm, psiE|psiH
 
 // Particle beam of one simulation.  Particles are kept sorted by cell
 // (stable), structure of arrays, ping-ponged per step like the fields;

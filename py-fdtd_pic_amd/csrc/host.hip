@@ -19,7 +19,11 @@ hipError_t launch_stencil(const SimDev<R>* sims, const int2* tiles, int ntiles, 
                           long long gstep0, int nsteps, int K, int S, int kind, const PersistArgs& pa,
                           hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
 template <typename R, bool KAHAN>
-int field_capacity_per_cu(int K, int kind);
+hipError_t launch_resident(const SimDev<R>* sims, const int4* tiles, int ntiles, long long launch_idx,
+                           long long gstep0, int kind, int W, const ResArgs& ra, hipStream_t st);
+template <typename R, bool KAHAN>
+int resident_capacity_per_cu(int kind, int W);
+hipError_t launch_box_empty(unsigned long long* box, size_t values, int stride, hipStream_t st);
 struct OpArgs {
     double* a[8];
     double s[4];
@@ -45,6 +49,9 @@ hipError_t launch_field_scatter(const SimDev<R>* sims, const int2* tiles, int nt
 }
 
 using namespace fdtd;
+
+constexpr int kTileWavesHost = 4;      // tiles (waves) per field workgroup
+constexpr int kResMaxSHost = 60;       // steps of a resident block (kResMaxS)
 
 static thread_local std::string g_err;
 
@@ -167,6 +174,8 @@ static int build_sim(fdtd_ctx* ctx, SimHost& s, const fdtd_sim_desc_t* q) {
         R* ie = img.data() + L.off[11] / rs;
         for (int i = 0; i < ns; ++i) ie[i] = (R)(1.0 / q->sl_e[i]);
     }
+    s.last_dead = q->Rs <= N && q->s_ke[nstrip - 1] == 0.0 && q->s_kh[nstrip - 1] == 0.0 && q->s_CbE[nstrip - 1] == 0.0 &&
+                  q->s_C2H[nstrip - 1] == 0.0 && q->src_cell != N && !(ns > 0 && q->R > N);
     put(12, q->srcE, T);
     put(13, q->srcH, T);
     // a new block is not referenced by queued launches: upload on the upload
@@ -273,6 +282,64 @@ static void* noalloc_scratch(int dev) {
 // ------------------------------------------------------------------------
 // C ABI
 // ------------------------------------------------------------------------
+// ------------------------------------------------------------------------
+// Resident launches in flight on a device, over every context and thread: a
+// launch is taken only while the shares of the device that they hold add up
+// to at most one, so that all tiles of each are resident together.
+// ------------------------------------------------------------------------
+struct ResUse {
+    fdtd_ctx* c;
+    hipEvent_t done;
+    double share;
+};
+static std::mutex g_res_mu;
+static std::vector<ResUse> g_res_use[kMaxDevices];
+
+static void res_release(fdtd_ctx* c) {
+    std::lock_guard<std::mutex> lock(g_res_mu);
+    std::vector<ResUse>& u = g_res_use[c->device];
+    u.erase(std::remove_if(u.begin(), u.end(), [&](const ResUse& x) { return x.c == c; }), u.end());
+}
+
+static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident);
+
+// Waits for the queued resident launches and, if one gave up (a neighbour
+// wait passed its bound: its tiles were not all resident), takes the counters
+// back to where it began and runs its steps, and those of the launches behind
+// it, which returned at once, with one-block launches.
+static int resolve_resident(fdtd_ctx* c) {
+    if (c->res_pending.empty()) return FDTD_OK;
+    HIPCHK(hipStreamSynchronize(c->st));
+    res_release(c);
+    std::vector<ResPending> pend;
+    pend.swap(c->res_pending);
+    const int32_t bad = __atomic_load_n(c->h_rerr, __ATOMIC_ACQUIRE);
+    if (bad == 0) return FDTD_OK;
+    __atomic_store_n(c->h_rerr, 0, __ATOMIC_RELEASE);
+    HIPCHK(hipMemsetAsync(c->d_rerr, 0, sizeof(int32_t), c->st));
+    c->box_stale = true;
+    size_t k = 0;
+    while (k < pend.size() && pend[k].ordinal != bad) ++k;
+    if (k == pend.size()) return fdtd_fail(FDTD_E_STATE, "resident launch: unknown ordinal in the give-up flag");
+    c->launch_idx = pend[k].launch_idx;
+    c->gstep = pend[k].gstep;
+    for (const ResPending::Sim& x : pend[k].sims) {
+        c->sims[x.id]->steps_done = x.steps_done;
+        c->sims[x.id]->launches = x.launches;
+    }
+    c->dirty = true;
+    long long again = 0;
+    for (; k < pend.size(); ++k) again += pend[k].nsteps;
+    return run_steps_host(c, again, false);
+}
+
+// Everything queued on the context's stream has finished.
+static int drain(fdtd_ctx* c) {
+    if (int rc = resolve_resident(c)) return rc;
+    HIPCHK(hipStreamSynchronize(c->st));
+    return FDTD_OK;
+}
+
 extern "C" {
 
 const char* fdtd_last_error(void) { return g_err.c_str(); }
@@ -303,13 +370,15 @@ int fdtd_ctx_create(int precision, fdtd_ctx** out) {
         return rc;
     }
     if (hipMalloc(&c->d_err, sizeof(int32_t)) != hipSuccess || hipMemset(c->d_err, 0, sizeof(int32_t)) != hipSuccess ||
-        hipMalloc(&c->d_perr, sizeof(int32_t)) != hipSuccess || hipMemset(c->d_perr, 0, sizeof(int32_t)) != hipSuccess) {
+        hipMalloc(&c->d_rerr, sizeof(int32_t)) != hipSuccess || hipMemset(c->d_rerr, 0, sizeof(int32_t)) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_rerr, sizeof(int32_t), hipHostMallocDefault) != hipSuccess) {
         if (c->d_err) (void)hipFree(c->d_err);
-        if (c->d_perr) (void)hipFree(c->d_perr);
+        if (c->d_rerr) (void)hipFree(c->d_rerr);
         (void)hipStreamDestroy(c->st);
         delete c;
         return fdtd_fail(FDTD_E_HIP, "allocation of the error flags failed");
     }
+    *c->h_rerr = 0;
     if (hipDeviceGetAttribute(&c->cu_count, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         c->cu_count = 0;
     if (hipDeviceGetAttribute(&c->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
@@ -332,8 +401,11 @@ int fdtd_ctx_destroy(fdtd_ctx* c) {
     for (BeamHost* b : c->beams)
         if (b) { if (b->block) (void)hipFree(b->block); delete b; }
     for (void* p : {(void*)c->d_beams, (void*)c->d_pblocks, (void*)c->d_pitems, (void*)c->d_err, c->d_scratch,
-                    (void*)c->d_perr, (void*)c->d_flags, (void*)c->d_nbr})
+                    (void*)c->d_rerr, (void*)c->d_rtiles, (void*)c->d_box})
         if (p) (void)hipFree(p);
+    res_release(c);
+    if (c->res_ev) (void)hipEventDestroy(c->res_ev);
+    if (c->h_rerr) (void)hipHostFree(c->h_rerr);
     if (c->d_sims) (void)hipFree(c->d_sims);
     if (c->d_tiles) (void)hipFree(c->d_tiles);
     for (auto& e : c->events) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
@@ -383,7 +455,7 @@ int fdtd_add_sim(fdtd_ctx* c, const fdtd_sim_desc_t* q, int* sim_id) {
 
 int fdtd_remove_sim(fdtd_ctx* c, int id) {
     if (!c || id < 0 || id >= (int)c->sims.size() || !c->sims[id]) return fdtd_fail(FDTD_E_ARG, "bad sim id");
-    HIPCHK(hipStreamSynchronize(c->st));
+    if (int rc = drain(c)) return rc;
     SimHost* s = c->sims[id];
     if (s->block) (void)hipFree(s->block);
     if (s->eblock) (void)hipFree(s->eblock);
@@ -403,6 +475,7 @@ int fdtd_remove_sim(fdtd_ctx* c, int id) {
 
 int fdtd_reset_sim(fdtd_ctx* c, int id) {
     if (!c || id < 0 || id >= (int)c->sims.size() || !c->sims[id]) return fdtd_fail(FDTD_E_ARG, "bad sim id");
+    if (int rc = resolve_resident(c)) return rc;
     SimHost* s = c->sims[id];
     const size_t state0 = s->lay_off[14];   // first state sub-array (after coefficients and sources)
     HIPCHK(hipMemsetAsync((char*)s->block + state0, 0, s->bytes - state0, c->st));
@@ -678,6 +751,192 @@ static int attach_t(fdtd_ctx* c, int id, SimHost& s, const fdtd_beam_desc_t* bd)
     return FDTD_OK;
 }
 
+// ------------------------------------------------------------------------
+// resident launches: the tile plan
+// ------------------------------------------------------------------------
+struct ResInterval {
+    int lo, hi;       // cells [lo, hi)
+    bool window;      // no part of a light tile's window may meet it (else only its own cells)
+};
+struct ResSim {
+    int id, N;
+    bool plain;                             // no D-form slab: the plain bodies
+    bool last_dead;                         // the last cell's fields never change
+    std::vector<ResInterval> heavy;         // slab, CPML strips, source, probes
+};
+
+// Tiles of one simulation, in order: light tiles (plain cells, Kl per lane)
+// where their windows meet nothing else, heavy ones (Kh per lane) elsewhere.
+// With Kl = 0 every tile is a heavy one.
+static int res_tile_sim(const ResSim& q, int Kh, int Kl, int S, int box0, std::vector<int4>* out) {
+    const int Uh = 64 * Kh - 2 * S, Ul = 64 * Kl - 2 * S;
+    auto kflag = [](int K) { return K == 4 ? kResK4 : K == 2 ? kResK2 : 0; };
+    int n = 0;
+    for (int o = 0; o <= q.N;) {
+        int light_end = Kl ? std::min(o + Ul, q.N + 1) : o;
+        for (const ResInterval& v : q.heavy) {
+            const int m = v.window ? S : 0;
+            if (v.hi > o - m) light_end = std::min(light_end, v.lo - m);
+        }
+        int e, flags;
+        // light where it covers at least what a heavy tile would
+        if (Kl && light_end - o >= std::min(Uh, Ul)) {
+            e = light_end;
+            flags = kResPlain | kflag(Kl);
+        } else {
+            e = std::min(o + Uh, q.N + 1);
+            flags = (q.plain ? kResPlain : 0) | kflag(Kh);
+        }
+        // the last cell alone is not worth a tile: the window holds it, and
+        // beyond it everything is zero
+        if (e == q.N && q.last_dead) e = q.N + 1;
+        if (out) out->push_back(make_int4(q.id | flags, o, e, box0));
+        ++n;
+        o = e;
+    }
+    return n;
+}
+
+// What a block of S steps of a wave with a SIMD to itself costs in FP64: ns
+// per step and ns for the hand-off, by cells per lane (measured per tile: the
+// slowest tile, which waits for nobody, sets the pace).  Heavy tiles by slab
+// kind; the strip, source and probe tiles' classes lie below the slabs' or
+// near them.
+struct ResCost {
+    double heavy[2], light[3];
+};
+static ResCost res_cost(int kind) {
+    const double l1 = 46, l2 = 60, l4 = 77;
+    return kind == SLAB_KERR_E     ? ResCost{{125, 158}, {l1, l2, l4}}
+           : kind == SLAB_KERR_REF ? ResCost{{3900, 7100}, {l1, l2, l4}}
+                                   : ResCost{{90, 115}, {l1, l2, l4}};
+}
+constexpr double kResHandNs[3] = {1000, 1500, 2600};     // K = 1, 2, 4
+
+// Decides whether the context's active simulations run resident, and their
+// tiles (res_ok, res_tiles, res_S, res_kind, res_stride).
+template <typename R>
+static int plan_resident(fdtd_ctx* c) {
+    constexpr bool f32 = sizeof(R) == 4;
+    if (!c->res_mode || c->cu_count <= 0 || c->tile_sims.empty()) return FDTD_OK;
+    // FP32 rounds by K and a cell's place in its tile (psi_next, and the
+    // emulated cells of slab-boundary tiles), so there the tiles and blocks are
+    // the one-block ones
+    if (f32 && (c->K_slab != c->K || c->K > 4)) return FDTD_OK;
+    if (f32 && (c->S_run > kResMaxSHost || 64 * c->K - 2 * c->S_run < 1)) return FDTD_OK;
+    bool kerr = f32;
+    for (int i : c->tile_sims) {
+        const SimHost& s = *c->sims[i];
+        if (s.e_every > 0) return FDTD_OK;            // energy is taken launch by launch
+        kerr = kerr || (s.d.slab_kind == SLAB_KERR_E && s.d.kerr_chi3 != 0.0);
+    }
+    int kind = SLAB_DIEL, stride = 1;
+    long long cells = 0;
+    std::vector<ResSim> sims;
+    for (int i : c->tile_sims) {
+        const fdtd_sim_desc_t& d = c->sims[i]->d;
+        ResSim q;
+        q.id = i;
+        q.N = d.N;
+        q.plain = d.slab_kind < SLAB_LINEAR;
+        q.last_dead = c->sims[i]->last_dead;
+        if (!q.plain) {
+            // FP64: a Kerr slab with chi3 = 0 is the linear slab bit for bit
+            // (the root's series is then exactly 1)
+            const int k = d.slab_kind == SLAB_KERR_E && !kerr ? SLAB_LINEAR : d.slab_kind;
+            if (kind != SLAB_DIEL && k != kind) return FDTD_OK;
+            kind = k;
+            q.heavy.push_back({d.F, d.R, true});
+        }
+        if (d.Ls > 0) q.heavy.push_back({0, d.Ls, true});
+        if (d.Rs <= d.N) q.heavy.push_back({d.Rs, d.N + 1, true});
+        q.heavy.push_back({d.src_cell - 1, d.src_cell + 1, true});
+        for (int p = 0; p < d.nprobe; ++p) q.heavy.push_back({d.probe_cell[p], d.probe_cell[p] + 1, false});
+        if (d.has_current) q.heavy.push_back({0, d.N + 1, true});       // the general class everywhere
+        if (f32) {
+            // no general class: a current, or more than two probes in one tile
+            if (d.has_current) return FDTD_OK;
+            const int U0 = 64 * c->K - 2 * c->S_run;
+            for (int p = 0; p < d.nprobe; ++p) {
+                int same = 0;
+                for (int r = 0; r < d.nprobe; ++r) same += d.probe_cell[r] / U0 == d.probe_cell[p] / U0;
+                if (same > 2) return FDTD_OK;
+            }
+        }
+        cells += d.N + 1;
+        sims.push_back(std::move(q));
+    }
+    if (cells > (1 << 28)) return FDTD_OK;
+    stride += (int)cells;
+    int bKh = 0, bKl = 0, bS = 0, bW = 0;
+    const int round = c->cu_count * kTileWavesHost;       // one wave per SIMD
+    auto count = [&](int Kh, int Kl, int S, long long most) {
+        if (cells / (64 * std::max(Kh, Kl) - 2 * S) > most) return most + 1;
+        long long n = 0;
+        for (const ResSim& q : sims) n += res_tile_sim(q, Kh, Kl, S, 0, nullptr);
+        return n;
+    };
+    long long nt = 0;
+    if (f32) {
+        bKh = c->K;
+        bS = c->S_run;
+        bW = bKh == 4 ? 1 : 2;
+        nt = count(bKh, 0, bS, 2 * round);
+        if (nt > (long long)resident_capacity_per_cu<R, f32>(kind, bW) * round) return FDTD_OK;
+    } else {
+        const ResCost cost = res_cost(kind);
+        const int cap2 = resident_capacity_per_cu<R, f32>(kind, 2);
+        double best = 1e30;
+        for (int Kh = 1; Kh <= 2; ++Kh)
+            for (int Kl = Kh; Kl <= 4; Kl *= 2)
+                for (int S = 4; S <= 32 * Kh - 4; S += 4) {
+                    const long long n = count(Kh, Kl, S, (long long)cap2 * round);
+                    if (n > (long long)cap2 * round) continue;
+                    const double rounds = (double)((n + round - 1) / round);
+                    const int l = Kl == 4 ? 2 : Kl - 1;
+                    const bool hand = n > (long long)sims.size();
+                    const double t = rounds * std::max(cost.heavy[Kh - 1] + (hand ? kResHandNs[Kh - 1] / S : 0.0),
+                                                       cost.light[l] + (hand ? kResHandNs[l] / S : 0.0));
+                    if (t < best) { best = t; bKh = Kh; bKl = Kl; bS = S; nt = n; }
+                }
+        if (!bKh) return FDTD_OK;
+        bW = nt > round ? 2 : 1;
+        if (nt > (long long)resident_capacity_per_cu<R, f32>(kind, bW) * round) return FDTD_OK;
+    }
+    std::vector<int4> tiles;
+    int box0 = 0;
+    for (const ResSim& q : sims) {
+        res_tile_sim(q, bKh, bKl, bS, box0, &tiles);
+        box0 += q.N + 1;
+    }
+    // mailbox: two sets of three slots
+    const size_t words = (size_t)2 * 3 * kResValues<R> * stride;
+    if (words * sizeof(unsigned long long) > c->d_box_cap) {
+        HIPCHK(hipStreamSynchronize(c->st));
+        if (c->d_box) HIPCHK(hipFree(c->d_box));
+        c->d_box = nullptr;
+        c->d_box_cap = 0;
+        if (hipMalloc((void**)&c->d_box, words * sizeof(unsigned long long)) != hipSuccess) {
+            (void)hipGetLastError();
+            return FDTD_OK;      // no room: one-block launches
+        }
+        c->d_box_cap = words * sizeof(unsigned long long);
+        c->box_stale = true;
+    }
+    auto same = [](const int4& a, const int4& b) { return a.x == b.x && a.y == b.y && a.z == b.z && a.w == b.w; };
+    if (c->res_S != bS || c->res_stride != stride || c->res_tiles.size() != tiles.size() ||
+        !std::equal(tiles.begin(), tiles.end(), c->res_tiles.begin(), same))
+        c->box_stale = true;     // words that no tile of the new plan empties may be full
+    c->res_tiles.swap(tiles);
+    c->res_S = bS;
+    c->res_stride = stride;
+    c->res_kind = kind;
+    c->res_W = bW;
+    c->res_cap = bW * round;
+    c->res_ok = true;
+    return FDTD_OK;
+}
+
 // Rebuild the device SimDev array and the tile list for active, unfinished sims.
 template <typename R>
 static int rebuild_t(fdtd_ctx* c) {
@@ -821,48 +1080,15 @@ static int rebuild_t(fdtd_ctx* c) {
     }
     ups.push_back({&c->d_sims, &c->d_sims_cap, devs.data(), sizeof(SimDev<R>) * devs.size()});
     ups.push_back({(void**)&c->d_tiles, &c->d_tiles_cap, tiles.data(), sizeof(int2) * tiles.size()});
-    // persistent launches: one tile group of uniform tiles whose halos lie in
-    // the neighbouring interiors (S <= U), no beam, and every tile resident at
-    // once; the neighbour table maps each tile to the tiles on either side
-    c->persist_ok = false;
-    std::vector<int2> nbr;
-    bool energy = false;
-    for (int i : c->tile_sims) energy = energy || c->sims[i]->e_every > 0;
-    if (c->persist && !pic && !energy && c->groups.size() == 1 && c->K_slab == c->K && c->S_run <= U &&
-        c->cu_count > 0) {
-        const int per_cu = field_capacity_per_cu<R, sizeof(R) == 4>(c->K, c->groups[0].kind);
-        const long long wgs = ((long long)tiles.size() + 3) / 4;
-        if (per_cu > 0 && wgs <= (long long)per_cu * c->cu_count) {
-            std::vector<std::pair<long long, int>> key(tiles.size());
-            for (size_t t = 0; t < tiles.size(); ++t)
-                key[t] = {((long long)(tiles[t].x & 0xffffff) << 32) | (unsigned)tiles[t].y, (int)t};
-            std::sort(key.begin(), key.end());
-            auto find = [&](int sim, long long o) {
-                const long long k = ((long long)sim << 32) | (unsigned)o;
-                auto it = std::lower_bound(key.begin(), key.end(), std::make_pair(k, INT32_MIN));
-                return (it != key.end() && it->first == k) ? it->second : -1;
-            };
-            nbr.resize(tiles.size());
-            for (size_t t = 0; t < tiles.size(); ++t) {
-                const int sim = tiles[t].x & 0xffffff, o = tiles[t].y;
-                nbr[t] = make_int2(o > 0 ? find(sim, (long long)o - U) : -1,
-                                   o + U <= c->sims[sim]->d.N ? find(sim, (long long)o + U) : -1);
-            }
-            ups.push_back({(void**)&c->d_nbr, &c->d_nbr_cap, nbr.data(), sizeof(int2) * nbr.size()});
-            if (sizeof(unsigned long long) * tiles.size() > c->d_flags_cap) {
-                // flags only grow: a fresh buffer starts at zero, below every block index
-                HIPCHK(hipStreamSynchronize(c->st));
-                if (c->d_flags) HIPCHK(hipFree(c->d_flags));
-                c->d_flags = nullptr;
-                c->d_flags_cap = 0;
-                const size_t bytes = sizeof(unsigned long long) * tiles.size() * 2;
-                HIPCHK(hipMalloc(&c->d_flags, bytes));
-                HIPCHK(hipMemsetAsync(c->d_flags, 0, bytes, c->st));
-                c->d_flags_cap = bytes;
-            }
-            c->persist_ok = true;
-        }
+    // resident launches, and the conditions of the persistent request
+    c->res_ok = false;
+    if (!pic && !c->grouped) {
+        int rc = plan_resident<R>(c);
+        if (rc) return rc;
     }
+    c->persist_ok = c->persist && c->res_ok && c->groups.size() == 1 && c->K_slab == c->K && c->S_run <= U;
+    if (c->res_ok)
+        ups.push_back({(void**)&c->d_rtiles, &c->d_rtiles_cap, c->res_tiles.data(), sizeof(int4) * c->res_tiles.size()});
     int rc = staged_upload(c, ups);
     if (rc) return rc;
     c->ntiles = (int)tiles.size();
@@ -907,9 +1133,8 @@ static EvPair* next_event(fdtd_ctx* c, int kind) {
 // kernel, ev->second at the end of the last one.  With fused, the last group
 // runs in one launch with the particle scatter (stamped by fev instead).
 static int launch_once(fdtd_ctx* c, int n, EvPair* ev, hipStream_t st, bool fused = false,
-                       EvPair* fev = nullptr, int nblocks = 1) {
-    PersistArgs pa{1, nullptr, nullptr, nullptr, 0, c->grouped ? c->halo : 0};
-    if (nblocks > 1) pa = PersistArgs{nblocks, c->d_flags, c->d_nbr, c->d_perr, kPersistSpinTicks, 0};
+                       EvPair* fev = nullptr) {
+    const PersistArgs pa{c->grouped ? c->halo : 0};
     const size_t ng = c->groups.size();
     const size_t nplain = fused ? ng - 1 : ng;
     for (size_t gi = 0; gi < ng; ++gi) {
@@ -986,54 +1211,106 @@ static int close_bracket(fdtd_ctx* c) {
     return FDTD_OK;
 }
 
-extern "C" {
+// Queues n steps of every active simulation as one resident launch; *taken =
+// false when other contexts' resident launches hold too much of the device.
+template <typename R>
+static int run_resident_t(fdtd_ctx* c, int64_t n, bool* taken) {
+    *taken = false;
+    if (!c->res_ev) HIPCHK(hipEventCreateWithFlags(&c->res_ev, hipEventDisableTiming));
+    const int nt = (int)c->res_tiles.size();
+    std::lock_guard<std::mutex> lock(g_res_mu);
+    std::vector<ResUse>& use = g_res_use[c->device];
+    const double share = (double)((nt + kTileWavesHost - 1) / kTileWavesHost) / (c->res_cap / kTileWavesHost);
+    double held = 0.0;
+    for (size_t k = 0; k < use.size();) {
+        if (use[k].c == c) { use.erase(use.begin() + k); continue; }     // this stream runs its launches in turn
+        const hipError_t e = hipEventQuery(use[k].done);
+        if (e == hipSuccess) { use.erase(use.begin() + k); continue; }
+        if (e == hipErrorNotReady) (void)hipGetLastError();
+        held += use[k].share;
+        ++k;
+    }
+    if (held + share > 1.0) return FDTD_OK;
+    const size_t slots = (size_t)3 * kResValues<R> * c->res_stride;
+    if (c->box_stale) {
+        const hipError_t e = launch_box_empty(c->d_box, (size_t)2 * 3 * kResValues<R>, c->res_stride, c->st);
+        if (e != hipSuccess) return fdtd_fail(FDTD_E_HIP, std::string("mailbox: ") + hipGetErrorString(e));
+        c->box_stale = false;
+    }
+    ResArgs ra{};
+    ra.box = c->d_box + (c->box_set ? slots : 0);
+    ra.other = c->d_box + (c->box_set ? 0 : slots);
+    ra.stride = c->res_stride;
+    ra.nsteps = (int)n;
+    ra.S = c->res_S;
+    ra.ordinal = ++c->res_ordinal;
+    ra.err = c->d_rerr;
+    ra.herr = c->h_rerr;
+    ra.max_polls = c->res_polls;
+    EvPair* ev = nullptr;
+    const int blocks = (int)((n + c->S_run - 1) / c->S_run);
+    if (c->profile > 0) {
+        ev = next_event(c, FDTD_KERNEL_STENCIL);
+        if (!ev) return FDTD_E_HIP;
+        ev->launches = blocks;      // the timing is per S steps
+        HIPCHK(hipEventRecord(ev->first, c->st));
+    }
+    const hipError_t e = launch_resident<R, sizeof(R) == 4>((const SimDev<R>*)c->d_sims, c->d_rtiles, nt, c->launch_idx,
+                                                            c->gstep, c->res_kind, c->res_W, ra, c->st);
+    if (e != hipSuccess) return fdtd_fail(FDTD_E_HIP, std::string("resident launch: ") + hipGetErrorString(e));
+    if (ev) HIPCHK(hipEventRecord(ev->second, c->st));
+    HIPCHK(hipEventRecord(c->res_ev, c->st));
+    use.push_back({c, c->res_ev, share});
+    *taken = true;
+    c->box_set ^= 1;
+    ResPending p{ra.ordinal, c->launch_idx, c->gstep, n, {}};
+    c->launches += blocks;
+    bool finished = false;
+    for (int i : c->tile_sims) {
+        SimHost* s = c->sims[i];
+        p.sims.push_back({i, s->steps_done, s->launches});
+        s->launches++;
+        const int64_t done = std::min<int64_t>(s->d.steps, c->gstep + n - s->t_begin);
+        s->steps_done = std::max<int64_t>(s->steps_done, done);
+        if (s->steps_done >= s->d.steps) finished = true;
+    }
+    c->res_pending.push_back(std::move(p));
+    c->launch_idx++;
+    c->gstep += n;
+    if (finished) c->dirty = true;
+    return FDTD_OK;
+}
+static int run_resident(fdtd_ctx* c, int64_t n, bool* taken) {
+    return c->prec == FDTD_F64 ? run_resident_t<double>(c, n, taken) : run_resident_t<float>(c, n, taken);
+}
 
-int fdtd_run(fdtd_ctx* c, int64_t nsteps) {
-    if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
-    if (nsteps < 0) return fdtd_fail(FDTD_E_ARG, "nsteps < 0");
+// allow_resident: false while the steps of a resident launch that gave up are
+// run again.
+static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
     int64_t remaining = nsteps;
     while (remaining > 0) {
         if (c->dirty) {
             int rc = close_bracket(c);
             if (rc) return rc;
+            rc = resolve_resident(c);
+            if (rc) return rc;
             rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
             if (rc) return rc;
         }
         if (c->ntiles == 0) break;
-        if (c->persist_ok && remaining >= 2 * (int64_t)c->S_run) {
-            // one persistent launch of nb blocks of S steps (see PersistArgs)
-            const int nb = (int)std::min<int64_t>(remaining / c->S_run, kPersistMaxBlocks);
+        if (c->res_ok && allow_resident) {
+            const int64_t n = std::min<int64_t>(remaining, kResMaxSteps);
             int rc = close_bracket(c);
             if (rc) return rc;
-            hipEvent_t pe0 = nullptr, pe1 = nullptr;
-            if (c->profile > 0) {
-                EvPair* ev = next_event(c, FDTD_KERNEL_STENCIL);
-                if (!ev) return FDTD_E_HIP;
-                ev->launches = nb;      // the timing is per block
-                pe0 = ev->first;
-                pe1 = ev->second;
-                HIPCHK(hipEventRecord(pe0, c->st));
-            }
-            rc = launch_once(c, c->S_run, nullptr, c->st, false, nullptr, nb);
+            bool taken = false;
+            rc = run_resident(c, n, &taken);
             if (rc) return rc;
-            if (pe1) HIPCHK(hipEventRecord(pe1, c->st));
-            rc = throttle(c);
-            if (rc) return rc;
-            c->launches += nb;
-            bool finished = false;
-            for (int i : c->tile_sims) {
-                SimHost* s = c->sims[i];
-                s->launches += nb;
-                const int64_t done = std::min<int64_t>(s->d.steps, c->gstep + (int64_t)nb * c->S_run - s->t_begin);
-                s->steps_done = std::max<int64_t>(s->steps_done, done);
-                if (s->steps_done >= s->d.steps) finished = true;
+            if (taken) {
+                remaining -= n;
+                continue;
             }
-            c->launch_idx += nb;
-            c->gstep += (int64_t)nb * c->S_run;
-            remaining -= (int64_t)nb * c->S_run;
-            if (finished) c->dirty = true;
-            continue;
         }
+        if (int rc = resolve_resident(c)) return rc;
         // steps this launch: S, bounded by the remaining request; one step when
         // a beam is coupled (the deposit feeds every E update)
         int n = (int)std::min<int64_t>(remaining, c->S_run);
@@ -1138,6 +1415,14 @@ int fdtd_run(fdtd_ctx* c, int64_t nsteps) {
     return close_bracket(c);
 }
 
+extern "C" {
+
+int fdtd_run(fdtd_ctx* c, int64_t nsteps) {
+    if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
+    if (nsteps < 0) return fdtd_fail(FDTD_E_ARG, "nsteps < 0");
+    return run_steps_host(c, nsteps, true);
+}
+
 int fdtd_run_all(fdtd_ctx* c) {
     if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
     int64_t most = 0;
@@ -1154,23 +1439,9 @@ static int check_pic_flag(fdtd_ctx* c) {
     return FDTD_OK;
 }
 
-// A persistent field launch whose neighbour wait timed out (the flag is
-// cleared once reported).  Call after the stream has drained.
-static int check_persist_flag(fdtd_ctx* c) {
-    if (!c->d_perr || !c->persist) return FDTD_OK;
-    int32_t e = 0;
-    HIPCHK(hipMemcpy(&e, c->d_perr, sizeof(e), hipMemcpyDeviceToHost));
-    if (!e) return FDTD_OK;
-    HIPCHK(hipMemset(c->d_perr, 0, sizeof(int32_t)));
-    return fdtd_fail(FDTD_E_STATE, "persistent field launch: a neighbour wait timed out (tiles not all resident "
-                                   "at once?); the fields of that run are invalid");
-}
-
 int fdtd_sync(fdtd_ctx* c) {
     if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
-    HIPCHK(hipStreamSynchronize(c->st));
-    int rc = check_persist_flag(c);
-    if (rc) return rc;
+    if (int rc = drain(c)) return rc;
     return c->has_pic ? check_pic_flag(c) : FDTD_OK;
 }
 
@@ -1283,6 +1554,7 @@ int fdtd_state_load(fdtd_ctx* c, int id, const void* buf, int64_t len) {
     std::vector<int64_t> esteps((size_t)h.n_esteps);
     if (h.n_esteps) std::memcpy(esteps.data(), o, sizeof(int64_t) * h.n_esteps);
     o += sizeof(int64_t) * h.n_esteps;
+    if (int rc = resolve_resident(c)) return rc;
     // ordered after the target's queued launches; the host buffer is
     // pageable, so the copies finish before returning
     HIPCHK(hipMemcpyAsync((char*)s->block + p.state0, o, p.state_bytes, hipMemcpyHostToDevice, c->st));
@@ -1290,7 +1562,7 @@ int fdtd_state_load(fdtd_ctx* c, int id, const void* buf, int64_t len) {
     if (p.beam_bytes) HIPCHK(hipMemcpyAsync(p.b->block, o, p.beam_bytes, hipMemcpyHostToDevice, c->st));
     o += p.beam_bytes;
     if (p.e_bytes) HIPCHK(hipMemcpyAsync(s->eblock, o, p.e_bytes, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
+    if (int rc = drain(c)) return rc;
     s->steps_done = h.steps_done;
     s->launches = h.launches;
     s->launch_begin = c->launch_idx - h.rel_launch;
@@ -1307,7 +1579,7 @@ int fdtd_set_energy(fdtd_ctx* c, int id, int every, int rows) {
     if (every < 0 || rows < 0 || (every > 0 && rows < 1))
         return fdtd_fail(FDTD_E_ARG, "energy: every >= 0 and rows >= 1 when on");
     SimHost* s = c->sims[id];
-    HIPCHK(hipStreamSynchronize(c->st));
+    if (int rc = drain(c)) return rc;
     if (s->eblock) {
         (void)hipFree(s->eblock);
         c->dev_bytes -= s->ebytes;
@@ -1339,7 +1611,7 @@ int fdtd_read_energy(fdtd_ctx* c, int id, double* values, int64_t* steps, int64_
         (cap > 0 && (!values || !steps)))
         return fdtd_fail(FDTD_E_ARG, "bad argument");
     SimHost* s = c->sims[id];
-    HIPCHK(hipStreamSynchronize(c->st));
+    if (int rc = drain(c)) return rc;
     const int64_t n = std::min<int64_t>(cap, s->e_count);
     *count = s->e_count;
     if (n > 0) {
@@ -1361,12 +1633,39 @@ int fdtd_set_persistent(fdtd_ctx* c, int on) {
 int fdtd_persistent_active(fdtd_ctx* c, int* active) {
     if (!c || !active) return fdtd_fail(FDTD_E_ARG, "null argument");
     if (c->dirty) {
-        int rc = close_bracket(c);
+        int rc = resolve_resident(c);
+        if (rc) return rc;
+        rc = close_bracket(c);
         if (rc) return rc;
         rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
         if (rc) return rc;
     }
     *active = c->persist_ok ? 1 : 0;
+    return FDTD_OK;
+}
+
+int fdtd_set_resident(fdtd_ctx* c, int on, int64_t max_wait_us) {
+    if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
+    if ((on != 0 && on != 1) || max_wait_us < 0 || max_wait_us > 60000000)
+        return fdtd_fail(FDTD_E_ARG, "resident flag must be 0 or 1, the wait 0 (default) .. 60 s");
+    if (int rc = resolve_resident(c)) return rc;
+    c->res_mode = on;
+    c->res_polls = max_wait_us > 0 ? (int)(2 * max_wait_us) : kResMaxPolls;
+    c->dirty = true;
+    return FDTD_OK;
+}
+
+int fdtd_resident_active(fdtd_ctx* c, int* active) {
+    if (!c || !active) return fdtd_fail(FDTD_E_ARG, "null argument");
+    if (c->dirty) {
+        int rc = resolve_resident(c);
+        if (rc) return rc;
+        rc = close_bracket(c);
+        if (rc) return rc;
+        rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
+        if (rc) return rc;
+    }
+    *active = c->res_ok ? 1 : 0;
     return FDTD_OK;
 }
 
@@ -1389,7 +1688,9 @@ int fdtd_set_halo_exchange(fdtd_ctx* c, int h) {
 int fdtd_halo_exchange_active(fdtd_ctx* c, int* active) {
     if (!c || !active) return fdtd_fail(FDTD_E_ARG, "null argument");
     if (c->dirty) {
-        int rc = close_bracket(c);
+        int rc = resolve_resident(c);
+        if (rc) return rc;
+        rc = close_bracket(c);
         if (rc) return rc;
         rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
         if (rc) return rc;
@@ -1404,7 +1705,7 @@ int fdtd_busy(fdtd_ctx* c, int* busy) {
     if (e == hipErrorNotReady) { *busy = 1; return FDTD_OK; }
     if (e != hipSuccess) return fdtd_fail(FDTD_E_HIP, std::string("hipStreamQuery: ") + hipGetErrorString(e));
     *busy = 0;
-    return FDTD_OK;
+    return resolve_resident(c);
 }
 
 int fdtd_kernel_timing(fdtd_ctx* c, int kind, double* ms, int64_t* launches) {
@@ -1412,7 +1713,7 @@ int fdtd_kernel_timing(fdtd_ctx* c, int kind, double* ms, int64_t* launches) {
     if (kind < FDTD_KERNEL_STENCIL || kind > FDTD_KERNEL_FIELD_SORT) return fdtd_fail(FDTD_E_ARG, "bad kernel kind");
     int rc = close_bracket(c);
     if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(c->st));
+    if (int rc = drain(c)) return rc;
     double tot = 0;
     int64_t n = 0;
     for (size_t i = 0; i < c->ev_used; ++i) {
@@ -1500,8 +1801,7 @@ static int xfer_field(fdtd_ctx* c, SimHost& s, int field, double* out, const dou
     if (len != want) return fdtd_fail(FDTD_E_ARG, "length mismatch: expected " + std::to_string(want));
     if (n == 0) return FDTD_OK;
     std::vector<R> h(n);
-    HIPCHK(hipStreamSynchronize(c->st));
-    if (int rc = check_persist_flag(c)) return rc;
+    if (int rc = drain(c)) return rc;
     if (out) {
         HIPCHK(hipMemcpy(h.data(), src, sizeof(R) * n, hipMemcpyDeviceToHost));
         if (!strip) {
@@ -1539,8 +1839,7 @@ static int xfer_field(fdtd_ctx* c, SimHost& s, int field, double* out, const dou
 template <typename R>
 static int read_plain(fdtd_ctx* c, const R* src, int64_t n, double* out) {
     std::vector<R> h(n);
-    HIPCHK(hipStreamSynchronize(c->st));
-    if (int rc = check_persist_flag(c)) return rc;
+    if (int rc = drain(c)) return rc;
     if (n) HIPCHK(hipMemcpy(h.data(), src, sizeof(R) * n, hipMemcpyDeviceToHost));
     for (int64_t i = 0; i < n; ++i) out[i] = (double)h[i];
     return FDTD_OK;
@@ -1556,6 +1855,7 @@ extern "C" {
 int fdtd_read_field(fdtd_ctx* c, int id, int field, double* out, int64_t len) {
     SimHost* s = get_sim(c, id);
     if (!s || !out) return fdtd_fail(FDTD_E_ARG, "bad sim id or null out");
+    if (int rc = resolve_resident(c)) return rc;
     return c->prec == FDTD_F64 ? xfer_field<double>(c, *s, field, out, nullptr, len)
                                : xfer_field<float>(c, *s, field, out, nullptr, len);
 }
@@ -1563,6 +1863,7 @@ int fdtd_read_field(fdtd_ctx* c, int id, int field, double* out, int64_t len) {
 int fdtd_write_field(fdtd_ctx* c, int id, int field, const double* in, int64_t len) {
     SimHost* s = get_sim(c, id);
     if (!s || !in) return fdtd_fail(FDTD_E_ARG, "bad sim id or null input");
+    if (int rc = resolve_resident(c)) return rc;
     if (field == FDTD_FIELD_J) return fdtd_fail(FDTD_E_ARG, "J is written by the deposit");
     return c->prec == FDTD_F64 ? xfer_field<double>(c, *s, field, nullptr, in, len)
                                : xfer_field<float>(c, *s, field, nullptr, in, len);
@@ -1571,6 +1872,7 @@ int fdtd_write_field(fdtd_ctx* c, int id, int field, const double* in, int64_t l
 int fdtd_read_probes(fdtd_ctx* c, int id, double* out, int64_t len) {
     SimHost* s = get_sim(c, id);
     if (!s || !out) return fdtd_fail(FDTD_E_ARG, "bad sim id or null out");
+    if (int rc = resolve_resident(c)) return rc;
     const int64_t n = (int64_t)s->d.nprobe * s->d.steps;
     if (len != n) return fdtd_fail(FDTD_E_ARG, "length mismatch: expected " + std::to_string(n));
     if (c->prec == FDTD_F64) { SimDev<double> d; fill_dev<double>(*s, d); return read_plain<double>(c, d.probe_out, n, out); }
@@ -1580,6 +1882,7 @@ int fdtd_read_probes(fdtd_ctx* c, int id, double* out, int64_t len) {
 int fdtd_read_snapshots(fdtd_ctx* c, int id, double* out, int64_t len) {
     SimHost* s = get_sim(c, id);
     if (!s || !out) return fdtd_fail(FDTD_E_ARG, "bad sim id or null out");
+    if (int rc = resolve_resident(c)) return rc;
     const int64_t n = (int64_t)s->d.snap_rows * (s->d.N + 1);
     if (len != n) return fdtd_fail(FDTD_E_ARG, "length mismatch: expected " + std::to_string(n));
     if (c->prec == FDTD_F64) { SimDev<double> d; fill_dev<double>(*s, d); return read_plain<double>(c, d.snap, n, out); }
@@ -1598,7 +1901,7 @@ static int read_beam(fdtd_ctx* c, SimHost& s, BeamHost& b, double* x, double* u,
     const int N = s.d.N;
     std::vector<int32_t> cl(n), id(n);
     std::vector<R> fr(n), ux(n), uy(n), uz(n);
-    HIPCHK(hipStreamSynchronize(c->st));
+    if (int rc = drain(c)) return rc;
     int rc = check_pic_flag(c);
     if (rc) return rc;
     const char* blk = (const char*)b.block;
@@ -1672,6 +1975,7 @@ int pic_read(fdtd_ctx* c, int id, double* x, double* u, int8_t* alive, int64_t n
 // its FP64 samples, and lengths; host side).
 template <typename R>
 static int spectra_series(fdtd_ctx* c, int nsims, const int* ids, int probe, const double** ptrs, int* lens) {
+    if (int rc = resolve_resident(c)) return rc;
     for (int k = 0; k < nsims; ++k) {
         SimHost* s = get_sim(c, ids[k]);
         if (!s) return fdtd_fail(FDTD_E_ARG, "bad sim id " + std::to_string(ids[k]));
@@ -1698,7 +2002,7 @@ static int spectra_run(fdtd_ctx* c, int nsims, const double* const* ptrs, const 
         if (e != hipSuccess) return fdtd_fail(FDTD_E_HIP, std::string("dft launch: ") + hipGetErrorString(e));
     }
     HIPCHK(hipMemcpyAsync(out, d_out, sizeof(double) * 2 * (size_t)nsims * nf, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
+    if (int rc = drain(c)) return rc;
     return FDTD_OK;
 }
 
@@ -1821,7 +2125,7 @@ extern "C" int fdtd_step_op(fdtd_ctx* c, int op, int narr, double* const* arrays
     if (e != hipSuccess) return fdtd_fail(FDTD_E_HIP, std::string("op launch: ") + hipGetErrorString(e));
     for (int k = 0; k < o.nout; ++k)
         if (lens[k]) HIPCHK(hipMemcpyAsync(arrays[k], g.a[k], sizeof(double) * lens[k], hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
+    if (int rc = drain(c)) return rc;
     (void)total;
     return FDTD_OK;
 }

@@ -15,6 +15,7 @@ struct SimHost {
     size_t bytes = 0;
     size_t lay_off[64] = {0};   // byte offsets of the sub-arrays inside block
     int ns = 0, nstrip = 0;     // slab cells, strip cells
+    bool last_dead = false;     // cell N has zero coefficients and no source: its fields stay as they are
     long long launch_begin = 0; // context launch index at admission (ping-pong parity base)
     long long t_begin = 0;      // context global step at admission
     long long steps_done = 0;
@@ -56,6 +57,20 @@ struct EvPair {
 struct TileGroup {
     int kind, offset, count;    // tiles [offset, offset+count) run the kernel for this slab kind
 };
+
+// State of the host's counters before a resident launch, to go back to when
+// the launch gave up.
+struct ResPending {
+    int ordinal;
+    long long launch_idx, gstep, nsteps;
+    struct Sim { int id; long long steps_done, launches; };
+    std::vector<Sim> sims;
+};
+
+// Bound of one wait for a neighbour inside a resident launch (50 ms of polls
+// of about 0.5 us), and the most steps of one such launch.
+constexpr int kResMaxPolls = 100000;
+constexpr long long kResMaxSteps = 1 << 20;
 
 struct fdtd_ctx {
     int prec = FDTD_F64;
@@ -109,19 +124,30 @@ struct fdtd_ctx {
     size_t throttle_head = 0;
     long long throttle_launches = 0;
     int32_t* d_err = nullptr;                // index-check flag of the sort kernel
-    // persistent field launches (fdtd_set_persistent)
-    bool persist = false;                    // requested
-    bool persist_ok = false;                 // the current tile list qualifies
+    bool persist = false;                    // fdtd_set_persistent: requested
+    bool persist_ok = false;                 // the current tiling meets that request's conditions
+    // resident field launches (ResArgs)
+    int res_mode = 1;                        // fdtd_set_resident
+    int res_polls = kResMaxPolls;
+    bool res_ok = false;                     // the active simulations fit (res_tiles, res_S, res_kind)
+    std::vector<int4> res_tiles;
+    int res_S = 0, res_kind = 0, res_stride = 0, res_W = 1, res_cap = 0;
+    int4* d_rtiles = nullptr;
+    size_t d_rtiles_cap = 0;
+    unsigned long long* d_box = nullptr;     // two mailbox sets
+    size_t d_box_cap = 0;
+    int box_set = 0;
+    bool box_stale = true;                   // to be emptied before the next resident launch
+    int32_t* d_rerr = nullptr;               // ordinal of the launch that gave up (0: none)
+    int32_t* h_rerr = nullptr;               // the same in host memory
+    int res_ordinal = 0;
+    std::vector<ResPending> res_pending;     // resident launches not yet known to have finished
+    hipEvent_t res_ev = nullptr;             // recorded after the last resident launch
     int cu_count = 0;
     int lds_max = 0;            // shared memory a workgroup may use (bytes; 0: unknown)
     int pc_rows = 0;            // forced LDS rows per cell of the one-cell PIC kernel (0: chosen per launch)
     int pc_xr = 1;              // the rows of the current tile list's launches
     int pc_single = -1;         // the one-cell items' beam when there is one, else -1
-    unsigned long long* d_flags = nullptr;   // per tile: last block finished (global launch index + 1)
-    size_t d_flags_cap = 0;
-    int2* d_nbr = nullptr;                   // per tile: left, right neighbour tile
-    size_t d_nbr_cap = 0;
-    int32_t* d_perr = nullptr;               // set by a tile whose neighbour wait timed out
     void* d_scratch = nullptr;               // spectra: pointer table, frequencies, results
     size_t d_scratch_cap = 0;
 };
@@ -145,12 +171,6 @@ constexpr long long kCoopGroupsPerCu = sizeof(R) == 4 ? 6 : 4;
 
 // Largest field launch (tiles) that takes the particle scatter into its grid.
 constexpr int kFuseMaxTiles = 2048;
-
-// Blocks of S steps in one persistent field launch (bounded so that a long
-// run still returns control to the host now and then), and the bound on one
-// neighbour wait inside it (2 s of the 100 MHz real-time counter).
-constexpr int kPersistMaxBlocks = 4096;
-constexpr long long kPersistSpinTicks = 200000000LL;
 
 constexpr int kThrottleEvery = 128;
 constexpr size_t kThrottleDepth = 4;

@@ -124,7 +124,7 @@ template <typename R, bool KAHAN, bool HASJ>
 __device__ __forceinline__ KerrZ<R> slab_u(R kD, R jD, R dH, R Jv, R E, R& D, R& cD, R& P, R& Pm, R& cP,
                                            R sA, R sB, R sC) {
     if constexpr (sizeof(R) == 4) {
-        const R Vn = sA * Pm - sB * P + sC * E;
+        const R Vn = __builtin_fmaf(sC, E, __builtin_fmaf(sA, Pm, -(sB * P)));
         Pm = Vn;
         if (KAHAN) kahan_add(P, cP, Vn); else P = P + Vn;
     } else {
@@ -303,9 +303,23 @@ __device__ __forceinline__ void e_pure_slab(TILE_PARAMS, const TileCtx<R>& c, co
     if constexpr (KIND == SLAB_KERR_E) kerr_fixup<R, K>(E, x, z, ied, c.chi3);
 }
 
+// psi' = b psi + c d of the CPML.  FP64 fuses b psi.  FP32 rounds as the
+// compiler fused the one-block loops: FORM < 0 leaves it to the compiler (the
+// one-block kernels themselves); a resident tile writes the fused product out:
+// b psi (0), or c d (1), which those loops fuse in the E half of a tile's
+// cells 1 .. K-1 at the even steps of a launch, and nowhere else (read from
+// the compiled loops of K = 1, 2 and 4; the tests hold resident FP32 runs to
+// the one-block runs bit for bit).
+template <int FORM, typename R>
+__device__ __forceinline__ R psi_next(R b, R psi, R c, R d) {
+    if constexpr (FORM < 0 || sizeof(R) == 8) return fmr(b, psi, c * d);
+    else if constexpr (FORM == 0) return __builtin_fmaf(b, psi, c * d);
+    else return __builtin_fmaf(c, d, b * psi);
+}
+
 // Mixed tile: every cell takes the interior update (+ CPML psi), slab cells
 // then take E from D - P through selects.
-template <typename R, int K, bool KAHAN, int KIND, bool STRIP, bool HASJ>
+template <typename R, int K, bool KAHAN, int KIND, bool STRIP, bool HASJ, int FORM = -1>
 __device__ __forceinline__ void e_mixed(TILE_PARAMS, const TileCtx<R>& c, const SimDev<R>& sd,
                                         const R (&dH)[K], const R (&Jv)[K]) {
     R Ev[K], cEv[K];
@@ -315,7 +329,8 @@ __device__ __forceinline__ void e_mixed(TILE_PARAMS, const TileCtx<R>& c, const 
         const R a = dH[j] - Jv[j];
         if (KAHAN) kahan_fma(Ev[j], cEv[j], a, ke[j]); else Ev[j] = fmr(a, ke[j], Ev[j]);
         if (STRIP) {
-            psE[j] = fmr(bE[j], psE[j], cEc[j] * dH[j]);
+            psE[j] = j == 0 ? psi_next<(FORM < 0 ? -1 : 0)>(bE[j], psE[j], cEc[j], dH[j])
+                            : psi_next<FORM>(bE[j], psE[j], cEc[j], dH[j]);
             Ev[j] = fmr(-CbE[j], psE[j], Ev[j]);
         }
     }
@@ -347,8 +362,21 @@ __device__ __forceinline__ void e_mixed(TILE_PARAMS, const TileCtx<R>& c, const 
     }
 }
 
+// Source and TFSF values of up to 64 steps, one step per lane.
+template <typename R>
+struct SrcChunk {
+    R E, H;
+    __device__ __forceinline__ void load(const TileCtx<R>& c, int t_first, int n) {
+        E = (c.lane < n && c.src_lane >= 0) ? c.srcE[t_first + c.lane] : R(0);
+        H = (c.lane < n && c.tf_lane >= 0) ? c.srcH[t_first + c.lane] : R(0);
+    }
+};
+
+// Steps c.s_lo .. c.s_hi-1.  pre: the source values, when the caller has
+// loaded them (a resident tile does while it waits for its halos).
 template <typename R, int K, bool KAHAN, int KIND, int MODE>
-__device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, const SimDev<R>& sd) {
+__device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, const SimDev<R>& sd,
+                                          const SrcChunk<R>* pre = nullptr) {
     constexpr bool SLAB_CODE = (MODE & (M_PURE_SLAB | M_MIXED)) != 0 && KIND >= SLAB_LINEAR;
     constexpr bool STRIP = (MODE & M_STRIP) != 0;
     constexpr bool SRC = (MODE & M_SRC) != 0;
@@ -379,6 +407,11 @@ __device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, cons
         }
 #pragma unroll
         for (int q = 0; q < kChunks; ++q) {
+            if (pre) {
+                srcEc[q] = q == 0 ? pre->E : R(0);      // at most 64 steps
+                srcHc[q] = q == 0 ? pre->H : R(0);
+                continue;
+            }
             const int ix = q * 64 + c.lane;
             const bool in = ix < (c.s_hi - c.s_lo);
             srcEc[q] = (in && c.src_lane >= 0) ? c.srcE[c.t_first + ix] : R(0);
@@ -534,49 +567,144 @@ __device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, cons
     if (s < c.s_hi) step(s);
 }
 
-// Wave-uniform copy of a 64-bit value (both halves through readfirstlane).
-__device__ __forceinline__ unsigned long long wave_uniform(unsigned long long v) {
-    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v & 0xffffffffull));
-    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
-    return ((unsigned long long)hi << 32) | lo;
+// Steps of a resident tile: the arithmetic of run_steps, cell by cell
+// and in its order, with the rest of the loop cut to what a block of at most
+// 64 steps needs.  The slowest tile of a launch sets the pace of all of them,
+// and with run_steps that was one tile at the grid's end: a CPML strip tile
+// of one cell per lane took 150 ns a step in FP64, a slab tile 57.  So here a tile
+// without source or probe has a class of its own, probe rows are written
+// without a branch (lanes that hold no probe write a spare word of their own)
+// and go out after the loop, and one chunk of source values needs no
+// rotation.
+constexpr int kResMaxS = 60;
+template <typename R, int K, bool KAHAN, int KIND, int MODE>
+__device__ __forceinline__ void res_steps(TILE_PARAMS, const TileCtx<R>& c, const SimDev<R>& sd,
+                                          const SrcChunk<R>& src, R* spare, const int n) {
+    constexpr bool SLAB_CODE = (MODE & (M_PURE_SLAB | M_MIXED)) != 0 && KIND >= SLAB_LINEAR;
+    constexpr bool STRIP = (MODE & M_STRIP) != 0;
+    constexpr bool SRC = (MODE & M_SRC) != 0;
+    constexpr bool PROBE = (MODE & M_PROBE) != 0;
+    R ms[K], mt[K], Jv[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) Jv[j] = R(0);
+    if constexpr (SRC) {
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            ms[j] = (c.src_lane >= 0 && c.lane == c.src_lane && j == c.src_j) ? R(1) : R(0);
+            mt[j] = (c.tf_lane >= 0 && c.lane == c.tf_lane && j == c.tf_j) ? R(1) : R(0);
+        }
+    }
+    // a probe's rows: E, then (FP32) its Kahan compensation 64 words on
+    R* row[2];
+    int inc[2];
+    if constexpr (PROBE) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const bool mine = k < c.npr && c.lane == c.pr_rel[k] / K;
+            row[k] = mine ? &c.prl[k][0][0] : spare + c.lane;
+            inc[k] = mine ? 1 : 0;
+        }
+    }
+    auto step = [&](const int s, auto form) {
+        constexpr int FORM = decltype(form)::value;
+        const R Hl = shr1(H[K - 1]);
+        R dH[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) dH[j] = H[j] - ((j == 0) ? Hl : H[j - 1]);
+        if constexpr (SLAB_CODE && (MODE & M_PURE_SLAB) && !STRIP) {
+            e_pure_slab<R, K, KAHAN, KIND, false>(TILE_ARGS, c, sd, dH, Jv);
+        } else if constexpr (SLAB_CODE) {
+            e_mixed<R, K, KAHAN, KIND, STRIP, false, FORM>(TILE_ARGS, c, sd, dH, Jv);
+        } else {
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                if (KAHAN) kahan_fma(E[j], cE[j], dH[j], ke[j]); else E[j] = fmr(dH[j], ke[j], E[j]);
+                if (STRIP) {
+                    psE[j] = j == 0 ? psi_next<0>(bE[j], psE[j], cEc[j], dH[j])
+                                    : psi_next<FORM>(bE[j], psE[j], cEc[j], dH[j]);
+                    E[j] = fmr(-CbE[j], psE[j], E[j]);
+                }
+            }
+        }
+        if constexpr (SRC) {
+            const R sv = lane_read(src.E, s);
+#pragma unroll
+            for (int j = 0; j < K; ++j) E[j] = fmr(ms[j], sv, E[j]);
+            if (c.tf_lane >= 0) {
+                const R hv = lane_read(src.H, s);
+#pragma unroll
+                for (int j = 0; j < K; ++j) H[j] = fmr(-mt[j], hv, H[j]);
+            }
+        }
+        const R Er = shl1(E[0]);
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const R dE = ((j == K - 1) ? Er : E[j + 1]) - E[j];
+            if (KAHAN) kahan_fma(H[j], cH[j], dE, kh[j]); else H[j] = fmr(dE, kh[j], H[j]);
+            if (STRIP) {
+                psH[j] = psi_next<0>(bH[j], psH[j], cHc[j], dE);
+                H[j] = fmr(C2H[j], psH[j], H[j]);
+            }
+        }
+        if constexpr (PROBE) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                row[k][0] = pick<R, K>(E, c.pr_rel[k] % K);
+                if (KAHAN) row[k][64] = pick<R, K>(cE, c.pr_rel[k] % K);
+                row[k] += inc[k];
+            }
+        }
+    };
+    int s = 0;
+    for (; s + 1 < n; s += 2) {
+        step(s, std::integral_constant<int, 1>{});
+        step(s + 1, std::integral_constant<int, 0>{});
+    }
+    if (s < n) step(s, std::integral_constant<int, 1>{});
+    if constexpr (PROBE) {
+        // the owning lanes' LDS stores come before the other lanes' reads
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int tt = c.t_first + c.lane;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (k < c.npr && c.lane < n && tt >= c.pr_t0[k] && tt <= c.pr_t1[k])
+                c.probe_out[(long long)c.pr_id[k] * c.T + tt] =
+                    KAHAN ? (double)c.prl[k][0][c.lane] - (double)c.prl[k][1][c.lane] : (double)c.prl[k][0][c.lane];
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
 }
 
-// Device-coherent loads and stores of the persistent halo exchange: relaxed
-// atomics at agent scope are issued with the device-scope cache bits, so each
-// access is coherent across the XCDs' L2 caches by itself, and no fence has to
-// write back or invalidate a whole L2 (an agent-scope fence per block and
-// tile made a 42-step block take 55 us against 12.8 us for a one-block launch).
-template <typename T>
-__device__ __forceinline__ T ld_dev(const T* p) {
-    return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Device-coherent loads and stores of the resident hand-off: relaxed atomics
+// at agent scope are issued with the device-scope cache bits, so each access
+// is coherent across the XCDs' L2 caches by itself, and no fence has to write
+// back or invalidate a whole L2 (an agent-scope fence per block and tile made
+// a 42-step block take 55 us against 12.8 us for a one-block launch).
+__device__ __forceinline__ unsigned long long ld_dev(const unsigned long long* p) {
+    return __hip_atomic_load(const_cast<unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-template <typename T>
-__device__ __forceinline__ void st_dev(T* p, T v) {
+__device__ __forceinline__ void st_dev(unsigned long long* p, unsigned long long v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-// Waits (wave-uniform) until *flag >= need; false when the real-time counter
-// passes deadline first.  The halo loads that follow are device-scope loads
-// issued after the flag was seen; the workgroup-scope acquire orders them
-// after it (it waits for the flag load and drops this CU's L1 lines).
-__device__ __forceinline__ bool wait_flag(unsigned long long* flag, unsigned long long need, long long deadline) {
-    for (;;) {
-        const unsigned long long v = wave_uniform(ld_dev(flag));
-        if (v >= need) break;
-        if ((long long)__builtin_amdgcn_s_memrealtime() > deadline) return false;
-        __builtin_amdgcn_s_sleep(2);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    return true;
+// Mailbox words: a value (FP64) or a pair of values (FP32).
+__device__ __forceinline__ unsigned long long pack2(double a, double) { return (unsigned long long)__double_as_longlong(a); }
+__device__ __forceinline__ unsigned long long pack2(float a, float b) {
+    return ((unsigned long long)__float_as_uint(b) << 32) | __float_as_uint(a);
+}
+__device__ __forceinline__ void unpack2(unsigned long long w, double& a, double&) { a = __longlong_as_double((long long)w); }
+__device__ __forceinline__ void unpack2(unsigned long long w, float& a, float& b) {
+    a = __uint_as_float((unsigned)(w & 0xffffffffull));
+    b = __uint_as_float((unsigned)(w >> 32));
 }
 
 // One tile: 64 lanes x K cells, S steps (the whole per-tile program); with
-// PERSIST, pa.nblocks blocks of S steps with the neighbour exchange between
-// them (a separate instance: the one-block kernel keeps its own register
-// allocation).
-template <typename R, int K, bool KAHAN, int KIND, bool PERSIST, bool GROUP = false>
+// RES, tile rt of a resident launch (ResArgs): all of the launch's steps, in
+// blocks of S with the hand-off between them (a separate instance: the
+// one-block kernel keeps its own register allocation).
+template <typename R, int K, bool KAHAN, int KIND, bool RES, bool GROUP = false>
 __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long long launch_idx, long long gstep0,
-                                          int nsteps, int S, int tid, const PersistArgs& pa) {
+                                          int nsteps, int S, const PersistArgs& pa, const int4 rt, const ResArgs& ra) {
     constexpr bool DFORM = KIND >= SLAB_LINEAR;
     const int lane = wave_lane();
     // the window [t0, t0 + 64K) and the cells it owns (writes back, probes):
@@ -588,7 +716,8 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
     const int hx = GROUP ? pa.halo : 0;
     const int t0 = GROUP ? out0_ : out0_ - S;
     const int out0 = GROUP ? t0 + (wv == 0 ? S : hx) : out0_;
-    const int U = GROUP ? 64 * K - (wv == 0 ? S : hx) - (wv == kTileWaves - 1 ? S : hx) : 64 * K - 2 * S;
+    const int U = RES ? rt.z - rt.y
+                  : GROUP ? 64 * K - (wv == 0 ? S : hx) - (wv == kTileWaves - 1 ? S : hx) : 64 * K - 2 * S;
     const int N = sd.N;
     const int par = (int)((launch_idx - sd.launch_begin) & 1);
     const int F = sd.F, Rr = sd.Rr, Ls = sd.Ls, Rs = sd.Rs;
@@ -599,7 +728,8 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
     TileCtx<R> c;
     // probe sample rows, one set per wave of the 256-thread workgroup
     __shared__ R pr_rows[kTileWaves][2][2][64];
-    c.prl = pr_rows[__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))];
+    const int wvi = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    c.prl = pr_rows[wvi];
     c.lane = lane;
     c.t0 = t0;
     c.wv = wv;
@@ -625,7 +755,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
         // from clamped cells without waiting for the live range, which only
         // masks them afterwards (the sum of j_from_sums, in its order).
         double raw[K <= 2 ? K : 1][4];
-        if constexpr (K <= 2 && !PERSIST) {
+        if constexpr (K <= 2 && !RES) {
 #pragma unroll
             for (int j = 0; j < K; ++j)
 #pragma unroll
@@ -636,7 +766,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
         }
         c.pcmin = sd.prange[par][0];
         c.pcmax = sd.prange[par][1];
-        if constexpr (K <= 2 && !PERSIST) {
+        if constexpr (K <= 2 && !RES) {
             c.jpre = true;
 #pragma unroll
             for (int j = 0; j < K; ++j) {
@@ -666,7 +796,8 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
 #pragma unroll
     for (int j = 0; j < K; ++j) {
         const int n = c.base + j;
-        const bool valid = (n >= 0) && (n <= N);
+        // a resident tile may own fewer cells than its window holds; the rest stays zero
+        const bool valid = (n >= 0) && (n <= N) && (!RES || n < out0 + U + S);
         E[j] = valid ? Ein[n] : R(0);
         H[j] = valid ? Hin[n] : R(0);
         cE[j] = cH[j] = R(0);
@@ -704,10 +835,12 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
     const bool any_slab = DFORM && __any(slab_mask != 0);
     const int tile_end = c.t0 + 64 * K;
     const int src = sd.src_cell;
-    const bool tile_src = src >= c.t0 && src < tile_end;
+    // (a resident tile's idle cells take no source)
+    const int src_end = RES ? min(tile_end, out0 + U + S) : tile_end;
+    const bool tile_src = src >= c.t0 && src < src_end;
     c.src_lane = tile_src ? (src - c.t0) / K : -1;
     c.src_j = tile_src ? (src - c.t0) % K : 0;
-    const bool tile_tf = sd.tfsf && (src - 1) >= c.t0 && (src - 1) < tile_end;
+    const bool tile_tf = sd.tfsf && (src - 1) >= c.t0 && (src - 1) < src_end;
     c.tf_lane = tile_tf ? (src - 1 - c.t0) / K : -1;
     c.tf_j = tile_tf ? (src - 1 - c.t0) % K : 0;
     c.probe_bits = 0;
@@ -747,7 +880,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
         cD[j] = cE[j];
         P[j] = Pm[j] = cP[j] = R(0);
     };
-    if constexpr (KIND == SLAB_KERR_E) {
+    if constexpr (KIND == SLAB_KERR_E || (RES && sizeof(R) == 8 && KIND == SLAB_LINEAR)) {
         const bool all_valid = __all(c.base >= 0 && c.base + K - 1 <= N);
         emu_tile = any_slab && !pure_slab && !extras && !gen && all_valid && sd.ke0 == sd.kD && sd.jD == R(1);
         if (emu_tile) {
@@ -764,93 +897,234 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
         }
     }
 
-    const int nblocks = PERSIST ? pa.nblocks : 1;
-    for (int blk = 0; blk < nblocks; ++blk) {
-        const long long li = launch_idx + blk;             // this block's global launch index
-        const int pb = (int)((li - sd.launch_begin) & 1);  // the buffer it reads
-        if (PERSIST && blk > 0) {
-            // both neighbours have written block li - 1: reload the halo cells
-            // (outside the interior), which lie in their interiors
-            const int2 nb = pa.nbr[tid];
-            const long long deadline = (long long)__builtin_amdgcn_s_memrealtime() + pa.spin_ticks;
-            bool ok = true;
-            if (nb.x >= 0) ok = wait_flag(pa.flags + nb.x, (unsigned long long)li, deadline);
-            if (ok && nb.y >= 0) ok = wait_flag(pa.flags + nb.y, (unsigned long long)li, deadline);
-            if (!ok) {
-                if (lane == 0) __hip_atomic_store(pa.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                return;
+    // the launch's steps of this simulation: local steps 0 .. total-1, the
+    // first at the simulation's step t0s
+    const long long lo = max(0LL, (long long)sd.t_begin - gstep0);
+    const int total = (int)max(0LL, min((long long)nsteps, (long long)c.T + sd.t_begin - gstep0) - lo);
+    const int t0s = (int)(gstep0 + lo - sd.t_begin);
+    c.emu_mask = emu_mask;
+    auto run = [&](const SrcChunk<R>* pre) {
+        constexpr int GM = GROUP ? M_GROUP : 0;
+        if (gen || RES)      // resident tiles: the general class only (FP64)
+            run_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP | M_SRC | M_GENERAL | GM>(TILE_ARGS, c, sd, pre);
+        else if ((pure_slab || emu_tile) && !extras)
+            run_steps<R, K, KAHAN, KIND, M_PURE_SLAB | GM>(TILE_ARGS, c, sd, pre);
+        else if (!any_slab && !extras)
+            run_steps<R, K, KAHAN, KIND, GM>(TILE_ARGS, c, sd, pre);
+        else if (!any_slab)
+            run_steps<R, K, KAHAN, KIND, M_STRIP | M_SRC | M_PROBE | GM>(TILE_ARGS, c, sd, pre);
+        else
+            run_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP | M_SRC | M_PROBE | GM>(TILE_ARGS, c, sd, pre);
+    };
+    // the compensation of E (FP32); an emulated vacuum cell carries it in cD: E - cE = D - cD
+    auto comp_e = [&](int j) {
+        return ((emu_mask >> j) & 1u) ? (R)((double)E[j] - ((double)D[j] - (double)cD[j])) : cE[j];
+    };
+    if constexpr (!RES) {
+        c.s_lo = (int)lo;
+        c.s_hi = (int)lo + total;
+        c.t_first = t0s;
+        run(nullptr);
+    } else {
+        // the words of this lane's cells: sent cells are owned and within S of
+        // a neighbour, received cells are the valid ones off the interior;
+        // lanes without one address the mailbox's spare cell, which is never
+        // empty, so the loads need no branch
+        const int spare = ra.stride - 1;
+        const bool has_l = out0 > 0, has_r = out0 + U <= N;
+        const bool any_strip = tile_strip;
+        unsigned send = 0;
+        int rv[K], rs[K], rp[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const int n = c.base + j;
+            const bool own = (interior_mask >> j) & 1u;
+            if (own && ((has_l && n < out0 + S) || (has_r && n >= out0 + U - S))) send |= 1u << j;
+            const bool rec = !own && n >= 0 && n <= N && n < out0 + U + S;
+            rv[j] = rec ? rt.w + n : spare;
+            rs[j] = rec && ((slab_mask >> j) & 1u) ? rt.w + n : spare;
+            rp[j] = rec && ((strip_mask >> j) & 1u) ? rt.w + n : spare;
+        }
+        constexpr int NV = kResValues<R>;
+        const size_t slot_words = (size_t)NV * ra.stride;
+        // every word of a cell this tile sends: w(v) is the word of value v
+        auto words = [&](int j, auto&& f) {
+            const int n = rt.w + c.base + j;
+            f(0, n); f(1, n);
+            if ((slab_mask >> j) & 1u) { f(2, n); f(3, n); f(4, n); }
+            if ((strip_mask >> j) & 1u) { f(5, n); if (NV > 6) f(NV - 1, n); }
+        };
+        auto empty = [&](unsigned long long* slot) {
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                if ((send >> j) & 1u)
+                    words(j, [&](int v, int n) { st_dev(slot + (size_t)v * ra.stride + n, kResEmpty); });
+        };
+        // what the launch before this one left in the other set
+        for (int q = 0; q < 3; ++q) empty(ra.other + q * slot_words);
+        SrcChunk<R> sc;
+        const int snap_interval = c.snap_interval;
+        c.snap_interval = 0;
+        c.s_lo = 0;
+        sc.load(c, t0s, min(S, total));
+        int q = 0;           // hand-offs so far; q3 = q % 3
+        int q3 = 0;
+        for (int k0 = 0; k0 < total;) {
+            // A block is cut at its snapshot steps: the lean loops run up to
+            // and including a snapshot step, then the row is stored from
+            // registers (t = 0 takes none).
+            const int kend = min(k0 + S, total);
+            bool fresh = true;
+            while (k0 < kend) {
+                int k1 = kend;
+                bool row = false;
+                if (snap_interval > 0) {
+                    const int t = max(t0s + k0, 1);
+                    const int ts = (t + snap_interval - 1) / snap_interval * snap_interval;
+                    if (ts - t0s < k1) {
+                        k1 = ts - t0s + 1;
+                        row = ts / snap_interval < c.snap_rows;
+                    }
+                }
+                c.t_first = t0s + k0;
+                c.s_hi = k1 - k0;
+                if (!fresh) sc.load(c, c.t_first, c.s_hi);
+                fresh = false;
+                {
+                    __shared__ R spare_rows[kTileWaves][2][64];
+                    R* sp = &spare_rows[wvi][0][0];
+                    const int n = c.s_hi;
+                    const bool srcs = tile_src || tile_tf, prb = c.npr > 0, ends = srcs || prb;
+                    if constexpr (K == 4 && sizeof(R) == 8)      // light tiles: plain cells only
+                        res_steps<R, K, KAHAN, KIND, 0>(TILE_ARGS, c, sd, sc, sp, n);
+                    else if (sizeof(R) == 8 && gen)
+                        run(&sc);
+                    else if ((pure_slab || emu_tile) && !extras)
+                        res_steps<R, K, KAHAN, KIND, M_PURE_SLAB>(TILE_ARGS, c, sd, sc, sp, n);
+                    else if (!any_slab && !extras)
+                        res_steps<R, K, KAHAN, KIND, 0>(TILE_ARGS, c, sd, sc, sp, n);
+                    else if (!any_slab && !ends)
+                        res_steps<R, K, KAHAN, KIND, M_STRIP>(TILE_ARGS, c, sd, sc, sp, n);
+                    else if (!any_slab && !prb)
+                        res_steps<R, K, KAHAN, KIND, M_STRIP | M_SRC>(TILE_ARGS, c, sd, sc, sp, n);
+                    else if (!any_slab && !srcs)
+                        res_steps<R, K, KAHAN, KIND, M_STRIP | M_PROBE>(TILE_ARGS, c, sd, sc, sp, n);
+                    else if (!any_slab)
+                        res_steps<R, K, KAHAN, KIND, M_STRIP | M_SRC | M_PROBE>(TILE_ARGS, c, sd, sc, sp, n);
+                    else if (!ends)
+                        res_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP>(TILE_ARGS, c, sd, sc, sp, n);
+                    else
+                        res_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP | M_SRC | M_PROBE>(TILE_ARGS, c, sd, sc, sp, n);
+                }
+                if (row) {
+                    R* o = c.snap + (long long)((t0s + k1 - 1) / snap_interval) * (N + 1) + c.base;
+#pragma unroll
+                    for (int j = 0; j < K; ++j)
+                        if ((interior_mask >> j) & 1u) o[j] = E[j];
+                }
+                k0 = k1;
+            }
+            if (k0 >= total) break;
+            // ---- hand-off q ----
+            unsigned long long* slot = ra.box + q3 * slot_words;
+            // the emptied words of the slot to come are in memory before this block's values go out
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                if (!((send >> j) & 1u)) continue;
+                unsigned long long* o = slot + rt.w + c.base + j;
+                const size_t st = (size_t)ra.stride;
+                st_dev(o, pack2(E[j], KAHAN ? comp_e(j) : R(0)));
+                st_dev(o + st, pack2(H[j], cH[j]));
+                if ((slab_mask >> j) & 1u) {
+                    st_dev(o + 2 * st, pack2(D[j], cD[j]));
+                    st_dev(o + 3 * st, pack2(P[j], cP[j]));
+                    st_dev(o + 4 * st, pack2(Pm[j], R(0)));
+                }
+                if ((strip_mask >> j) & 1u) {
+                    st_dev(o + 5 * st, pack2(psE[j], psH[j]));
+                    if constexpr (sizeof(R) == 8) st_dev(o + 6 * st, pack2(psH[j], R(0)));
+                }
+            }
+            sc.load(c, t0s + k0, min(S, total - k0));
+            int polls = 0;
+            unsigned long long w[K][NV];
+            for (;;) {
+                bool here = true;
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    const size_t st = (size_t)ra.stride;
+                    w[j][0] = ld_dev(slot + rv[j]);
+                    w[j][1] = ld_dev(slot + st + rv[j]);
+                    if (any_slab) {
+#pragma unroll
+                        for (int v = 2; v < 5; ++v) w[j][v] = ld_dev(slot + v * st + rs[j]);
+                    }
+                    if (any_strip) {
+#pragma unroll
+                        for (int v = 5; v < NV; ++v) w[j][v] = ld_dev(slot + v * st + rp[j]);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    here = here && w[j][0] != kResEmpty && w[j][1] != kResEmpty;
+                    if (any_slab) here = here && w[j][2] != kResEmpty && w[j][3] != kResEmpty && w[j][4] != kResEmpty;
+                    if (any_strip) here = here && w[j][5] != kResEmpty && w[j][NV - 1] != kResEmpty;
+                }
+                if (__all(here)) break;
+                if (++polls > ra.max_polls) {
+                    if (lane == 0) {
+                        __hip_atomic_store(ra.err, ra.ordinal, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        __hip_atomic_store(ra.herr, ra.ordinal, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+                    return;
+                }
             }
 #pragma unroll
             for (int j = 0; j < K; ++j) {
-                const int n = c.base + j;
-                if (((interior_mask >> j) & 1u) || n < 0 || n > N) continue;
-                E[j] = ld_dev(sd.E[pb] + n);
-                H[j] = ld_dev(sd.H[pb] + n);
-                if (KAHAN) { cE[j] = ld_dev(sd.cE[pb] + n); cH[j] = ld_dev(sd.cH[pb] + n); }
-                if ((slab_mask >> j) & 1u) {
-                    const int i = n - F;
-                    D[j] = ld_dev(sd.D[pb] + i); P[j] = ld_dev(sd.P[pb] + i); Pm[j] = ld_dev(sd.Pm[pb] + i);
-                    if (KAHAN) { cD[j] = ld_dev(sd.cD[pb] + i); cP[j] = ld_dev(sd.cP[pb] + i); }
+                R none;
+                if (rv[j] != spare) {
+                    unpack2(w[j][0], E[j], cE[j]);
+                    unpack2(w[j][1], H[j], cH[j]);
+                    if ((emu_mask >> j) & 1u) emulate(j);
                 }
-                if ((strip_mask >> j) & 1u) {
-                    const int i = n < Ls ? n : Ls + (n - Rs);
-                    psE[j] = ld_dev(sd.psiE[pb] + i); psH[j] = ld_dev(sd.psiH[pb] + i);
+                if (any_slab && rs[j] != spare) {
+                    unpack2(w[j][2], D[j], cD[j]);
+                    unpack2(w[j][3], P[j], cP[j]);
+                    unpack2(w[j][4], Pm[j], none);
                 }
-                if ((emu_mask >> j) & 1u) emulate(j);
+                if (any_strip && rp[j] != spare) {
+                    unpack2(w[j][5], psE[j], psH[j]);
+                    if constexpr (sizeof(R) == 8) unpack2(w[j][NV - 1], psH[j], none);
+                }
             }
+            // hand-off q - 1 has been read by everyone who needs it
+            if (q > 0) empty(ra.box + (q3 == 0 ? 2 : q3 - 1) * slot_words);
+            ++q;
+            q3 = q3 == 2 ? 0 : q3 + 1;
         }
-        // valid local steps of this block: t = gstep + s - t_begin in [0, T)
-        const long long gs = gstep0 + (long long)blk * S;
-        c.gstep0 = gs;
-        c.s_lo = (int)max(0LL, c.t_begin - gs);
-        c.s_hi = (int)min((long long)nsteps, (long long)c.T + c.t_begin - gs);
-        c.t_first = (int)(gs + c.s_lo - c.t_begin);
-        constexpr int GM = GROUP ? M_GROUP : 0;
-        c.emu_mask = emu_mask;
-        if (gen)
-            run_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP | M_SRC | M_GENERAL | GM>(TILE_ARGS, c, sd);
-        else if ((pure_slab || emu_tile) && !extras)
-            run_steps<R, K, KAHAN, KIND, M_PURE_SLAB | GM>(TILE_ARGS, c, sd);
-        else if (!any_slab && !extras)
-            run_steps<R, K, KAHAN, KIND, GM>(TILE_ARGS, c, sd);
-        else if (!any_slab)
-            run_steps<R, K, KAHAN, KIND, M_STRIP | M_SRC | M_PROBE | GM>(TILE_ARGS, c, sd);
-        else
-            run_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP | M_SRC | M_PROBE | GM>(TILE_ARGS, c, sd);
+    }
 
-        // ---------------- write back the interior ----------------
-        // (persistent: device-scope stores, which the neighbours' halo loads see)
-        const int po = pb ^ 1;
-        auto put = [&](R* p, R v) {
-            if constexpr (PERSIST) st_dev(p, v); else *p = v;
-        };
+    // ---------------- write back the interior ----------------
+    const int po = par ^ 1;
 #pragma unroll
-        for (int j = 0; j < K; ++j) {
-            if (!((interior_mask >> j) & 1u)) continue;
-            const int n = c.base + j;
-            put(sd.E[po] + n, E[j]);
-            put(sd.H[po] + n, H[j]);
-            if (KAHAN) {
-                // an emulated vacuum cell carries its compensation in cD: E - cE = D - cD
-                const R ce = ((emu_mask >> j) & 1u) ? (R)((double)E[j] - ((double)D[j] - (double)cD[j])) : cE[j];
-                put(sd.cE[po] + n, ce);
-                put(sd.cH[po] + n, cH[j]);
-            }
-            if ((slab_mask >> j) & 1u) {
-                const int i = n - F;
-                put(sd.D[po] + i, D[j]); put(sd.P[po] + i, P[j]); put(sd.Pm[po] + i, Pm[j]);
-                if (KAHAN) { put(sd.cD[po] + i, cD[j]); put(sd.cP[po] + i, cP[j]); }
-            }
-            if ((strip_mask >> j) & 1u) {
-                const int i = n < Ls ? n : Ls + (n - Rs);
-                put(sd.psiE[po] + i, psE[j]); put(sd.psiH[po] + i, psH[j]);
-            }
+    for (int j = 0; j < K; ++j) {
+        if (!((interior_mask >> j) & 1u)) continue;
+        const int n = c.base + j;
+        sd.E[po][n] = E[j];
+        sd.H[po][n] = H[j];
+        if (KAHAN) {
+            sd.cE[po][n] = comp_e(j);
+            sd.cH[po][n] = cH[j];
         }
-        if constexpr (PERSIST) {
-            // publish: the workgroup-scope release waits until every lane's
-            // device-scope stores above have completed, then the flag goes out
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-            if (lane == 0) st_dev(pa.flags + tid, (unsigned long long)(li + 1));
+        if ((slab_mask >> j) & 1u) {
+            const int i = n - F;
+            sd.D[po][i] = D[j]; sd.P[po][i] = P[j]; sd.Pm[po][i] = Pm[j];
+            if (KAHAN) { sd.cD[po][i] = cD[j]; sd.cP[po][i] = cP[j]; }
+        }
+        if ((strip_mask >> j) & 1u) {
+            const int i = n < Ls ? n : Ls + (n - Rs);
+            sd.psiE[po][i] = psE[j]; sd.psiH[po][i] = psH[j];
         }
     }
 }
@@ -867,29 +1141,27 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
 // interior cell): narrow tiles hold KW/2 cells per lane, the others KW, so
 // tiles with costly slab cells can be made narrower than plain ones within
 // one launch.
-template <typename R, int KW, bool KAHAN, int KIND, bool PERSIST = false, bool GROUP = false>
+template <typename R, int KW, bool KAHAN, int KIND, bool GROUP = false>
 __device__ __forceinline__ void field_tile(const SimDev<R>* __restrict__ sims, const int2* __restrict__ tiles,
                                            int tid, long long launch_idx, long long gstep0, int nsteps, int S,
                                            const PersistArgs& pa) {
     const int2 tl = tiles[tid];
     const SimDev<R>& sd = sims[tl.x & 0xffffff];
-    if constexpr (GROUP) {
-        tile_body<R, KW, KAHAN, KIND, false, true>(sd, tl.y, launch_idx, gstep0, nsteps, S, tid, pa);
-        return;
-    }
-    if constexpr (KW > 1 && !PERSIST) {
+    const int4 rt{0, 0, 0, 0};
+    const ResArgs ra{};
+    if constexpr (KW > 1 && !GROUP) {
         if (tl.x >> 24) {
-            tile_body<R, KW / 2, KAHAN, KIND, false>(sd, tl.y, launch_idx, gstep0, nsteps, S, tid, pa);
+            tile_body<R, KW / 2, KAHAN, KIND, false>(sd, tl.y, launch_idx, gstep0, nsteps, S, pa, rt, ra);
             return;
         }
     }
-    tile_body<R, KW, KAHAN, KIND, PERSIST>(sd, tl.y, launch_idx, gstep0, nsteps, S, tid, pa);
+    tile_body<R, KW, KAHAN, KIND, false, GROUP>(sd, tl.y, launch_idx, gstep0, nsteps, S, pa, rt, ra);
 }
 
 // GROUP: the halo-exchange instance; its tile list holds whole workgroups
 // (ntiles a multiple of kTileWaves, every wave of a workgroup from one
 // simulation), so every wave reaches the exchange barriers.
-template <typename R, int KW, bool KAHAN, int KIND, bool PERSIST, bool GROUP = false>
+template <typename R, int KW, bool KAHAN, int KIND, bool GROUP = false>
 __global__ __launch_bounds__(64 * kTileWaves) void stencil_tiles(const SimDev<R>* __restrict__ sims,
                                                                  const int2* __restrict__ tiles, int ntiles,
                                                                  long long launch_idx, long long gstep0,
@@ -897,30 +1169,94 @@ __global__ __launch_bounds__(64 * kTileWaves) void stencil_tiles(const SimDev<R>
     // wave-uniform tile index, so the descriptors come in through scalar loads
     const int tid = kTileWaves * (int)blockIdx.x + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     if (tid >= ntiles) return;
-    field_tile<R, KW, KAHAN, KIND, PERSIST, GROUP>(sims, tiles, tid, launch_idx, gstep0, nsteps, S, pa);
+    field_tile<R, KW, KAHAN, KIND, GROUP>(sims, tiles, tid, launch_idx, gstep0, nsteps, S, pa);
+}
+
+// Resident launch: tile t is wave t % 4 of workgroup t / 4; W workgroups fit
+// on a CU.  RESDOC
+// FP64 tiles hold 1 or 2 cells per lane, plain ones up to 4; FP32 tiles are
+// the one-block tiles of the context's K: 1 and 2 with W = 2, 4 with W = 1.
+template <typename R, bool KAHAN, int KIND, int W>
+__global__ __launch_bounds__(64 * kTileWaves, W) void stencil_resident(const SimDev<R>* __restrict__ sims,
+                                                                       const int4* __restrict__ tiles, int ntiles,
+                                                                       long long launch_idx, long long gstep0,
+                                                                       ResArgs ra) {
+    const int tid = kTileWaves * (int)blockIdx.x + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (tid >= ntiles) return;
+    const int4 rt = tiles[tid];
+    const SimDev<R>& sd = sims[rt.x & 0xffffff];
+    if (*ra.err) return;      // an earlier launch gave up: the host runs these steps again
+    const PersistArgs pa{0};
+    auto body = [&](auto k, auto kind) {
+        tile_body<R, decltype(k)::value, KAHAN, decltype(kind)::value, true>(sd, rt.y, launch_idx, gstep0, ra.nsteps,
+                                                                             ra.S, pa, rt, ra);
+    };
+    using std::integral_constant;
+    using Kind = integral_constant<int, KIND>;
+    using Plain = integral_constant<int, SLAB_DIEL>;
+    using K1 = integral_constant<int, 1>;
+    using K2 = integral_constant<int, 2>;
+    using K4 = integral_constant<int, 4>;
+    const bool plain = KIND == SLAB_DIEL || (rt.x & kResPlain);
+    if constexpr (sizeof(R) == 4 && W == 1) {
+        if (!plain) body(K4{}, Kind{});
+        else body(K4{}, Plain{});
+    } else {
+        if (!plain) {
+            if (rt.x & kResK2) body(K2{}, Kind{});
+            else body(K1{}, Kind{});
+        } else if (sizeof(R) == 8 && (rt.x & kResK4)) {
+            if constexpr (sizeof(R) == 8) body(K4{}, Plain{});
+        } else if (rt.x & kResK2) {
+            body(K2{}, Plain{});
+        } else {
+            body(K1{}, Plain{});
+        }
+    }
+}
+
+template <typename R, bool KAHAN, int KIND>
+hipError_t launch_resident_kind(const SimDev<R>* sims, const int4* tiles, int ntiles, long long launch_idx,
+                                long long gstep0, int W, const ResArgs& ra, hipStream_t st) {
+    const dim3 grid((ntiles + kTileWaves - 1) / kTileWaves), block(64 * kTileWaves);
+    if (W == 1)
+        hipLaunchKernelGGL((stencil_resident<R, KAHAN, KIND, 1>), grid, block, 0, st, sims, tiles, ntiles, launch_idx,
+                           gstep0, ra);
+    else
+        hipLaunchKernelGGL((stencil_resident<R, KAHAN, KIND, 2>), grid, block, 0, st, sims, tiles, ntiles, launch_idx,
+                           gstep0, ra);
+    return hipGetLastError();
+}
+
+// Workgroups of the resident kernel that one CU holds at once (register and
+// LDS limits).
+template <typename R, bool KAHAN, int KIND>
+int resident_per_cu(int W) {
+    int nb = 0;
+    const hipError_t e =
+        W == 1 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, stencil_resident<R, KAHAN, KIND, 1>, 64 * kTileWaves, 0)
+               : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, stencil_resident<R, KAHAN, KIND, 2>, 64 * kTileWaves, 0);
+    return e == hipSuccess ? nb : 0;
 }
 
 // Host-side launcher (called from host.hip).
 // With profiling events the launch goes through hipExtLaunchKernelGGL, which
 // stamps ev0/ev1 from the kernel's own dispatch packet (kernel execution time
 // only, the figure a kernel trace reports).
-template <typename R, int K, bool KAHAN, int KIND, bool PERSIST, bool GROUP = false>
+template <typename R, int K, bool KAHAN, int KIND, bool GROUP = false>
 static hipError_t launch_kp(const SimDev<R>* sims, const int2* tiles, int ntiles, long long launch_idx,
                             long long gstep0, int nsteps, int S, const PersistArgs& pa, hipStream_t st,
                             hipEvent_t ev0, hipEvent_t ev1) {
     if (GROUP && ntiles % kTileWaves) return hipErrorInvalidValue;
     const int grid = (ntiles + kTileWaves - 1) / kTileWaves;
     if (ev0 || ev1)
-        hipExtLaunchKernelGGL((stencil_tiles<R, K, KAHAN, KIND, PERSIST, GROUP>), dim3(grid), dim3(64 * kTileWaves), 0,
-                              st, ev0, ev1, 0, sims, tiles, ntiles, launch_idx, gstep0, nsteps, S, pa);
+        hipExtLaunchKernelGGL((stencil_tiles<R, K, KAHAN, KIND, GROUP>), dim3(grid), dim3(64 * kTileWaves), 0, st, ev0,
+                              ev1, 0, sims, tiles, ntiles, launch_idx, gstep0, nsteps, S, pa);
     else
-        hipLaunchKernelGGL((stencil_tiles<R, K, KAHAN, KIND, PERSIST, GROUP>), dim3(grid), dim3(64 * kTileWaves), 0, st,
-                           sims, tiles, ntiles, launch_idx, gstep0, nsteps, S, pa);
+        hipLaunchKernelGGL((stencil_tiles<R, K, KAHAN, KIND, GROUP>), dim3(grid), dim3(64 * kTileWaves), 0, st, sims,
+                           tiles, ntiles, launch_idx, gstep0, nsteps, S, pa);
     return hipGetLastError();
 }
-
-// Persistent instances exist for K <= kPersistMaxK (the host declines wider tiles).
-constexpr int kPersistMaxK = 4;
 
 template <typename R, int K, bool KAHAN, int KIND>
 static hipError_t launch_k(const SimDev<R>* sims, const int2* tiles, int ntiles, long long launch_idx,
@@ -929,19 +1265,13 @@ static hipError_t launch_k(const SimDev<R>* sims, const int2* tiles, int ntiles,
     if (pa.halo > 0) {
         // halo-exchange instances: K = 2 and 4 (hx / K <= kHaloMaxLanes)
         if constexpr (K == 2 || K == 4) {
-            if (pa.halo % K || pa.halo / K > kHaloMaxLanes || pa.nblocks > 1) return hipErrorInvalidValue;
-            return launch_kp<R, K, KAHAN, KIND, false, true>(sims, tiles, ntiles, launch_idx, gstep0, nsteps, S, pa,
-                                                            st, ev0, ev1);
+            if (pa.halo % K || pa.halo / K > kHaloMaxLanes) return hipErrorInvalidValue;
+            return launch_kp<R, K, KAHAN, KIND, true>(sims, tiles, ntiles, launch_idx, gstep0, nsteps, S, pa, st, ev0,
+                                                     ev1);
         }
         return hipErrorInvalidValue;
     }
-    if (pa.nblocks > 1) {
-        if constexpr (K <= kPersistMaxK)
-            return launch_kp<R, K, KAHAN, KIND, true>(sims, tiles, ntiles, launch_idx, gstep0, nsteps, S, pa, st,
-                                                     ev0, ev1);
-        return hipErrorInvalidValue;
-    }
-    return launch_kp<R, K, KAHAN, KIND, false>(sims, tiles, ntiles, launch_idx, gstep0, nsteps, S, pa, st, ev0, ev1);
+    return launch_kp<R, K, KAHAN, KIND>(sims, tiles, ntiles, launch_idx, gstep0, nsteps, S, pa, st, ev0, ev1);
 }
 
 template <typename R, bool KAHAN, int KIND>
@@ -955,22 +1285,6 @@ hipError_t launch_kind(const SimDev<R>* sims, const int2* tiles, int ntiles, lon
         case 8: return launch_k<R, 8, KAHAN, KIND>(sims, tiles, ntiles, launch_idx, gstep0, nsteps, S, pa, st, ev0, ev1);
         default: return hipErrorInvalidValue;
     }
-}
-
-// Workgroups of the persistent field kernel for K cells per lane that one
-// CU holds at once (register and LDS limits): a persistent launch needs
-// every tile resident.  0 where no persistent instance exists.
-template <typename R, bool KAHAN, int KIND>
-int field_blocks_per_cu(int K) {
-    int nb = 0;
-    hipError_t e = hipErrorInvalidValue;
-    switch (K) {
-        case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, stencil_tiles<R, 1, KAHAN, KIND, true>, 64 * kTileWaves, 0); break;
-        case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, stencil_tiles<R, 2, KAHAN, KIND, true>, 64 * kTileWaves, 0); break;
-        case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, stencil_tiles<R, 4, KAHAN, KIND, true>, 64 * kTileWaves, 0); break;
-        default: break;
-    }
-    return e == hipSuccess ? nb : 0;
 }
 
 }  // namespace fdtd

@@ -71,6 +71,8 @@ SIGNATURES = {
     "fdtd_set_pic_lds_rows": (C.c_int, [_vp, C.c_int]),
     "fdtd_set_persistent": (C.c_int, [_vp, C.c_int]),
     "fdtd_persistent_active": (C.c_int, [_vp, C.POINTER(C.c_int)]),
+    "fdtd_set_resident": (C.c_int, [_vp, C.c_int, C.c_int64]),
+    "fdtd_resident_active": (C.c_int, [_vp, C.POINTER(C.c_int)]),
     "fdtd_set_halo_exchange": (C.c_int, [_vp, C.c_int]),
     "fdtd_halo_exchange_active": (C.c_int, [_vp, C.POINTER(C.c_int)]),
     "fdtd_add_sim": (C.c_int, [_vp, C.POINTER(SimDesc), C.POINTER(C.c_int)]),

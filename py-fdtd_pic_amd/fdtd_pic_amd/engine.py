@@ -217,6 +217,19 @@ class Context:
         check(self.lib.fdtd_persistent_active(self.h, C.byref(v)))
         return bool(v.value)
 
+    def set_resident(self, on=True, max_wait_us=0):
+        """Resident field launches (default on): a whole run() in one launch
+        when every tile fits on the device at once (bitwise the same results).
+        max_wait_us bounds one wait for a neighbour (0: 50 ms); a launch that
+        passes it is run again with one launch per S steps."""
+        check(self.lib.fdtd_set_resident(self.h, 1 if on else 0, int(max_wait_us)))
+
+    def resident_active(self):
+        """True when the next run() uses resident launches."""
+        v = C.c_int()
+        check(self.lib.fdtd_resident_active(self.h, C.byref(v)))
+        return bool(v.value)
+
     def set_halo_exchange(self, h=8):
         """Workgroup halo exchange every h steps between the four adjacent
         windows of a field workgroup (0: off); declined where it does not apply."""

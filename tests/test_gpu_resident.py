@@ -1,0 +1,132 @@
+"""Resident field launches (fdtd_set_resident) against one launch per S steps.
+
+A resident launch runs a whole fdtd_run with every tile's window in registers
+and the tiles' edge cells handed over through a mailbox.  Tile widths, owned
+ranges and (FP64) the block length differ from the one-block tiles', yet every
+result must be the same bits: fields, slab state, CPML psi, probes, snapshots.
+Sizes sit where a plan can go wrong: a grid of one tile, a last cell alone, odd
+sizes, slabs of a few cells and slabs that reach into a CPML strip, sources
+beside a slab, more probes than a tile captures, runs shorter than a block,
+runs cut into pieces, several simulations of different lengths.  A launch whose
+waits are bounded to one microsecond gives up and is run again: the results
+stay the same.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("E", "H", "D", "P", "PM", "PSIE", "PSIH")
+
+
+def _phys(N, steps, slab="kerr", F=None, R=None, **kw):
+    from fdtd_pic_amd import configs, engine
+    rng = np.random.default_rng(N)
+    F = N // 2 if F is None else F
+    R = min(F + N // 4, N - N // 6) if R is None else R
+    p = configs.base(N, steps, slab_start=F, slab_stop=F if slab == "none" else R, src_cell=min(60, N // 4),
+                     src_t0=4e-15, src_tau=1.5e-15, src_amp=1.8e8, probes=[N // 5 if N < 300 else 45, N - min(40, N // 6)],
+                     pml_width=min(32, N // 8))
+    if slab == "kerr":
+        p.update(chi3=1e-19, eps_inf=rng.uniform(1, 3, max(R - F, 0)))
+    p.update(kw)
+    return engine.physical_spec(p)
+
+
+def _dropin(kind, Nz=700, T=500, W=90, **kw):
+    """A pass of a drop-in integrator (snapshots every 50 steps, TFSF)."""
+    import Solver_Engine as SE
+    from refcases import product_objects, small_setup
+    setup = small_setup(Nz=Nz, T=T, W=W, F=kw.pop("F", 330), R=kw.pop("R", Nz - 1), nzsrc=150)
+    flags = dict(SineCont=True, TFSF=True)
+    flags.update({"linlor": dict(LorentzMed=True), "nl": dict(nonLinMed=True), "free": {}}[kind])
+    V, P, C_V, C_P = product_objects(setup, 9e9, **flags)
+    if kind == "nl":
+        P.FreeSpace, P.Periods = False, 1000
+    if kind == "free":
+        P.epsRe = 2.25
+    plan = {"linlor": SE.plan_linlor, "nl": SE.plan_nl, "free": SE.plan_free_space}[kind](
+        V, P, C_V, C_P, int(0.7 * T), int(0.05 * T))
+    return plan.passes[-1][0]
+
+
+def _run(specs, prec, resident, cuts=(), tiling=None, wait_us=0):
+    from fdtd_pic_amd import engine
+    with engine.Context(prec) as c:
+        if tiling:
+            c.set_tiling(*tiling)
+        c.set_resident(resident, wait_us)
+        sims = [c.add(s) for s in specs]
+        active = c.resident_active()
+        for n in cuts:
+            c.run(n)
+        c.run_all()
+        out = []
+        for sim, s in zip(sims, specs):
+            o = {f: sim.read(f) for f in FIELDS if f in ("E", "H", "PSIE", "PSIH") or s.R > s.F}
+            o["probes"], o["progress"] = sim.probes(), sim.progress()
+            if s.snap_rows:
+                o["snap"] = sim.snapshots()
+            out.append(o)
+    return active, out
+
+
+def _same(specs, prec, tag, **kw):
+    print(f"resident {prec} {tag}", flush=True)
+    taken = kw.pop("taken", True)
+    on, a = _run(specs, prec, True, **kw)
+    kw.pop("wait_us", None)
+    off, b = _run(specs, prec, False, **kw)
+    assert on == taken and not off
+    for k, (x, y) in enumerate(zip(a, b)):
+        assert np.abs(y["E"]).max() > 0
+        for f in y:
+            assert np.array_equal(x[f], y[f]), (tag, k, f)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("N,slab,kw", [
+    (40, "none", {}), (127, "linear", {}), (192, "kerr", {}), (193, "kerr", {}), (1000, "linear", {}),
+    (4097, "kerr", {}), (4098, "kerr", dict(F=2000, R=2003)), (3001, "kerr", dict(F=1500, R=1501)),
+    (2500, "linear", dict(F=1200, R=2490)), (2500, "kerr", dict(F=70, R=2400)),
+    (9001, "kerr", dict(src_cell=4490)), (6000, "kerr", dict(probes=[3000, 3001, 3002, 3050, 3100, 700])),
+    (25013, "linear", {}), (65536, "kerr", {}), (30000, "none", {})])
+def test_resident_equals_launch_per_block(prec, N, slab, kw):
+    # FP32 has no resident class for more than two probes in a tile
+    _same([_phys(N, 411, slab, **kw)], prec, f"N={N} {slab} {kw}", taken=prec == "f64" or len(kw.get("probes", ())) < 3)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("tiling", [(1, 24), (2, 16), (2, 48)])
+def test_resident_at_set_tilings(prec, tiling):
+    _same([_phys(5000, 301)], prec, f"tiling {tiling}", tiling=tiling)
+
+
+@pytest.mark.parametrize("kind,kw", [("linlor", {}), ("nl", {}), ("free", {}), ("linlor", dict(Nz=2111, T=333, F=900)),
+                                     ("free", dict(Nz=1500, F=700, R=1200))])
+def test_resident_dropin_passes(kind, kw):
+    spec = _dropin(kind, **kw)
+    assert spec.snap_rows > 0 and spec.tfsf
+    _same([spec], "f64", f"{kind} {kw}")
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_resident_several_simulations_and_pieces(prec):
+    specs = [_phys(3000, 500), _phys(800, 260, "none"), _phys(5001, 611), _phys(1200, 90, "linear", chi3=0.0)]
+    _same(specs, prec, "four simulations", cuts=(96, 5, 192))
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_resident_gives_up_and_runs_again(prec):
+    """Waits bounded to 1 us: the launch gives up where a wait takes longer,
+    whatever was done stays unseen, and its steps are run again."""
+    _same([_phys(9000, 900), _phys(2000, 333, "none")], prec, "1 us waits", wait_us=1, cuts=(96, 192))
+
+
+def test_resident_not_taken():
+    from fdtd_pic_amd import engine
+    with engine.Context("f64") as c:
+        s = c.add(_phys(1000, 100))
+        assert c.resident_active()
+        s.set_energy(1, 8)
+        assert not c.resident_active()
