@@ -82,6 +82,7 @@ struct ResArgs {
     unsigned long long* other;   // the other set
     int stride;                  // cells of the mailbox (all simulations, with one spare)
     int nsteps, S;
+    int formK;                   // FP32: cells per lane of the one-block tiles (psi_next)
     int ordinal;
     int32_t* err;                // device
     int32_t* herr;               // host memory
@@ -91,6 +92,7 @@ struct ResArgs {
 // and the one after the last, w = the simulation's first cell in the mailbox.
 constexpr int kResK2 = 1 << 24, kResK4 = 1 << 25;   // cells per lane: 1, 2 or 4
 constexpr int kResPlain = 1 << 26;                  // no D-form slab cell in its window: the plain bodies
+constexpr int kResEmu = 1 << 27;                    // FP32: the vacuum cells of the window are emulated slab cells
 constexpr unsigned long long kResEmpty = 0x7ff45ea17fb45ea1ull;
 template <typename R>
 constexpr int kResValues = sizeof(R) == 8 ? 7 : 6;   // FP64 E H D P Pm psiE psiH; FP32 pairs E H D P, Pm, psiE|psiH

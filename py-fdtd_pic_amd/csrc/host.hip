@@ -369,16 +369,14 @@ int fdtd_ctx_create(int precision, fdtd_ctx** out) {
         delete c;
         return rc;
     }
-    if (hipMalloc(&c->d_err, sizeof(int32_t)) != hipSuccess || hipMemset(c->d_err, 0, sizeof(int32_t)) != hipSuccess ||
-        hipMalloc(&c->d_rerr, sizeof(int32_t)) != hipSuccess || hipMemset(c->d_rerr, 0, sizeof(int32_t)) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_rerr, sizeof(int32_t), hipHostMallocDefault) != hipSuccess) {
+    if (hipMalloc(&c->d_err, 2 * sizeof(int32_t)) != hipSuccess ||
+        hipMemset(c->d_err, 0, 2 * sizeof(int32_t)) != hipSuccess) {
         if (c->d_err) (void)hipFree(c->d_err);
-        if (c->d_rerr) (void)hipFree(c->d_rerr);
         (void)hipStreamDestroy(c->st);
         delete c;
         return fdtd_fail(FDTD_E_HIP, "allocation of the error flags failed");
     }
-    *c->h_rerr = 0;
+    c->d_rerr = c->d_err + 1;
     if (hipDeviceGetAttribute(&c->cu_count, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         c->cu_count = 0;
     if (hipDeviceGetAttribute(&c->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
@@ -401,11 +399,10 @@ int fdtd_ctx_destroy(fdtd_ctx* c) {
     for (BeamHost* b : c->beams)
         if (b) { if (b->block) (void)hipFree(b->block); delete b; }
     for (void* p : {(void*)c->d_beams, (void*)c->d_pblocks, (void*)c->d_pitems, (void*)c->d_err, c->d_scratch,
-                    (void*)c->d_rerr, (void*)c->d_rtiles, (void*)c->d_box})
+                    (void*)c->d_rtiles, (void*)c->d_box})
         if (p) (void)hipFree(p);
     res_release(c);
     if (c->res_ev) (void)hipEventDestroy(c->res_ev);
-    if (c->h_rerr) (void)hipHostFree(c->h_rerr);
     if (c->d_sims) (void)hipFree(c->d_sims);
     if (c->d_tiles) (void)hipFree(c->d_tiles);
     for (auto& e : c->events) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
@@ -518,6 +515,7 @@ struct Upload {
 // (which keep reading the old contents until then).  The staging buffer is
 // reused only after the previous upload has run; a device array that must
 // grow is reallocated after the queued launches have finished with it.
+constexpr size_t kStageHead = 256;
 static int staged_upload(fdtd_ctx* c, const std::vector<Upload>& ups) {
     auto pad = [](size_t b) { return (b + 255) & ~size_t(255); };
     size_t total = 0;
@@ -534,8 +532,12 @@ static int staged_upload(fdtd_ctx* c, const std::vector<Upload>& ups) {
         if (c->stage) HIPCHK(hipHostFree(c->stage));
         c->stage = nullptr;
         c->stage_cap = 0;
-        HIPCHK(hipHostMalloc(&c->stage, total * 2, hipHostMallocDefault));
+        // the first words are the resident launches' give-up flag (resolved
+        // before a rebuild, so none is in flight here)
+        HIPCHK(hipHostMalloc(&c->stage, kStageHead + total * 2, hipHostMallocDefault));
         c->stage_cap = total * 2;
+        c->h_rerr = (int32_t*)c->stage;
+        *c->h_rerr = 0;
     }
     if (grow) HIPCHK(hipStreamSynchronize(c->st));
     size_t off = 0;
@@ -548,7 +550,7 @@ static int staged_upload(fdtd_ctx* c, const std::vector<Upload>& ups) {
             *u.cap = u.bytes * 2;
         }
         if (u.bytes) {
-            char* s = (char*)c->stage + off;
+            char* s = (char*)c->stage + kStageHead + off;
             std::memcpy(s, u.src, u.bytes);
             HIPCHK(hipMemcpyAsync(*u.dst, s, u.bytes, hipMemcpyHostToDevice, c->st));
         }
@@ -763,29 +765,34 @@ struct ResSim {
     bool plain;                             // no D-form slab: the plain bodies
     bool last_dead;                         // the last cell's fields never change
     std::vector<ResInterval> heavy;         // slab, CPML strips, source, probes
+    std::vector<std::pair<int, int>> emu;   // FP32: cells of the one-block tiles that emulate their vacuum cells
 };
 
 // Tiles of one simulation, in order: light tiles (plain cells, Kl per lane)
 // where their windows meet nothing else, heavy ones (Kh per lane) elsewhere.
-// With Kl = 0 every tile is a heavy one.
+// A tile owns cells of emulating one-block tiles only, or of none.
 static int res_tile_sim(const ResSim& q, int Kh, int Kl, int S, int box0, std::vector<int4>* out) {
     const int Uh = 64 * Kh - 2 * S, Ul = 64 * Kl - 2 * S;
     auto kflag = [](int K) { return K == 4 ? kResK4 : K == 2 ? kResK2 : 0; };
     int n = 0;
+    size_t ne = 0;
     for (int o = 0; o <= q.N;) {
-        int light_end = Kl ? std::min(o + Ul, q.N + 1) : o;
+        while (ne < q.emu.size() && q.emu[ne].second <= o) ++ne;
+        const bool emu = ne < q.emu.size() && q.emu[ne].first <= o;
+        const int stop = ne == q.emu.size() ? q.N + 1 : emu ? q.emu[ne].second : q.emu[ne].first;
+        int light_end = emu ? o : std::min(o + Ul, stop);
         for (const ResInterval& v : q.heavy) {
             const int m = v.window ? S : 0;
             if (v.hi > o - m) light_end = std::min(light_end, v.lo - m);
         }
         int e, flags;
         // light where it covers at least what a heavy tile would
-        if (Kl && light_end - o >= std::min(Uh, Ul)) {
+        if (light_end - o >= std::min(Uh, Ul)) {
             e = light_end;
             flags = kResPlain | kflag(Kl);
         } else {
-            e = std::min(o + Uh, q.N + 1);
-            flags = (q.plain ? kResPlain : 0) | kflag(Kh);
+            e = std::min(o + Uh, stop);
+            flags = (q.plain ? kResPlain : 0) | kflag(Kh) | (emu ? kResEmu : 0);
         }
         // the last cell alone is not worth a tile: the window holds it, and
         // beyond it everything is zero
@@ -797,7 +804,7 @@ static int res_tile_sim(const ResSim& q, int Kh, int Kl, int S, int box0, std::v
     return n;
 }
 
-// What a block of S steps of a wave with a SIMD to itself costs in FP64: ns
+// What a block of S steps of a wave with a SIMD to itself costs: ns
 // per step and ns for the hand-off, by cells per lane (measured per tile: the
 // slowest tile, which waits for nobody, sets the pace).  Heavy tiles by slab
 // kind; the strip, source and probe tiles' classes lie below the slabs' or
@@ -805,7 +812,8 @@ static int res_tile_sim(const ResSim& q, int Kh, int Kl, int S, int box0, std::v
 struct ResCost {
     double heavy[2], light[3];
 };
-static ResCost res_cost(int kind) {
+static ResCost res_cost(int kind, bool f32) {
+    if (f32) return kind == SLAB_KERR_E ? ResCost{{100, 140}, {46, 60, 85}} : ResCost{{85, 115}, {46, 60, 85}};
     const double l1 = 46, l2 = 60, l4 = 77;
     return kind == SLAB_KERR_E     ? ResCost{{125, 158}, {l1, l2, l4}}
            : kind == SLAB_KERR_REF ? ResCost{{3900, 7100}, {l1, l2, l4}}
@@ -819,12 +827,13 @@ template <typename R>
 static int plan_resident(fdtd_ctx* c) {
     constexpr bool f32 = sizeof(R) == 4;
     if (!c->res_mode || c->cu_count <= 0 || c->tile_sims.empty()) return FDTD_OK;
-    // FP32 rounds by K and a cell's place in its tile (psi_next, and the
-    // emulated cells of slab-boundary tiles), so there the tiles and blocks are
-    // the one-block ones
-    if (f32 && (c->K_slab != c->K || c->K > 4)) return FDTD_OK;
-    if (f32 && (c->S_run > kResMaxSHost || 64 * c->K - 2 * c->S_run < 1)) return FDTD_OK;
-    bool kerr = f32;
+    // FP32 keeps the block length and the rounding of the one-block tiles
+    // (psi_next, and the emulated cells of slab-boundary tiles): uniform tiles
+    // whose lanes start at cells of one residue
+    if (f32 && (c->K_slab != c->K || c->K > 4 || c->S_run > kResMaxSHost || 2 * c->S_run % c->K != 0 ||
+                64 * c->K - 2 * c->S_run < 1))
+        return FDTD_OK;
+    bool kerr = false;
     for (int i : c->tile_sims) {
         const SimHost& s = *c->sims[i];
         if (s.e_every > 0) return FDTD_OK;            // energy is taken launch by launch
@@ -841,8 +850,8 @@ static int plan_resident(fdtd_ctx* c) {
         q.plain = d.slab_kind < SLAB_LINEAR;
         q.last_dead = c->sims[i]->last_dead;
         if (!q.plain) {
-            // FP64: a Kerr slab with chi3 = 0 is the linear slab bit for bit
-            // (the root's series is then exactly 1)
+            // a Kerr slab with chi3 = 0 is the linear slab bit for bit (the
+            // root's series is then exactly 1)
             const int k = d.slab_kind == SLAB_KERR_E && !kerr ? SLAB_LINEAR : d.slab_kind;
             if (kind != SLAB_DIEL && k != kind) return FDTD_OK;
             kind = k;
@@ -862,6 +871,19 @@ static int plan_resident(fdtd_ctx* c) {
                 for (int r = 0; r < d.nprobe; ++r) same += d.probe_cell[r] / U0 == d.probe_cell[p] / U0;
                 if (same > 2) return FDTD_OK;
             }
+            // the one-block tiles whose vacuum cells are emulated (tile_body)
+            const int L = 64 * c->K, S0 = c->S_run;
+            if (d.slab_kind == SLAB_KERR_E && (float)d.ke0 == (float)d.kD && (float)d.jD == 1.0f)
+                for (int t = std::max(0, (d.F - L) / U0); t * U0 <= d.N && t * U0 - S0 < d.R; ++t) {
+                    const int t0 = t * U0 - S0, t1 = t0 + L;
+                    if (t1 <= d.F || (t0 >= d.F && t1 <= d.R)) continue;              // no slab, or only slab
+                    if (t0 < 0 || t1 - 1 > d.N || t0 < d.Ls || t1 > d.Rs) continue;   // cells off the grid, strips
+                    if ((d.src_cell >= t0 && d.src_cell < t1) || (d.tfsf && d.src_cell - 1 >= t0 && d.src_cell - 1 < t1))
+                        continue;
+                    bool probe = false;
+                    for (int p = 0; p < d.nprobe; ++p) probe = probe || d.probe_cell[p] / U0 == t;
+                    if (!probe) q.emu.push_back({t * U0, std::min((t + 1) * U0, d.N + 1)});
+                }
         }
         cells += d.N + 1;
         sims.push_back(std::move(q));
@@ -877,32 +899,25 @@ static int plan_resident(fdtd_ctx* c) {
         return n;
     };
     long long nt = 0;
-    if (f32) {
-        bKh = c->K;
-        bS = c->S_run;
-        bW = bKh == 4 ? 1 : 2;
-        nt = count(bKh, 0, bS, 2 * round);
-        if (nt > (long long)resident_capacity_per_cu<R, f32>(kind, bW) * round) return FDTD_OK;
-    } else {
-        const ResCost cost = res_cost(kind);
-        const int cap2 = resident_capacity_per_cu<R, f32>(kind, 2);
-        double best = 1e30;
-        for (int Kh = 1; Kh <= 2; ++Kh)
-            for (int Kl = Kh; Kl <= 4; Kl *= 2)
-                for (int S = 4; S <= 32 * Kh - 4; S += 4) {
-                    const long long n = count(Kh, Kl, S, (long long)cap2 * round);
-                    if (n > (long long)cap2 * round) continue;
-                    const double rounds = (double)((n + round - 1) / round);
-                    const int l = Kl == 4 ? 2 : Kl - 1;
-                    const bool hand = n > (long long)sims.size();
-                    const double t = rounds * std::max(cost.heavy[Kh - 1] + (hand ? kResHandNs[Kh - 1] / S : 0.0),
-                                                       cost.light[l] + (hand ? kResHandNs[l] / S : 0.0));
-                    if (t < best) { best = t; bKh = Kh; bKl = Kl; bS = S; nt = n; }
-                }
-        if (!bKh) return FDTD_OK;
-        bW = nt > round ? 2 : 1;
-        if (nt > (long long)resident_capacity_per_cu<R, f32>(kind, bW) * round) return FDTD_OK;
-    }
+    const ResCost cost = res_cost(kind, f32);
+    const int cap2 = resident_capacity_per_cu<R, f32>(kind, 2);
+    double best = 1e30;
+    for (int Kh = 1; Kh <= 2; ++Kh)
+        for (int Kl = Kh; Kl <= 4; Kl *= 2)
+            for (int S = f32 ? c->S_run : 4; S <= (f32 ? c->S_run : 32 * Kh - 4); S += 4) {
+                if (64 * Kh - 2 * S < 4) continue;
+                const long long n = count(Kh, Kl, S, (long long)cap2 * round);
+                if (n > (long long)cap2 * round) continue;
+                const double rounds = (double)((n + round - 1) / round);
+                const int l = Kl == 4 ? 2 : Kl - 1;
+                const bool hand = n > (long long)sims.size();
+                const double t = rounds * std::max(cost.heavy[Kh - 1] + (hand ? kResHandNs[Kh - 1] / S : 0.0),
+                                                   cost.light[l] + (hand ? kResHandNs[l] / S : 0.0));
+                if (t < best) { best = t; bKh = Kh; bKl = Kl; bS = S; nt = n; }
+            }
+    if (!bKh) return FDTD_OK;
+    bW = nt > round ? 2 : 1;
+    if (nt > (long long)resident_capacity_per_cu<R, f32>(kind, bW) * round) return FDTD_OK;
     std::vector<int4> tiles;
     int box0 = 0;
     for (const ResSim& q : sims) {
@@ -1243,6 +1258,7 @@ static int run_resident_t(fdtd_ctx* c, int64_t n, bool* taken) {
     ra.stride = c->res_stride;
     ra.nsteps = (int)n;
     ra.S = c->res_S;
+    ra.formK = c->K;
     ra.ordinal = ++c->res_ordinal;
     ra.err = c->d_rerr;
     ra.herr = c->h_rerr;

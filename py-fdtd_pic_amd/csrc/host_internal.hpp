@@ -138,8 +138,8 @@ struct fdtd_ctx {
     size_t d_box_cap = 0;
     int box_set = 0;
     bool box_stale = true;                   // to be emptied before the next resident launch
-    int32_t* d_rerr = nullptr;               // ordinal of the launch that gave up (0: none)
-    int32_t* h_rerr = nullptr;               // the same in host memory
+    int32_t* d_rerr = nullptr;               // ordinal of the launch that gave up (0: none; beside d_err)
+    int32_t* h_rerr = nullptr;               // the same in host memory (the head of stage)
     int res_ordinal = 0;
     std::vector<ResPending> res_pending;     // resident launches not yet known to have finished
     hipEvent_t res_ev = nullptr;             // recorded after the last resident launch

@@ -152,7 +152,9 @@ __device__ __forceinline__ R slab_e_simple(const SimDev<R>& sd, double u, R D, R
         const double A = cubic_root0_1728(sd.kerr_a, sd.kerr_b, sd.kerr_c, -(fabs(dd) * fabs(dd)));
         return (R)((double)D / (sd.kerr_e0 * sd.kerr_lin + sd.kerr_e0 * sd.kerr_chi3 * A));
     } else {
-        return (R)(u * (double)ie);
+#pragma clang fp contract(off)
+        // FP32: u comes from a float; the product rounds as it does through FP64 (48 bits are exact there)
+        return (R)u * ie;
     }
 }
 
@@ -210,6 +212,7 @@ struct TileCtx {
     // emulated vacuum cells (E-form Kerr slab-boundary tiles)
     int wv, hx;
     unsigned emu_mask;
+    unsigned first_mask;    // FP32 resident tiles: cells that are a lane's first one in the one-block tiles
 };
 
 // What a tile's step loop has to handle (compile-time, one loop per class).
@@ -306,15 +309,20 @@ __device__ __forceinline__ void e_pure_slab(TILE_PARAMS, const TileCtx<R>& c, co
 // psi' = b psi + c d of the CPML.  FP64 fuses b psi.  FP32 rounds as the
 // compiler fused the one-block loops: FORM < 0 leaves it to the compiler (the
 // one-block kernels themselves); a resident tile writes the fused product out:
-// b psi (0), or c d (1), which those loops fuse in the E half of a tile's
-// cells 1 .. K-1 at the even steps of a launch, and nowhere else (read from
-// the compiled loops of K = 1, 2 and 4; the tests hold resident FP32 runs to
-// the one-block runs bit for bit).
+// b psi (0), or, where FORM is 1 and the cell is not a lane's first one in
+// the one-block tiles, c d.  Those loops fuse c d in the E half of a lane's
+// later cells at the even steps of a launch, and b psi everywhere else (read
+// from the compiled loops of K = 1, 2 and 4; the tests hold resident FP32 runs
+// to the one-block runs bit for bit).
 template <int FORM, typename R>
-__device__ __forceinline__ R psi_next(R b, R psi, R c, R d) {
-    if constexpr (FORM < 0 || sizeof(R) == 8) return fmr(b, psi, c * d);
-    else if constexpr (FORM == 0) return __builtin_fmaf(b, psi, c * d);
-    else return __builtin_fmaf(c, d, b * psi);
+__device__ __forceinline__ R psi_next(R b, R psi, R c, R d, bool first) {
+    if constexpr (FORM < 0 || sizeof(R) == 8) {
+        return fmr(b, psi, c * d);
+    } else {
+        const R v = __builtin_fmaf(b, psi, c * d);
+        if constexpr (FORM == 0) return v;
+        else return first ? v : __builtin_fmaf(c, d, b * psi);
+    }
 }
 
 // Mixed tile: every cell takes the interior update (+ CPML psi), slab cells
@@ -329,8 +337,7 @@ __device__ __forceinline__ void e_mixed(TILE_PARAMS, const TileCtx<R>& c, const 
         const R a = dH[j] - Jv[j];
         if (KAHAN) kahan_fma(Ev[j], cEv[j], a, ke[j]); else Ev[j] = fmr(a, ke[j], Ev[j]);
         if (STRIP) {
-            psE[j] = j == 0 ? psi_next<(FORM < 0 ? -1 : 0)>(bE[j], psE[j], cEc[j], dH[j])
-                            : psi_next<FORM>(bE[j], psE[j], cEc[j], dH[j]);
+            psE[j] = psi_next<FORM>(bE[j], psE[j], cEc[j], dH[j], (c.first_mask >> j) & 1u);
             Ev[j] = fmr(-CbE[j], psE[j], Ev[j]);
         }
     }
@@ -620,8 +627,7 @@ __device__ __forceinline__ void res_steps(TILE_PARAMS, const TileCtx<R>& c, cons
             for (int j = 0; j < K; ++j) {
                 if (KAHAN) kahan_fma(E[j], cE[j], dH[j], ke[j]); else E[j] = fmr(dH[j], ke[j], E[j]);
                 if (STRIP) {
-                    psE[j] = j == 0 ? psi_next<0>(bE[j], psE[j], cEc[j], dH[j])
-                                    : psi_next<FORM>(bE[j], psE[j], cEc[j], dH[j]);
+                    psE[j] = psi_next<FORM>(bE[j], psE[j], cEc[j], dH[j], (c.first_mask >> j) & 1u);
                     E[j] = fmr(-CbE[j], psE[j], E[j]);
                 }
             }
@@ -642,7 +648,7 @@ __device__ __forceinline__ void res_steps(TILE_PARAMS, const TileCtx<R>& c, cons
             const R dE = ((j == K - 1) ? Er : E[j + 1]) - E[j];
             if (KAHAN) kahan_fma(H[j], cH[j], dE, kh[j]); else H[j] = fmr(dE, kh[j], H[j]);
             if (STRIP) {
-                psH[j] = psi_next<0>(bH[j], psH[j], cHc[j], dE);
+                psH[j] = psi_next<0>(bH[j], psH[j], cHc[j], dE, true);
                 H[j] = fmr(C2H[j], psH[j], H[j]);
             }
         }
@@ -735,6 +741,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
     c.wv = wv;
     c.hx = hx;
     c.emu_mask = 0;
+    c.first_mask = 0;
     c.base = c.t0 + lane * K;
     c.N = N;
     c.T = sd.T;
@@ -825,6 +832,8 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
             psE[j] = sd.psiE[par][i]; psH[j] = sd.psiH[par][i];
         }
         if (valid && n >= out0 && n < out0 + U) interior_mask |= 1u << j;
+        if constexpr (RES && sizeof(R) == 4)
+            if ((n + S) % ra.formK == 0) c.first_mask |= 1u << j;
         ied[j] = (double)ie[j];
         kz[j] = c.chi3 * ied[j];
     }
@@ -880,9 +889,12 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
         cD[j] = cE[j];
         P[j] = Pm[j] = cP[j] = R(0);
     };
-    if constexpr (KIND == SLAB_KERR_E || (RES && sizeof(R) == 8 && KIND == SLAB_LINEAR)) {
+    if constexpr (KIND == SLAB_KERR_E || (RES && KIND == SLAB_LINEAR)) {
         const bool all_valid = __all(c.base >= 0 && c.base + K - 1 <= N);
         emu_tile = any_slab && !pure_slab && !extras && !gen && all_valid && sd.ke0 == sd.kD && sd.jD == R(1);
+        // FP32 rounds an emulated cell's E as D - cD, so a resident tile
+        // emulates where the one-block tile that owns its cells does
+        if constexpr (RES && sizeof(R) == 4) emu_tile = (rt.x & kResEmu) != 0;
         if (emu_tile) {
 #pragma unroll
             for (int j = 0; j < K; ++j) {
@@ -995,7 +1007,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
                     R* sp = &spare_rows[wvi][0][0];
                     const int n = c.s_hi;
                     const bool srcs = tile_src || tile_tf, prb = c.npr > 0, ends = srcs || prb;
-                    if constexpr (K == 4 && sizeof(R) == 8)      // light tiles: plain cells only
+                    if constexpr (K == 4)      // light tiles: plain cells only
                         res_steps<R, K, KAHAN, KIND, 0>(TILE_ARGS, c, sd, sc, sp, n);
                     else if (sizeof(R) == 8 && gen)
                         run(&sc);
@@ -1174,8 +1186,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void stencil_tiles(const SimDev<R>
 
 // Resident launch: tile t is wave t % 4 of workgroup t / 4; W workgroups fit
 // on a CU.  RESDOC
-// FP64 tiles hold 1 or 2 cells per lane, plain ones up to 4; FP32 tiles are
-// the one-block tiles of the context's K: 1 and 2 with W = 2, 4 with W = 1.
+// Tiles hold 1 or 2 cells per lane, plain ones up to 4.
 template <typename R, bool KAHAN, int KIND, int W>
 __global__ __launch_bounds__(64 * kTileWaves, W) void stencil_resident(const SimDev<R>* __restrict__ sims,
                                                                        const int4* __restrict__ tiles, int ntiles,
@@ -1198,20 +1209,15 @@ __global__ __launch_bounds__(64 * kTileWaves, W) void stencil_resident(const Sim
     using K2 = integral_constant<int, 2>;
     using K4 = integral_constant<int, 4>;
     const bool plain = KIND == SLAB_DIEL || (rt.x & kResPlain);
-    if constexpr (sizeof(R) == 4 && W == 1) {
-        if (!plain) body(K4{}, Kind{});
-        else body(K4{}, Plain{});
+    if (!plain) {
+        if (rt.x & kResK2) body(K2{}, Kind{});
+        else body(K1{}, Kind{});
+    } else if (rt.x & kResK4) {
+        body(K4{}, Plain{});
+    } else if (rt.x & kResK2) {
+        body(K2{}, Plain{});
     } else {
-        if (!plain) {
-            if (rt.x & kResK2) body(K2{}, Kind{});
-            else body(K1{}, Kind{});
-        } else if (sizeof(R) == 8 && (rt.x & kResK4)) {
-            if constexpr (sizeof(R) == 8) body(K4{}, Plain{});
-        } else if (rt.x & kResK2) {
-            body(K2{}, Plain{});
-        } else {
-            body(K1{}, Plain{});
-        }
+        body(K1{}, Plain{});
     }
 }
 
