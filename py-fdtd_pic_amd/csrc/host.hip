@@ -103,6 +103,7 @@ static void fill_dev(SimHost& s, SimDev<R>& d) {
     d.ke0 = (R)q.ke0; d.kh0 = (R)q.kh0; d.keS = (R)q.keS; d.khS = (R)q.khS; d.kD = (R)q.kD; d.jD = (R)q.jD;
     d.kerr_a = q.kerr_a; d.kerr_b = q.kerr_b; d.kerr_c = q.kerr_c;
     d.kerr_e0 = q.kerr_e0; d.kerr_lin = q.kerr_lin; d.kerr_chi3 = q.kerr_chi3;
+    if (q.slab_kind == FDTD_SLAB_KERR_REF) d.cub = cubic_const(q.kerr_a, q.kerr_b, q.kerr_c);
     auto P = [&](int k) { return (R*)(blk + s.lay_off[k]); };
     int k = 0;
     const R* cs[8];
@@ -816,7 +817,7 @@ static ResCost res_cost(int kind, bool f32) {
     if (f32) return kind == SLAB_KERR_E ? ResCost{{100, 140}, {46, 60, 85}} : ResCost{{85, 115}, {46, 60, 85}};
     const double l1 = 46, l2 = 60, l4 = 77;
     return kind == SLAB_KERR_E     ? ResCost{{125, 158}, {l1, l2, l4}}
-           : kind == SLAB_KERR_REF ? ResCost{{3900, 7100}, {l1, l2, l4}}
+           : kind == SLAB_KERR_REF ? ResCost{{810, 1230}, {l1, l2, l4}}
                                    : ResCost{{90, 115}, {l1, l2, l4}};
 }
 constexpr double kResHandNs[3] = {1000, 1500, 2600};     // K = 1, 2, 4

@@ -67,7 +67,8 @@ __global__ __launch_bounds__(256) void step_op(int op, OpArgs g) {
             break;
         case 7: {  // Acubic[n] = root 0 of (cub, qua, one, -|Dx/eps0|^2)
             const double dd = a[1][n] / g.s[3];
-            a[0][n] = cubic_root0_1728(g.s[0], g.s[1], g.s[2], -(fabs(dd) * fabs(dd)));
+            a[0][n] = cubic_root0_1728(g.s[0], g.s[1], g.s[2], cubic_const(g.s[0], g.s[1], g.s[2]),
+                                       -(fabs(dd) * fabs(dd)));
             break;
         }
         case 8:   // Ex[n] = Dx[n] / (eps0 * sqrt(1.2) + eps0 * chi3 * Acubic[n])

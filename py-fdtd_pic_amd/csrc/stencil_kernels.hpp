@@ -149,7 +149,7 @@ template <typename R, int KIND>
 __device__ __forceinline__ R slab_e_simple(const SimDev<R>& sd, double u, R D, R ie) {
     if constexpr (KIND == SLAB_KERR_REF) {
         const double dd = (double)D / sd.kerr_e0;
-        const double A = cubic_root0_1728(sd.kerr_a, sd.kerr_b, sd.kerr_c, -(fabs(dd) * fabs(dd)));
+        const double A = cubic_root0_1728(sd.kerr_a, sd.kerr_b, sd.kerr_c, sd.cub, -(fabs(dd) * fabs(dd)));
         return (R)((double)D / (sd.kerr_e0 * sd.kerr_lin + sd.kerr_e0 * sd.kerr_chi3 * A));
     } else {
 #pragma clang fp contract(off)
