@@ -83,20 +83,26 @@ def Ricker(V, P):
     """Empty in the reference (BaseFDTD11.py:101-102)."""
 
 
-def SmoothTurnOn(V, P, tempfreq=0):
-    """BaseFDTD11.SmoothTurnOn (:104-120): sine for Periods periods, then zero."""
+def _smooth_tables(V, P, tempfreq=0):
+    """The tables of SmoothTurnOn as arrays, and how many steps carry the sine
+    (None: not the first ones alone)."""
     frq = tempfreq if tempfreq != 0 else P.freq_in
     ppw = P.c0 / (frq * P.dz)
-    Exs, Hys = [], []
-    limit = P.period * P.Periods
-    for timer in range(P.timeSteps):
-        if timer * P.delT < limit:
-            Exs.append(float(np.sin(2.0 * np.pi / ppw * (P.courantNo * timer))))
-            Hys.append(float(np.sin(2.0 * np.pi / ppw * (P.courantNo * (timer + 1)))))
-        else:
-            Exs.append(0)
-            Hys.append(0)
-    return Exs, Hys
+    n = len(range(P.timeSteps))
+    timer = np.arange(n + 1, dtype=np.float64)
+    on = timer[:n] * P.delT < P.period * P.Periods
+    wave = np.sin(2.0 * np.pi / ppw * (P.courantNo * timer))
+    live = int(np.count_nonzero(on))
+    return np.where(on, wave[:n], 0.0), np.where(on, wave[1:], 0.0), live if on[:live].all() else None
+
+
+def SmoothTurnOn(V, P, tempfreq=0):
+    """BaseFDTD11.SmoothTurnOn (:104-120): sine for Periods periods, then zero."""
+    Exs, Hys, live = _smooth_tables(V, P, tempfreq)
+    if live is None:                          # NaN or a negative step: zeros are not a tail
+        return Exs.tolist(), Hys.tolist()
+    tail = [0] * (len(Exs) - live)
+    return Exs[:live].tolist() + tail, Hys[:live].tolist() + tail
 
 
 def EmptySpaceCalc(V, P):
@@ -186,50 +192,44 @@ def CPML_HY_RC_Define(V, P, C_V, C_P):
     return C_V.bmY, C_V.cmY
 
 
+def _strip_cells(n, W):
+    """Cells [0, W) and (n - W, n - 1], the second run from the end as the reference walks it."""
+    return np.array([*range(0, W), *range(n - 1, n - W, -1)], dtype=np.intp)
+
+
 def CPML_Ex_Update_Coef(V, P, C_V, C_P):
     """BaseFDTD11.CPML_Ex_Update_Coef (:299-318): Cb on [0,W) and (n-W, n-1]."""
     betaE = (0.5 * V.plasmaFreqE * V.plasmaFreqE * P.permit_0 * P.delT) / (1 + 0.5 * V.gammaE * P.delT)
     a = (2 * P.permit_0 - betaE * P.delT) / (2 * P.permit_0 + betaE * P.delT)
     n = len(V.Hy)
-    for nz in list(range(0, P.pmlWidth)) + list(range(n - 1, n - P.pmlWidth, -1)):
-        C_V.eLoss_CPML[nz] = (C_V.sigma_Ex[nz] * P.delT) / (2 * P.permit_0)
-        C_V.Ca[nz] = a
-        C_V.Cb[nz] = V.UpExHcompsCo[nz] * V.UpExMat[nz]
-        C_V.Cc[nz] = P.delT / ((1 + C_V.eLoss_CPML[nz]) * P.permit_0)
+    nz = _strip_cells(n, P.pmlWidth)
+    C_V.eLoss_CPML[nz] = (C_V.sigma_Ex[nz] * P.delT) / (2 * P.permit_0)
+    C_V.Ca[nz] = a
+    C_V.Cb[nz] = V.UpExHcompsCo[nz] * V.UpExMat[nz]
+    C_V.Cc[nz] = P.delT / ((1 + C_V.eLoss_CPML[nz]) * P.permit_0)
     return C_V.eLoss_CPML, C_V.Ca, C_V.Cb, C_V.Cc
 
 
 def CPML_Hy_Update_Coef(V, P, C_V, C_P):
     """BaseFDTD11.CPML_Hy_Update_Coef (:321-330): C2 = dt/mu0 on the same cells as Cb."""
     n = len(V.Hy)
-    for nz in list(range(0, P.pmlWidth)) + list(range(n - 1, n - P.pmlWidth, -1)):
-        C_V.C1[nz] = 1
-        C_V.C2[nz] = P.delT / P.permea_0
-        C_V.C3[nz] = P.delT / ((1 + C_V.mLoss_CPML[nz]) * P.permea_0)
+    nz = _strip_cells(n, P.pmlWidth)
+    C_V.C1[nz] = 1
+    C_V.C2[nz] = P.delT / P.permea_0
+    C_V.C3[nz] = P.delT / ((1 + C_V.mLoss_CPML[nz]) * P.permea_0)
     return C_V.mLoss_CPML, C_V.C1, C_V.C2, C_V.C3
 
 
 def denominators(V, P, C_V, C_P):
     """BaseFDTD11.denominators (:332-357): 1/kappa, mirrored indices on the right."""
     n = len(V.Hy)
-    jj = P.pmlWidth
-    for j in range(n):
-        if j <= P.pmlWidth and P.CPMLXm:
-            C_V.den_Hydz[j] = 1 / C_V.kappa_Hy[j]
-        elif j >= n - P.pmlWidth and P.CPMLXp:
-            C_V.den_Hydz[j] = 1 / C_V.kappa_Hy[jj]
-            jj -= 1
-        else:
-            C_V.den_Hydz[j] = 1.0
-    jj = P.pmlWidth - 1
-    for j in range(n):
-        if j <= P.pmlWidth and P.CPMLXm:
-            C_V.den_Exdz[j] = 1 / C_V.kappa_Ex[j]
-        elif j >= n - P.pmlWidth and P.CPMLXp:
-            C_V.den_Exdz[j] = 1 / C_V.kappa_Ex[jj]
-            jj -= 1
-        else:
-            C_V.den_Exdz[j] = 1.0
+    W = P.pmlWidth
+    left = min(W + 1, n) if P.CPMLXm else 0
+    right = max(n - W, left, 0) if P.CPMLXp else n
+    for den, kappa, first in ((C_V.den_Hydz, C_V.kappa_Hy, W), (C_V.den_Exdz, C_V.kappa_Ex, W - 1)):
+        den[left:right] = 1.0
+        den[:left] = 1 / kappa[:left]
+        den[right:n] = 1 / kappa[first - np.arange(n - right)]
     return C_V.den_Exdz, C_V.den_Hydz
 
 

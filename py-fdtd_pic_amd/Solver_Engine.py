@@ -60,16 +60,16 @@ def boundCondManager(V, P, C_V, C_P):
 def SourceManager(V, P, C_V, C_P):
     """Solver_Engine.SourceManager (:89-124): SineCont (with the NL pump) or Gaussian tables."""
     if P.SineCont:
-        Exs, Hys1 = BaseFDTD11.SmoothTurnOn(V, P)
+        Exs, Hys1, _ = BaseFDTD11._smooth_tables(V, P)
         Exp, Hyp1 = np.zeros(P.timeSteps), np.zeros(P.timeSteps)
         if P.nonLinMed:
-            Exp, Hyp1 = BaseFDTD11.SmoothTurnOn(V, P, tempfreq=P.freq_in * 0.8)
-            Exp = np.asarray(Exp) * P.courantNo
-            Hyp1 = np.asarray(Hyp1) * P.courantNo
+            Exp, Hyp1, _ = BaseFDTD11._smooth_tables(V, P, tempfreq=P.freq_in * 0.8)
+            Exp = Exp * P.courantNo
+            Hyp1 = Hyp1 * P.courantNo
             Exp *= 0.1
             Hyp1 *= 0.01
-        Exs = np.asarray(Exs) * P.courantNo + Exp
-        Hys1 = np.asarray(Hys1) * P.courantNo + Hyp1
+        Exs = Exs * P.courantNo + Exp
+        Hys1 = Hys1 * P.courantNo + Hyp1
         if P.TFSF:
             Hys1 = Hys1 * (1 / P.CharImp)
         return Exs, Hys1
