@@ -805,6 +805,13 @@ static int res_tile_sim(const ResSim& q, int Kh, int Kl, int S, int box0, std::v
     return n;
 }
 
+// A tile of plain cells only, of K cells per lane (a plan whose light tiles
+// have their own K; with one K for both the heavy ones of plain simulations
+// carry the same flags and count as light).
+static bool res_light(const int4& t, int K) {
+    return (t.x & kResPlain) && !(t.x & kResEmu) && (t.x & (kResK2 | kResK4)) == (K == 4 ? kResK4 : K == 2 ? kResK2 : 0);
+}
+
 // What a block of S steps of a wave with a SIMD to itself costs: ns
 // per step and ns for the hand-off, by cells per lane (measured per tile: the
 // slowest tile, which waits for nobody, sets the pace).  Heavy tiles by slab
@@ -901,6 +908,36 @@ static int plan_resident(fdtd_ctx* c) {
     };
     long long nt = 0;
     const ResCost cost = res_cost(kind, f32);
+    // More tiles than the device holds at once: the same tiles and loops, one
+    // block per launch.  Nothing is handed over, so they need no residency;
+    // heavy tiles keep the context's cells per lane, light ones take those
+    // that cost least in all.  Snapshot rows fall between blocks, which only a
+    // resident launch can cut.  A sweep of 48 FP32 grids of up to 65,536
+    // cells at (2, 48): 82 us per launch against 124 us of one-block tiles (two
+    // launches, one per slab kind, every tile of 32 cells).
+    auto plan_blocks = [&] {
+        if (c->K > 2 || c->K_slab != c->K || 64 * c->K - 2 * c->S_run < 4) return;
+        for (int i : c->tile_sims)
+            if (c->sims[i]->d.snap_interval > 0 || c->sims[i]->d.has_current) return;
+        double least = 0.0;
+        int Kl = 0;
+        for (int k = c->K; k <= 4; k *= 2) {
+            std::vector<int4> t;
+            for (const ResSim& q : sims) res_tile_sim(q, c->K, k, c->S_run, 0, &t);
+            const long long nl = std::count_if(t.begin(), t.end(), [&](const int4& x) { return res_light(x, k); });
+            const double w = nl * cost.light[k == 4 ? 2 : k - 1] + ((long long)t.size() - nl) * cost.heavy[c->K - 1];
+            if (Kl && w >= least) continue;
+            least = w;
+            Kl = k;
+            c->res_tiles.swap(t);
+        }
+        std::stable_partition(c->res_tiles.begin(), c->res_tiles.end(), [&](const int4& x) { return !res_light(x, Kl); });
+        c->res_S = c->S_run;
+        c->res_kind = kind;
+        c->res_W = 2;
+        c->box_stale = true;                    // the mailbox belongs to another plan
+        c->blk_ok = true;
+    };
     const int cap2 = resident_capacity_per_cu<R, f32>(kind, 2);
     double best = 1e30;
     for (int Kh = 1; Kh <= 2; ++Kh)
@@ -916,9 +953,11 @@ static int plan_resident(fdtd_ctx* c) {
                                                    cost.light[l] + (hand ? kResHandNs[l] / S : 0.0));
                 if (t < best) { best = t; bKh = Kh; bKl = Kl; bS = S; nt = n; }
             }
-    if (!bKh) return FDTD_OK;
-    bW = nt > round ? 2 : 1;
-    if (nt > (long long)resident_capacity_per_cu<R, f32>(kind, bW) * round) return FDTD_OK;
+    if (bKh) bW = nt > round ? 2 : 1;
+    if (!bKh || nt > (long long)resident_capacity_per_cu<R, f32>(kind, bW) * round) {
+        plan_blocks();
+        return FDTD_OK;
+    }
     std::vector<int4> tiles;
     int box0 = 0;
     for (const ResSim& q : sims) {
@@ -1097,13 +1136,13 @@ static int rebuild_t(fdtd_ctx* c) {
     ups.push_back({&c->d_sims, &c->d_sims_cap, devs.data(), sizeof(SimDev<R>) * devs.size()});
     ups.push_back({(void**)&c->d_tiles, &c->d_tiles_cap, tiles.data(), sizeof(int2) * tiles.size()});
     // resident launches, and the conditions of the persistent request
-    c->res_ok = false;
+    c->res_ok = c->blk_ok = false;
     if (!pic && !c->grouped) {
         int rc = plan_resident<R>(c);
         if (rc) return rc;
     }
     c->persist_ok = c->persist && c->res_ok && c->groups.size() == 1 && c->K_slab == c->K && c->S_run <= U;
-    if (c->res_ok)
+    if (c->res_ok || c->blk_ok)
         ups.push_back({(void**)&c->d_rtiles, &c->d_rtiles_cap, c->res_tiles.data(), sizeof(int4) * c->res_tiles.size()});
     int rc = staged_upload(c, ups);
     if (rc) return rc;
@@ -1150,6 +1189,22 @@ static EvPair* next_event(fdtd_ctx* c, int kind) {
 // runs in one launch with the particle scatter (stamped by fev instead).
 static int launch_once(fdtd_ctx* c, int n, EvPair* ev, hipStream_t st, bool fused = false,
                        EvPair* fev = nullptr) {
+    if (c->blk_ok) {
+        if (n > c->res_S) return fdtd_fail(FDTD_E_STATE, "a block launch of more than S steps");
+        ResArgs ra{};
+        ra.nsteps = n;
+        ra.S = c->res_S;
+        ra.formK = c->K;
+        ra.stride = 1;
+        ra.err = c->d_rerr;
+        const hipError_t e = c->prec == FDTD_F64
+            ? launch_resident<double, false>((const SimDev<double>*)c->d_sims, c->d_rtiles, (int)c->res_tiles.size(),
+                                             c->launch_idx, c->gstep, c->res_kind, c->res_W, ra, st)
+            : launch_resident<float, true>((const SimDev<float>*)c->d_sims, c->d_rtiles, (int)c->res_tiles.size(),
+                                           c->launch_idx, c->gstep, c->res_kind, c->res_W, ra, st);
+        if (e != hipSuccess) return fdtd_fail(FDTD_E_HIP, std::string("block launch: ") + hipGetErrorString(e));
+        return FDTD_OK;
+    }
     const PersistArgs pa{c->grouped ? c->halo : 0};
     const size_t ng = c->groups.size();
     const size_t nplain = fused ? ng - 1 : ng;

@@ -130,6 +130,7 @@ struct fdtd_ctx {
     int res_mode = 1;                        // fdtd_set_resident
     int res_polls = kResMaxPolls;
     bool res_ok = false;                     // the active simulations fit (res_tiles, res_S, res_kind)
+    bool blk_ok = false;                     // they do not, and launches of S steps take the same tiles
     std::vector<int4> res_tiles;
     int res_S = 0, res_kind = 0, res_stride = 0, res_W = 1, res_cap = 0;
     int4* d_rtiles = nullptr;

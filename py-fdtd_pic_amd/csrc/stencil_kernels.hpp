@@ -951,7 +951,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
         for (int j = 0; j < K; ++j) {
             const int n = c.base + j;
             const bool own = (interior_mask >> j) & 1u;
-            if (own && ((has_l && n < out0 + S) || (has_r && n >= out0 + U - S))) send |= 1u << j;
+            if (ra.box && own && ((has_l && n < out0 + S) || (has_r && n >= out0 + U - S))) send |= 1u << j;
             const bool rec = !own && n >= 0 && n <= N && n < out0 + U + S;
             rv[j] = rec ? rt.w + n : spare;
             rs[j] = rec && ((slab_mask >> j) & 1u) ? rt.w + n : spare;
@@ -1036,7 +1036,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
                 }
                 k0 = k1;
             }
-            if (k0 >= total) break;
+            if (k0 >= total || !ra.box) break;      // one block: nothing to hand over
             // ---- hand-off q ----
             unsigned long long* slot = ra.box + q3 * slot_words;
             // the emptied words of the slot to come are in memory before this block's values go out

@@ -130,3 +130,15 @@ def test_resident_not_taken():
         assert c.resident_active()
         s.set_energy(1, 8)
         assert not c.resident_active()
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("slab,tiling", [("kerr", None), ("linear", (2, 48)), ("none", (2, 16)), ("kerr", (1, 24))])
+def test_more_tiles_than_the_device_holds(prec, slab, tiling):
+    # one launch per block of steps with the resident plan's tiles: grids of one
+    # or two tiles, ragged ones, different lengths, a run cut into pieces
+    grids = [(65536, {}), (65003, {}), (40, {}), (61007, dict(F=70, R=20000)), (193, {}),
+             (4097, dict(F=2000, R=2003))] + [(65536 - 977 * i, {}) for i in range(19)]
+    specs = [_phys(n, 120 + k, "none" if n == 40 else slab, **(kw if slab != "none" else {}))
+             for k, (n, kw) in enumerate(grids)]
+    _same(specs, prec, f"blocks {slab} {tiling}", taken=False, cuts=(37, 1), tiling=tiling)
