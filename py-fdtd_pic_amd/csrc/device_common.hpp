@@ -96,6 +96,9 @@ struct ResArgs {
     int32_t* herr;               // host memory
     int max_polls;
 };
+// Flags of a one-block tile entry beside the simulation's index.
+constexpr int kTileNarrow = 1 << 24;     // half the cells per lane
+constexpr int kTilePlain = 1 << 25;      // no D-form slab, in a launch of a slab kind (field_scatter)
 // Tile of a resident launch: x = simulation | flags, y, z = first owned cell
 // and the one after the last, w = the simulation's first cell in the mailbox.
 constexpr int kResK2 = 1 << 24, kResK4 = 1 << 25;   // cells per lane: 1, 2 or 4

@@ -1041,7 +1041,7 @@ static int rebuild_t(fdtd_ctx* c) {
         }
         for (int o = 0; o <= s->d.N;) {
             const bool narrow = slabby && o - c->S_run < s->d.R && o + U + c->S_run > s->d.F;
-            by_kind[kind].push_back(make_int2(i | (narrow ? 1 << 24 : 0), o));
+            by_kind[kind].push_back(make_int2(i | (narrow ? kTileNarrow : 0), o));
             o += narrow ? Un : U;
         }
     }
@@ -1115,7 +1115,7 @@ static int rebuild_t(fdtd_ctx* c) {
         for (size_t t0 = 0; t0 < by_kind[k].size(); t0 += step) {
             const int2 t = by_kind[k][t0];
             const SimHost* sh = c->sims[t.x & 0xffffff];
-            const int Ut = (t.x >> 24) ? Un : U;
+            const int Ut = (t.x & kTileNarrow) ? Un : U;
             const int lo = c->grouped ? t.y : t.y - c->S_run;
             const int hi = c->grouped ? t.y + Lg : t.y + Ut + c->S_run;
             bool h = (sh->d.slab_kind >= FDTD_SLAB_LINEAR && lo < sh->d.R && hi > sh->d.F) || lo < sh->d.Ls ||
@@ -1125,6 +1125,17 @@ static int rebuild_t(fdtd_ctx* c) {
         }
         by_kind[k].swap(heavy);
         by_kind[k].insert(by_kind[k].end(), light.begin(), light.end());
+    }
+    // A beam step's field tiles in one launch with the scatter: the plain
+    // simulations' join those of the slab kind, where there is one only
+    if (c->has_pic && c->fuse_pic && (c->K == 1 || c->K == 2) && !by_kind[SLAB_DIEL].empty()) {
+        int other = -1, others = 0;
+        for (int k = SLAB_DIEL + 1; k < 5; ++k)
+            if (!by_kind[k].empty()) { other = k; ++others; }
+        if (others == 1 && by_kind[SLAB_DIEL].size() + by_kind[other].size() <= (size_t)kFuseMaxTiles) {
+            for (int2 t : by_kind[SLAB_DIEL]) by_kind[other].push_back(make_int2(t.x | kTilePlain, t.y));
+            by_kind[SLAB_DIEL].clear();
+        }
     }
     std::vector<int2> tiles;
     c->groups.clear();
@@ -1390,12 +1401,13 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
         const bool prof = c->profile > 0 && (c->launches % c->profile) == 0;
         // event handles are copied out at once: next_event may grow (move) the vector
         hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, e3 = nullptr;
-        // the fused launch takes field tiles of 1 or 2 cells per lane, and
-        // only a small field launch: the fused kernel has the field tile's
+        // the fused launch takes field tiles of 1 or 2 cells per lane, and no
+        // very large field launch: the fused kernel has the field tile's
         // register count, which cuts the scatter's occupancy (FP32: 8 -> 3
-        // waves per SIMD), so a large field launch keeps its own (config 4's
-        // 2,048 beam passes: 2.11 ms per step fused against 1.74 separate;
-        // config 3's 1,024 tiles: 13.8 us fused against 4.8 + 11.9)
+        // waves per SIMD).  config 4's 2,048 beam passes: 2.11 ms per step
+        // fused against 1.74 separate; sweeps of 24 beam points (~6,000 tiles)
+        // 147 / 153 us per step in FP32, 178 / 183 in FP64; of 64 (~16,000)
+        // 362 / 361 and 430 / 440; config 3's 1,024 tiles 13.8 / 16.7
         const bool fused = c->has_pic && c->fuse_pic && (c->K == 1 || c->K == 2) && !c->groups.empty() &&
                            c->groups.back().count <= kFuseMaxTiles;
         if (c->has_pic) {
@@ -1822,6 +1834,7 @@ int fdtd_set_profile(fdtd_ctx* c, int every) {
 int fdtd_set_pic_fusion(fdtd_ctx* c, int on) {
     if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
     if (on != 0 && on != 1) return fdtd_fail(FDTD_E_ARG, "pic fusion flag must be 0 or 1");
+    if (c->fuse_pic != (on != 0)) c->dirty = true;      // the tile groups follow it
     c->fuse_pic = on != 0;
     return FDTD_OK;
 }

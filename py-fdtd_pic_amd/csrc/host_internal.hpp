@@ -171,7 +171,7 @@ template <typename R>
 constexpr long long kCoopGroupsPerCu = sizeof(R) == 4 ? 6 : 4;
 
 // Largest field launch (tiles) that takes the particle scatter into its grid.
-constexpr int kFuseMaxTiles = 2048;
+constexpr int kFuseMaxTiles = 8192;
 
 constexpr int kThrottleEvery = 128;
 constexpr size_t kThrottleDepth = 4;

@@ -1162,7 +1162,7 @@ __device__ __forceinline__ void field_tile(const SimDev<R>* __restrict__ sims, c
     const int4 rt{0, 0, 0, 0};
     const ResArgs ra{};
     if constexpr (KW > 1 && !GROUP) {
-        if (tl.x >> 24) {
+        if (tl.x & kTileNarrow) {
             tile_body<R, KW / 2, KAHAN, KIND, false>(sd, tl.y, launch_idx, gstep0, nsteps, S, pa, rt, ra);
             return;
         }

@@ -287,3 +287,38 @@ def test_group_per_workgroup_equals_group_per_wave(prec, per_cell, group):
     assert np.abs(outs[0]["J"]).max() > 0
     for k in outs[0]:
         assert np.array_equal(outs[0][k], outs[1][k]), k
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_plain_and_slab_beams_share_a_launch(prec):
+    """A vacuum beam's field tiles ride in the launch of the slab beams': the
+    same bits as alone in a context, also when the fusion is switched off and
+    on between runs."""
+    from fdtd_pic_amd import configs, engine
+    rng = np.random.default_rng(5)
+
+    def spec(N, slab):
+        p = configs.base(N, 90, slab_start=60, slab_stop=90 if slab else 60, src_cell=200, probes=[150, N - 60],
+                         src_t0=5e-15, src_tau=2e-15, src_amp=1e6)
+        return engine.physical_spec(p)
+
+    def beam():
+        return engine.Beam(300 + rng.uniform(0.0, 80, 4000), rng.normal(0.0, 0.15, (4000, 3)), -configs.E_CHARGE,
+                           configs.M_ELECTRON, 1e9, configs.DT, configs.DZ)
+
+    jobs = [(spec(700, True), beam()), (spec(641, False), beam()), (spec(1003, False), beam())]
+    outs = []
+    for group in ([jobs], [[j] for j in jobs]):
+        out = []
+        for part in group:
+            with engine.Context(prec, K=1, S=1) as c:
+                sims = [c.add(s, beam=b) for s, b in part]
+                for k, n in enumerate((30, 30, 30)):
+                    c.set_pic_fusion(k != 1)
+                    c.run(n)
+                out += [{"E": s.read("E"), "H": s.read("H"), "J": s.read("J"), "u": s.particles()[1]} for s in sims]
+        outs.append(out)
+    for x, y in zip(*outs):
+        assert np.abs(x["J"]).max() > 0
+        for k in x:
+            assert np.array_equal(x[k], y[k]), k
