@@ -151,6 +151,8 @@ struct fdtd_ctx {
     int pc_single = -1;         // the one-cell items' beam when there is one, else -1
     void* d_scratch = nullptr;               // spectra: pointer table, frequencies, results
     size_t d_scratch_cap = 0;
+    void* op_stage = nullptr;                // pinned: the cells of a single step function (fdtd_step_op)
+    size_t op_cap = 0;
 };
 
 int fdtd_fail(int code, const std::string& msg);
