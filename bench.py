@@ -43,8 +43,8 @@ def parse():
     ap.add_argument("--S", type=int, default=0)
     ap.add_argument("--K-slab", type=int, default=0, help="cells per lane of slab tiles (K or K/2; 0: default)")
     ap.add_argument("--persistent", default="off", choices=["on", "off"],
-                    help="config 2: persistent field launches (many blocks of S steps per launch; measured "
-                         "slower than one-block launches at K=2 S=48, faster at K=1 and K=4 shapes)")
+                    help="config 2: ask for persistent launches (resident launches under uniform tiles with "
+                         "S <= 64K - 2S); resident launches are the default wherever the tiles fit")
     ap.add_argument("--halo", type=int, default=0,
                     help="config 2: workgroup halo exchange every H steps (0: off)")
     ap.add_argument("--cpu-seconds", type=float, default=10.0, help="target CPU baseline sample length")
@@ -338,6 +338,7 @@ def config2_line(a, precision):
     ctx.set_halo_exchange(a.halo)
     sim = ctx.add(engine.physical_spec(p))
     persistent = ctx.persistent_active()
+    resident = ctx.resident_active()
     halo = a.halo if ctx.halo_exchange_active() else 0
     for _ in range(a.warmup):
         sim.reset()
@@ -356,7 +357,7 @@ def config2_line(a, precision):
     cells = p["N"] * p["steps"]
     value = cells / (wall / a.steps) / 1e9
     bpc = configs.bytes_per_cell_update(p, precision)
-    launch_ms = kern_ms / max(sampled, 1)                 # average launch-to-launch duration
+    launch_ms = kern_ms / max(sampled, 1)                 # average duration of S steps (a launch, or a resident block)
     achieved = bpc * p["N"] * S / (launch_ms / 1e3) / 1e9 if kern_ms > 0 else 0.0
     out = {
         "metric": METRIC,
@@ -373,7 +374,7 @@ def config2_line(a, precision):
         "data": "synthetic (seeded config 2 parameters)",
         "config": {"workload": "config2: N=65536 cells, 50000 steps, Lorentz+Kerr slab [20000,40000)",
                    "sim_steps": p["steps"], "K": K, "K_slab": Ks, "S": S, "precision": precision,
-                   "persistent": persistent, "halo_exchange": halo},
+                   "persistent": persistent, "resident": resident, "halo_exchange": halo},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": measured_traffic(precision, K, S, Ks),
@@ -381,9 +382,10 @@ def config2_line(a, precision):
                      "bytes_per_cell_update": round(bpc, 2),
                      "avg_launch_us": round(launch_ms * 1e3, 2), "sampled_launches": sampled,
                      "launches": a.steps * ((p["steps"] + S - 1) // S),
-                     "note": "achieved = algorithmic bytes of the one-step streaming count per launch over the "
-                             "launch time: an effective figure (temporal blocking keeps the state on chip); "
-                             "the DRAM bytes the kernel moves are `traffic`, dram_frac their rate over the peak"},
+                     "note": "a launch here is a block of S steps (resident runs do all of them in one kernel); "
+                             "achieved = algorithmic bytes of the one-step streaming count per block over its "
+                             "time: an effective figure (the state stays on chip); the DRAM bytes the kernel "
+                             "moves are `traffic`, dram_frac their rate over the peak"},
     }
     tr = out["roofline"]["traffic"]
     if tr and kern_ms > 0:

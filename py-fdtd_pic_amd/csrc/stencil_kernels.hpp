@@ -1099,6 +1099,11 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
                     unpack2(w[j][0], E[j], cE[j]);
                     unpack2(w[j][1], H[j], cH[j]);
                     if ((emu_mask >> j) & 1u) emulate(j);
+                } else if (KAHAN && ((emu_mask >> j) & 1u)) {
+                    // a block of its own would read E and its compensation back: (D, cD) is the same
+                    // value, but where |cD| is half a unit of D in the last place E is not D
+                    cE[j] = comp_e(j);
+                    emulate(j);
                 }
                 if (any_slab && rs[j] != spare) {
                     unpack2(w[j][2], D[j], cD[j]);
@@ -1184,9 +1189,26 @@ __global__ __launch_bounds__(64 * kTileWaves) void stencil_tiles(const SimDev<R>
     field_tile<R, KW, KAHAN, KIND, GROUP>(sims, tiles, tid, launch_idx, gstep0, nsteps, S, pa);
 }
 
-// Resident launch: tile t is wave t % 4 of workgroup t / 4; W workgroups fit
-// on a CU.  RESDOC
-// Tiles hold 1 or 2 cells per lane, plain ones up to 4.
+// Resident launch: tile t is wave t % 4 of workgroup t / 4, W workgroups fit
+// on a CU, and a whole run is one launch.  A tile keeps its window in registers
+// from the first step to the last; every S steps it hands its edge cells to its
+// neighbours through the mailbox (tile_body) and reads theirs.
+//
+// Bound: the instruction stream of the slowest tile plus its hand-off.  A
+// Lorentz run of 2,000 cells (one cell per lane, S = 28): 95-100 ns per step of
+// the source and slab tiles and 1.25 us per hand-off (0.25 to send, one trip
+// over the fabric to read), 150 ns per step in all; one launch per block took
+// 459 ns.  A Kerr grid of 65,536 cells, two cells per lane, S = 48: 146-152 ns
+// per step and 1.75 us per hand-off, 226 ns per step (FP32) against 273; FP64
+// 305 against 503.  XCDs run at clocks that differ by a tenth, and the slowest
+// one sets the pace of all tiles.
+//
+// Tiles hold 1 or 2 cells per lane, plain ones up to 4: light tiles (plain
+// cells alone) take 46, 60 and 77-85 ns per step at 1, 2 and 4 cells per lane,
+// so wide ones leave waves for narrow slab tiles.
+//
+// With ra.box null the launch is one block of at most S steps: nothing is
+// handed over and the tiles need not be on the device together.
 template <typename R, bool KAHAN, int KIND, int W>
 __global__ __launch_bounds__(64 * kTileWaves, W) void stencil_resident(const SimDev<R>* __restrict__ sims,
                                                                        const int4* __restrict__ tiles, int ntiles,

@@ -142,3 +142,14 @@ def test_more_tiles_than_the_device_holds(prec, slab, tiling):
     specs = [_phys(n, 120 + k, "none" if n == 40 else slab, **(kw if slab != "none" else {}))
              for k, (n, kw) in enumerate(grids)]
     _same(specs, prec, f"blocks {slab} {tiling}", taken=False, cuts=(37, 1), tiling=tiling)
+
+
+@pytest.mark.parametrize("slab", ["kerr", "linear"])
+def test_resident_f32_long_runs(slab):
+    """Roundings that a run meets once in some 1e8 cell-steps: an emulated
+    vacuum cell beside the slab whose compensation is half a unit of its value
+    in the last place, so that E is not D."""
+    for n in (25013, 24007, 23011, 22003, 9001, 5003):
+        F = n // 2
+        _same([_phys(n, 24001, slab, F=F, R=F + 400 + n % 100, src_cell=100, probes=[60, n - 42],
+                     **(dict(chi3=0.0) if slab == "linear" else {}))], "f32", f"long {slab} {n}")
