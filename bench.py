@@ -5,11 +5,11 @@
 One bench step = one complete simulation of the workload (N = 65,536 cells,
 50,000 time steps, Lorentz+Kerr slab of 20,000 cells with per-cell eps_inf
 and w0), with coefficients already resident on the device: the timed region
-holds the state reset and every stencil launch.  The metric is cell-updates
+holds the state reset and every field launch (one resident launch per run).  The metric is cell-updates
 per second (N * steps / time).  The roofline object prices the stencil at
 the algorithmic bytes of a one-step streaming schedule (bytes/cell-update x
-cells x steps per launch) over the average launch duration measured with HIP
-events on the context stream; cpu_baseline times the C restatement
+cells x steps per block) over the average duration of a block of S steps,
+measured with HIP events on the context stream; cpu_baseline times the C restatement
 (oracle/fdtd_cpu.c, FP64, OpenMP over cells) on a bounded slice of the same
 workload.
 """
@@ -77,8 +77,8 @@ def parse():
     return ap.parse_args()
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "stencil_tiles_config2_hbm_traffic.txt")
-ISSUE_FILE = os.path.join(ROOT, "profiles", "stencil_tiles_config2_valu_issue.txt")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "stencil_resident_config2_hbm_traffic.txt")
+ISSUE_FILE = os.path.join(ROOT, "profiles", "stencil_resident_config2_valu_issue.txt")
 # VALU issue peak without packed FP32: 256 CUs x 4 SIMDs x 2.4 GHz, one wave64
 # instruction per 4 cycles per SIMD (G wave-instructions/s)
 VALU_ISSUE_PEAK = 256 * 4 * 2.4 / 4
@@ -97,7 +97,7 @@ def calibrate_copy():
 
 
 def measured_traffic(precision, K, S, Ks):
-    """HBM bytes per stencil launch from the committed rocprofv3 --pmc summary
+    """HBM bytes per block of S steps from the committed rocprofv3 --pmc summary
     (FETCH_SIZE and WRITE_SIZE per dispatch, scaled by a copy-kernel
     calibration), or None when no summary matches this tiling."""
     if not os.path.exists(TRAFFIC_FILE):
@@ -111,7 +111,7 @@ def measured_traffic(precision, K, S, Ks):
 
 
 def measured_issue(precision, K, S, Ks):
-    """VALU wave-instructions per field launch from the committed rocprofv3
+    """VALU wave-instructions per block of S steps from the committed rocprofv3
     --pmc SQ_INSTS_VALU summary, or None when none matches this tiling."""
     if not os.path.exists(ISSUE_FILE):
         return None
@@ -387,20 +387,17 @@ def config2_line(a, precision):
                              "time: an effective figure (the state stays on chip); the DRAM bytes the kernel "
                              "moves are `traffic`, dram_frac their rate over the peak"},
     }
-    tr = out["roofline"]["traffic"]
+    tr = out["roofline"]["traffic"] = out["roofline"]["traffic"] if resident else None    # measured on resident runs
     if tr and kern_ms > 0:
         out["roofline"]["dram_frac"] = round(tr / (launch_ms / 1e3) / 1e9 / HBM_PEAK_GBS, 4)
     issued = measured_issue(precision, K, S, Ks)
-    if issued and kern_ms > 0 and not persistent:
+    if issued and kern_ms > 0 and resident:
         rate = issued / (launch_ms / 1e3) / 1e9
-        U = 64 * K - 2 * S
         out["issue"] = {"bound": "valu_issue", "achieved": round(rate, 1), "peak": VALU_ISSUE_PEAK,
                         "unit": "G wave-instructions/s", "frac": round(rate / VALU_ISSUE_PEAK, 4),
                         "wave_insts_per_launch": issued,
                         "lane_insts_per_cell_update": round(issued * 64 / (p["N"] * S), 1),
-                        "useful_fraction": round(U / (64 * K), 3),
-                        "useful_lane_insts_per_cell_update": round(issued * 64 / (p["N"] * S) * U / (64 * K), 1),
-                        "source": "rocprofv3 --pmc SQ_INSTS_VALU (profiles/stencil_tiles_config2_valu_issue.txt) "
+                        "source": "rocprofv3 --pmc SQ_INSTS_VALU (profiles/stencil_resident_config2_valu_issue.txt) "
                                   "over the live launch time"}
     ctx.close()
     return out, p
