@@ -830,8 +830,106 @@ static ResCost res_cost(int kind, bool f32) {
 }
 constexpr double kResHandNs[3] = {1000, 1500, 2600};     // K = 1, 2, 4
 
+// Simulation i for the tile plan; false where its tiles have no lean class.
+template <typename R>
+static bool res_sim(const fdtd_ctx* c, int i, ResSim& q) {
+    constexpr bool f32 = sizeof(R) == 4;
+    const fdtd_sim_desc_t& d = c->sims[i]->d;
+    q.id = i;
+    q.N = d.N;
+    q.plain = d.slab_kind < SLAB_LINEAR;
+    q.last_dead = c->sims[i]->last_dead;
+    if (!q.plain) q.heavy.push_back({d.F, d.R, true});
+    if (d.Ls > 0) q.heavy.push_back({0, d.Ls, true});
+    if (d.Rs <= d.N) q.heavy.push_back({d.Rs, d.N + 1, true});
+    q.heavy.push_back({d.src_cell - 1, d.src_cell + 1, true});
+    for (int p = 0; p < d.nprobe; ++p) q.heavy.push_back({d.probe_cell[p], d.probe_cell[p] + 1, false});
+    if (d.has_current) q.heavy.push_back({0, d.N + 1, true});       // the general class everywhere
+    if (f32) {
+        // no general class: a current, or more than two probes in one tile
+        if (d.has_current) return false;
+        const int U0 = 64 * c->K - 2 * c->S_run;
+        for (int p = 0; p < d.nprobe; ++p) {
+            int same = 0;
+            for (int r = 0; r < d.nprobe; ++r) same += d.probe_cell[r] / U0 == d.probe_cell[p] / U0;
+            if (same > 2) return false;
+        }
+        // the one-block tiles whose vacuum cells are emulated (tile_body)
+        const int L = 64 * c->K, S0 = c->S_run;
+        if (d.slab_kind == SLAB_KERR_E && (float)d.ke0 == (float)d.kD && (float)d.jD == 1.0f)
+            for (int t = std::max(0, (d.F - L) / U0); t * U0 <= d.N && t * U0 - S0 < d.R; ++t) {
+                const int t0 = t * U0 - S0, t1 = t0 + L;
+                if (t1 <= d.F || (t0 >= d.F && t1 <= d.R)) continue;              // no slab, or only slab
+                if (t0 < 0 || t1 - 1 > d.N || t0 < d.Ls || t1 > d.Rs) continue;   // cells off the grid, strips
+                if ((d.src_cell >= t0 && d.src_cell < t1) || (d.tfsf && d.src_cell - 1 >= t0 && d.src_cell - 1 < t1))
+                    continue;
+                bool probe = false;
+                for (int p = 0; p < d.nprobe; ++p) probe = probe || d.probe_cell[p] / U0 == t;
+                if (!probe) q.emu.push_back({t * U0, std::min((t + 1) * U0, d.N + 1)});
+            }
+    }
+    return true;
+}
+
+// More tiles than the device holds at once: the resident plan's tiles and
+// loops, one block per launch.  Nothing is handed over, so they need no
+// residency; heavy tiles keep the context's cells per lane, light ones take
+// those that cost a simulation least.  Snapshot rows fall between blocks,
+// which only a resident launch can cut.  A sweep of 48 FP32 grids of up to
+// 65,536 cells at (2, 48): 82 us per launch against 124 us of one-block tiles
+// (two launches, one per slab kind, every tile of 32 cells).
+// A simulation's list is kept for the (K, S) it was made for: a batch of
+// thousands is planned again whenever one of them ends.
+template <typename R>
+static int plan_blocks(fdtd_ctx* c, int kind, const ResCost& cost) {
+    if (c->K > 2 || c->K_slab != c->K || 64 * c->K - 2 * c->S_run < 4) return FDTD_OK;
+    size_t nt = 0, nh = 0;
+    for (int i : c->tile_sims) {
+        SimHost& s = *c->sims[i];
+        if (s.d.snap_interval > 0 || s.d.has_current) return FDTD_OK;
+        if (s.blk_K != c->K || s.blk_S != c->S_run) {
+            s.blk_K = c->K;
+            s.blk_S = c->S_run;
+            s.blk.clear();
+            s.blk_heavy = 0;
+            ResSim q;
+            s.blk_fit = res_sim<R>(c, i, q);
+            double least = 0.0;
+            for (int k = c->K; k <= 4 && s.blk_fit; k *= 2) {
+                std::vector<int4> t;
+                res_tile_sim(q, c->K, k, c->S_run, 0, &t);
+                const auto mid = std::stable_partition(t.begin(), t.end(), [&](const int4& x) { return !res_light(x, k); });
+                const double w = (t.end() - mid) * cost.light[k == 4 ? 2 : k - 1] + (mid - t.begin()) * cost.heavy[c->K - 1];
+                if (!s.blk.empty() && w >= least) continue;
+                least = w;
+                s.blk_heavy = (int)(mid - t.begin());
+                s.blk.swap(t);
+            }
+        }
+        if (!s.blk_fit) return FDTD_OK;
+        nt += s.blk.size();
+        nh += s.blk_heavy;
+    }
+    // costly tiles first
+    c->res_tiles.resize(nt);
+    size_t h = 0, l = nh;
+    for (int i : c->tile_sims) {
+        const SimHost& s = *c->sims[i];
+        std::copy(s.blk.begin(), s.blk.begin() + s.blk_heavy, c->res_tiles.begin() + h);
+        std::copy(s.blk.begin() + s.blk_heavy, s.blk.end(), c->res_tiles.begin() + l);
+        h += s.blk_heavy;
+        l += s.blk.size() - s.blk_heavy;
+    }
+    c->res_S = c->S_run;
+    c->res_kind = kind;
+    c->res_W = 2;
+    c->box_stale = true;                    // the mailbox belongs to another plan
+    c->blk_ok = true;
+    return FDTD_OK;
+}
+
 // Decides whether the context's active simulations run resident, and their
-// tiles (res_ok, res_tiles, res_S, res_kind, res_stride).
+// tiles (res_ok, res_tiles, res_S, res_kind, res_stride), or in blocks.
 template <typename R>
 static int plan_resident(fdtd_ctx* c) {
     constexpr bool f32 = sizeof(R) == 4;
@@ -843,103 +941,46 @@ static int plan_resident(fdtd_ctx* c) {
                 64 * c->K - 2 * c->S_run < 1))
         return FDTD_OK;
     bool kerr = false;
+    long long cells = 0;
     for (int i : c->tile_sims) {
         const SimHost& s = *c->sims[i];
         if (s.e_every > 0) return FDTD_OK;            // energy is taken launch by launch
         kerr = kerr || (s.d.slab_kind == SLAB_KERR_E && s.d.kerr_chi3 != 0.0);
+        cells += s.d.N + 1;
     }
-    int kind = SLAB_DIEL, stride = 1;
-    long long cells = 0;
-    std::vector<ResSim> sims;
+    int kind = SLAB_DIEL;
     for (int i : c->tile_sims) {
         const fdtd_sim_desc_t& d = c->sims[i]->d;
+        if (d.slab_kind < SLAB_LINEAR) continue;
+        // a Kerr slab with chi3 = 0 is the linear slab bit for bit (the
+        // root's series is then exactly 1)
+        const int k = d.slab_kind == SLAB_KERR_E && !kerr ? SLAB_LINEAR : d.slab_kind;
+        if (kind != SLAB_DIEL && k != kind) return FDTD_OK;
+        kind = k;
+    }
+    const ResCost cost = res_cost(kind, f32);
+    const int cap2 = resident_capacity_per_cu<R, f32>(kind, 2);
+    const int round = c->cu_count * kTileWavesHost;       // one wave per SIMD
+    const int widest = 64 * 4 - 2 * (f32 ? c->S_run : 4);
+    if (cells > (1 << 28) || cells / widest > (long long)cap2 * round) return plan_blocks<R>(c, kind, cost);
+    std::vector<ResSim> sims;
+    for (int i : c->tile_sims) {
         ResSim q;
-        q.id = i;
-        q.N = d.N;
-        q.plain = d.slab_kind < SLAB_LINEAR;
-        q.last_dead = c->sims[i]->last_dead;
-        if (!q.plain) {
-            // a Kerr slab with chi3 = 0 is the linear slab bit for bit (the
-            // root's series is then exactly 1)
-            const int k = d.slab_kind == SLAB_KERR_E && !kerr ? SLAB_LINEAR : d.slab_kind;
-            if (kind != SLAB_DIEL && k != kind) return FDTD_OK;
-            kind = k;
-            q.heavy.push_back({d.F, d.R, true});
-        }
-        if (d.Ls > 0) q.heavy.push_back({0, d.Ls, true});
-        if (d.Rs <= d.N) q.heavy.push_back({d.Rs, d.N + 1, true});
-        q.heavy.push_back({d.src_cell - 1, d.src_cell + 1, true});
-        for (int p = 0; p < d.nprobe; ++p) q.heavy.push_back({d.probe_cell[p], d.probe_cell[p] + 1, false});
-        if (d.has_current) q.heavy.push_back({0, d.N + 1, true});       // the general class everywhere
-        if (f32) {
-            // no general class: a current, or more than two probes in one tile
-            if (d.has_current) return FDTD_OK;
-            const int U0 = 64 * c->K - 2 * c->S_run;
-            for (int p = 0; p < d.nprobe; ++p) {
-                int same = 0;
-                for (int r = 0; r < d.nprobe; ++r) same += d.probe_cell[r] / U0 == d.probe_cell[p] / U0;
-                if (same > 2) return FDTD_OK;
-            }
-            // the one-block tiles whose vacuum cells are emulated (tile_body)
-            const int L = 64 * c->K, S0 = c->S_run;
-            if (d.slab_kind == SLAB_KERR_E && (float)d.ke0 == (float)d.kD && (float)d.jD == 1.0f)
-                for (int t = std::max(0, (d.F - L) / U0); t * U0 <= d.N && t * U0 - S0 < d.R; ++t) {
-                    const int t0 = t * U0 - S0, t1 = t0 + L;
-                    if (t1 <= d.F || (t0 >= d.F && t1 <= d.R)) continue;              // no slab, or only slab
-                    if (t0 < 0 || t1 - 1 > d.N || t0 < d.Ls || t1 > d.Rs) continue;   // cells off the grid, strips
-                    if ((d.src_cell >= t0 && d.src_cell < t1) || (d.tfsf && d.src_cell - 1 >= t0 && d.src_cell - 1 < t1))
-                        continue;
-                    bool probe = false;
-                    for (int p = 0; p < d.nprobe; ++p) probe = probe || d.probe_cell[p] / U0 == t;
-                    if (!probe) q.emu.push_back({t * U0, std::min((t + 1) * U0, d.N + 1)});
-                }
-        }
-        cells += d.N + 1;
+        if (!res_sim<R>(c, i, q)) return FDTD_OK;
         sims.push_back(std::move(q));
     }
-    if (cells > (1 << 28)) return FDTD_OK;
-    stride += (int)cells;
+    const int stride = 1 + (int)cells;
     int bKh = 0, bKl = 0, bS = 0, bW = 0;
-    const int round = c->cu_count * kTileWavesHost;       // one wave per SIMD
     auto count = [&](int Kh, int Kl, int S, long long most) {
         if (cells / (64 * std::max(Kh, Kl) - 2 * S) > most) return most + 1;
         long long n = 0;
-        for (const ResSim& q : sims) n += res_tile_sim(q, Kh, Kl, S, 0, nullptr);
+        for (const ResSim& q : sims) {
+            n += res_tile_sim(q, Kh, Kl, S, 0, nullptr);
+            if (n > most) break;
+        }
         return n;
     };
     long long nt = 0;
-    const ResCost cost = res_cost(kind, f32);
-    // More tiles than the device holds at once: the same tiles and loops, one
-    // block per launch.  Nothing is handed over, so they need no residency;
-    // heavy tiles keep the context's cells per lane, light ones take those
-    // that cost least in all.  Snapshot rows fall between blocks, which only a
-    // resident launch can cut.  A sweep of 48 FP32 grids of up to 65,536
-    // cells at (2, 48): 82 us per launch against 124 us of one-block tiles (two
-    // launches, one per slab kind, every tile of 32 cells).
-    auto plan_blocks = [&] {
-        if (c->K > 2 || c->K_slab != c->K || 64 * c->K - 2 * c->S_run < 4) return;
-        for (int i : c->tile_sims)
-            if (c->sims[i]->d.snap_interval > 0 || c->sims[i]->d.has_current) return;
-        double least = 0.0;
-        int Kl = 0;
-        for (int k = c->K; k <= 4; k *= 2) {
-            std::vector<int4> t;
-            for (const ResSim& q : sims) res_tile_sim(q, c->K, k, c->S_run, 0, &t);
-            const long long nl = std::count_if(t.begin(), t.end(), [&](const int4& x) { return res_light(x, k); });
-            const double w = nl * cost.light[k == 4 ? 2 : k - 1] + ((long long)t.size() - nl) * cost.heavy[c->K - 1];
-            if (Kl && w >= least) continue;
-            least = w;
-            Kl = k;
-            c->res_tiles.swap(t);
-        }
-        std::stable_partition(c->res_tiles.begin(), c->res_tiles.end(), [&](const int4& x) { return !res_light(x, Kl); });
-        c->res_S = c->S_run;
-        c->res_kind = kind;
-        c->res_W = 2;
-        c->box_stale = true;                    // the mailbox belongs to another plan
-        c->blk_ok = true;
-    };
-    const int cap2 = resident_capacity_per_cu<R, f32>(kind, 2);
     double best = 1e30;
     for (int Kh = 1; Kh <= 2; ++Kh)
         for (int Kl = Kh; Kl <= 4; Kl *= 2)
@@ -955,10 +996,7 @@ static int plan_resident(fdtd_ctx* c) {
                 if (t < best) { best = t; bKh = Kh; bKl = Kl; bS = S; nt = n; }
             }
     if (bKh) bW = nt > round ? 2 : 1;
-    if (!bKh || nt > (long long)resident_capacity_per_cu<R, f32>(kind, bW) * round) {
-        plan_blocks();
-        return FDTD_OK;
-    }
+    if (!bKh || nt > (long long)resident_capacity_per_cu<R, f32>(kind, bW) * round) return plan_blocks<R>(c, kind, cost);
     std::vector<int4> tiles;
     int box0 = 0;
     for (const ResSim& q : sims) {
@@ -1030,6 +1068,16 @@ static int rebuild_t(fdtd_ctx* c) {
         }
         if (s->steps_done >= s->d.steps) continue;
         c->tile_sims.push_back(i);
+    }
+    // resident launches, or blocks with the same tiles, which need no other list
+    c->res_ok = c->blk_ok = false;
+    if (!pic && !c->grouped) {
+        int rc = plan_resident<R>(c);
+        if (rc) return rc;
+    }
+    for (int i : c->tile_sims) {
+        if (c->blk_ok) break;
+        const SimHost* s = c->sims[i];
         const int kind = s->d.slab_kind == FDTD_SLAB_NONE ? FDTD_SLAB_DIEL : s->d.slab_kind;
         // a tile whose plain-width window [o - S, o + U + S) meets a D-form
         // slab is narrow (K/2 cells per lane) when the tiling asks for it
@@ -1146,19 +1194,15 @@ static int rebuild_t(fdtd_ctx* c) {
         tiles.insert(tiles.end(), by_kind[k].begin(), by_kind[k].end());
     }
     ups.push_back({&c->d_sims, &c->d_sims_cap, devs.data(), sizeof(SimDev<R>) * devs.size()});
-    ups.push_back({(void**)&c->d_tiles, &c->d_tiles_cap, tiles.data(), sizeof(int2) * tiles.size()});
-    // resident launches, and the conditions of the persistent request
-    c->res_ok = c->blk_ok = false;
-    if (!pic && !c->grouped) {
-        int rc = plan_resident<R>(c);
-        if (rc) return rc;
-    }
+    if (!c->blk_ok)
+        ups.push_back({(void**)&c->d_tiles, &c->d_tiles_cap, tiles.data(), sizeof(int2) * tiles.size()});
+    // the conditions of the persistent request
     c->persist_ok = c->persist && c->res_ok && c->groups.size() == 1 && c->K_slab == c->K && c->S_run <= U;
     if (c->res_ok || c->blk_ok)
         ups.push_back({(void**)&c->d_rtiles, &c->d_rtiles_cap, c->res_tiles.data(), sizeof(int4) * c->res_tiles.size()});
     int rc = staged_upload(c, ups);
     if (rc) return rc;
-    c->ntiles = (int)tiles.size();
+    c->ntiles = (int)(c->blk_ok ? c->res_tiles.size() : tiles.size());
     c->dirty = false;
     return FDTD_OK;
 }

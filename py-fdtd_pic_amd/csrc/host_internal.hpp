@@ -27,6 +27,10 @@ struct SimHost {
     int e_every = 0, e_rows = 0, e_count = 0;
     long long e_launches = 0;   // launches in which this simulation stepped, since energy was set
     std::vector<int64_t> e_steps;   // step index after which each row was taken
+    // its tiles in block launches, costly ones first, made for (blk_K, blk_S)
+    std::vector<int4> blk;
+    int blk_heavy = 0, blk_K = 0, blk_S = 0;
+    bool blk_fit = false;
 };
 
 // One particle beam attached to a simulation (at most one per simulation).
