@@ -156,9 +156,11 @@ int fdtd_set_pic_lds_rows(fdtd_ctx *ctx, int rows);
  * neighbour is bounded (max_wait_us; 0: 50 ms): a launch that passes the bound
  * because something else holds the device leaves its starting state as it
  * was, and the next call on the context runs its steps again with one launch
- * per S steps.  No counterpart in the reference; it replaces the per-S-steps
- * relaunch of this library's own loop (the `for counts in range(P.timeSteps)`
- * bodies of Solver_Engine.py:167,236,294). */
+ * per S steps.  Where the tiles do not fit (and no simulation records
+ * snapshots), the same tiles run S steps per launch.  No counterpart in the
+ * reference; it replaces the relaunch every S steps of this library's own loop
+ * (the `for counts in range(P.timeSteps)` bodies of
+ * Solver_Engine.py:167,236,294). */
 int fdtd_set_resident(fdtd_ctx *ctx, int on, int64_t max_wait_us);
 /* *active = 1 when the next fdtd_run uses resident launches. */
 int fdtd_resident_active(fdtd_ctx *ctx, int *active);
