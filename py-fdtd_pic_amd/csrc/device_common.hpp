@@ -76,7 +76,9 @@ struct PersistArgs {
 // it has come.  Hand-off q of a launch uses slot q % 3; a tile empties the
 // words of hand-off q - 1 once it has received hand-off q (its readers sent q
 // after they had read q - 1), two blocks before they are written again, and
-// waits for those stores before its next sends.  Launches alternate the sets:
+// waits until those stores are in memory (stores_done) before its next sends: a
+// neighbour that has hand-off q + 1 may poll the slot for q + 2, and must not
+// find q - 1 there.  Launches alternate the sets:
 // each empties what the launch before it left in the other one.
 //
 // A wait of more than max_polls loads of the halo (each goes to memory and

@@ -584,6 +584,13 @@ __device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, cons
 // and go out after the loop, and one chunk of source values needs no
 // rotation.
 constexpr int kResMaxS = 60;
+
+// Every vector store this wave has issued is in memory (and the compiler moves
+// none across).  A release fence at workgroup scope does not say so: on gfx950
+// it waits for LDS alone, since the waves of a workgroup share their L1.  One
+// at agent scope would write back an L2 besides.
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 template <typename R, int K, bool KAHAN, int KIND, int MODE>
 __device__ __forceinline__ void res_steps(TILE_PARAMS, const TileCtx<R>& c, const SimDev<R>& sd,
                                           const SrcChunk<R>& src, R* spare, const int n) {
@@ -667,6 +674,9 @@ __device__ __forceinline__ void res_steps(TILE_PARAMS, const TileCtx<R>& c, cons
         step(s + 1, std::integral_constant<int, 0>{});
     }
     if (s < n) step(s, std::integral_constant<int, 1>{});
+    // the words emptied after the last hand-off, before the next one sends (ResArgs); they are a
+    // block old here, while the probe samples and the snapshot rows to come need no wait
+    stores_done();
     if constexpr (PROBE) {
         // the owning lanes' LDS stores come before the other lanes' reads
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1009,8 +1019,10 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
                     const bool srcs = tile_src || tile_tf, prb = c.npr > 0, ends = srcs || prb;
                     if constexpr (K == 4)      // light tiles: plain cells only
                         res_steps<R, K, KAHAN, KIND, 0>(TILE_ARGS, c, sd, sc, sp, n);
-                    else if (sizeof(R) == 8 && gen)
+                    else if (sizeof(R) == 8 && gen) {
                         run(&sc);
+                        stores_done();
+                    }
                     else if ((pure_slab || emu_tile) && !extras)
                         res_steps<R, K, KAHAN, KIND, M_PURE_SLAB>(TILE_ARGS, c, sd, sc, sp, n);
                     else if (!any_slab && !extras)
@@ -1039,8 +1051,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
             if (k0 >= total || !ra.box) break;      // one block: nothing to hand over
             // ---- hand-off q ----
             unsigned long long* slot = ra.box + q3 * slot_words;
-            // the emptied words of the slot to come are in memory before this block's values go out
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            // (the words emptied after hand-off q - 1 are in memory: the steps end with stores_done)
 #pragma unroll
             for (int j = 0; j < K; ++j) {
                 if (!((send >> j) & 1u)) continue;
