@@ -110,6 +110,16 @@ constexpr unsigned long long kResEmpty = 0x7ff45ea17fb45ea1ull;
 template <typename R>
 constexpr int kResValues = sizeof(R) == 8 ? 7 : 6;   // FP64 E H D P Pm psiE psiH; FP32 pairs E H D P, Pm, psiE|psiH
 
+// First local step k in [k0, kend) of a launch that began at step t0s whose
+// step t0s + k stores a snapshot row (a positive multiple of interval), or
+// kend.  interval may be any positive int: no sum here passes t0s + kend.
+__host__ __device__ inline int snap_step(int t0s, int k0, int kend, int interval) {
+    const int k = t0s + k0 > 0 ? k0 : 1 - t0s;         // step 0 stores none
+    const int past = (t0s + k) % interval;
+    const int wait = past ? interval - past : 0;
+    return k < kend && wait < kend - k ? k + wait : kend;
+}
+
 // Particle beam of one simulation.  Particles are kept sorted by cell
 // (stable), structure of arrays, ping-ponged per step like the fields;
 // start[c] is the first particle of cell c (start[N+1] = np).  Live

@@ -1001,11 +1001,10 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
                 int k1 = kend;
                 bool row = false;
                 if (snap_interval > 0) {
-                    const int t = max(t0s + k0, 1);
-                    const int ts = (t + snap_interval - 1) / snap_interval * snap_interval;
-                    if (ts - t0s < k1) {
-                        k1 = ts - t0s + 1;
-                        row = ts / snap_interval < c.snap_rows;
+                    const int ks = snap_step(t0s, k0, kend, snap_interval);
+                    if (ks < kend) {
+                        k1 = ks + 1;
+                        row = (t0s + ks) / snap_interval < c.snap_rows;
                     }
                 }
                 c.t_first = t0s + k0;

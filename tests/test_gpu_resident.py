@@ -153,3 +153,11 @@ def test_resident_f32_long_runs(slab):
         F = n // 2
         _same([_phys(n, 24001, slab, F=F, R=F + 400 + n % 100, src_cell=100, probes=[60, n - 42],
                      **(dict(chi3=0.0) if slab == "linear" else {}))], "f32", f"long {slab} {n}")
+
+
+@pytest.mark.parametrize("interval", [1, 7, 48, 2 ** 30, 2 ** 31 - 2, 2 ** 31 - 1])
+def test_resident_snapshot_intervals(interval):
+    # up to the largest interval the library takes: no row then but the first, which stays empty
+    spec = _phys(2100, 301, "linear")
+    spec.snap_interval, spec.snap_rows = interval, min(301 // interval + 1, 40)
+    _same([spec], "f64", f"snapshots every {interval}", cuts=(5, 96))
