@@ -768,11 +768,13 @@ struct ResSim {
     bool last_dead;                         // the last cell's fields never change
     std::vector<ResInterval> heavy;         // slab, CPML strips, source, probes
     std::vector<std::pair<int, int>> emu;   // FP32: cells of the one-block tiles that emulate their vacuum cells
+    std::vector<int> probe;                 // FP32: probe cells, ascending (a tile records two of them)
 };
 
 // Tiles of one simulation, in order: light tiles (plain cells, Kl per lane)
 // where their windows meet nothing else, heavy ones (Kh per lane) elsewhere.
-// A tile owns cells of emulating one-block tiles only, or of none.
+// A tile owns cells of emulating one-block tiles only, or of none, and in FP32,
+// which has no general class, at most two probes.
 static int res_tile_sim(const ResSim& q, int Kh, int Kl, int S, int box0, std::vector<int4>* out) {
     const int Uh = 64 * Kh - 2 * S, Ul = 64 * Kl - 2 * S;
     auto kflag = [](int K) { return K == 4 ? kResK4 : K == 2 ? kResK2 : 0; };
@@ -787,18 +789,20 @@ static int res_tile_sim(const ResSim& q, int Kh, int Kl, int S, int box0, std::v
             const int m = v.window ? S : 0;
             if (v.hi > o - m) light_end = std::min(light_end, v.lo - m);
         }
-        int e, flags;
+        int e, flags, third = q.N + 1;
         // light where it covers at least what a heavy tile would
         if (light_end - o >= std::min(Uh, Ul)) {
             e = light_end;
             flags = kResPlain | kflag(Kl);
         } else {
-            e = std::min(o + Uh, stop);
+            const auto p = std::lower_bound(q.probe.begin(), q.probe.end(), o);
+            third = q.probe.end() - p > 2 ? p[2] : q.N + 1;
+            e = std::min({o + Uh, stop, third});
             flags = (q.plain ? kResPlain : 0) | kflag(Kh) | (emu ? kResEmu : 0);
         }
         // the last cell alone is not worth a tile: the window holds it, and
         // beyond it everything is zero
-        if (e == q.N && q.last_dead) e = q.N + 1;
+        if (e == q.N && q.last_dead && third > q.N) e = q.N + 1;
         if (out) out->push_back(make_int4(q.id | flags, o, e, box0));
         ++n;
         o = e;
@@ -853,7 +857,9 @@ static bool res_sim(const fdtd_ctx* c, int i, ResSim& q) {
             int same = 0;
             for (int r = 0; r < d.nprobe; ++r) same += d.probe_cell[r] / U0 == d.probe_cell[p] / U0;
             if (same > 2) return false;
+            q.probe.push_back(d.probe_cell[p]);
         }
+        std::sort(q.probe.begin(), q.probe.end());
         // the one-block tiles whose vacuum cells are emulated (tile_body)
         const int L = 64 * c->K, S0 = c->S_run;
         if (d.slab_kind == SLAB_KERR_E && (float)d.ke0 == (float)d.kD && (float)d.jD == 1.0f)

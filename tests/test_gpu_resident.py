@@ -161,3 +161,40 @@ def test_resident_snapshot_intervals(interval):
     spec = _phys(2100, 301, "linear")
     spec.snap_interval, spec.snap_rows = interval, min(301 // interval + 1, 40)
     _same([spec], "f64", f"snapshots every {interval}", cuts=(5, 96))
+
+
+def _probe_sims(N, tile):
+    """Three probes in adjacent cells, and three a one-block tile apart, around
+    two of the one-block tiles' boundaries."""
+    at = [b + k for b in (900 // tile * tile, 900 // tile * tile + tile) for k in (-3, -2, -1, 0, 1)]
+    sets = [[a, a + 1, a + 2] for a in at] + [[a, a + tile, a + 2 * tile] for a in at]
+    return [_phys(N, 1601, "none" if i % 2 else "kerr", src_cell=860, probes=p) for i, p in enumerate(sets)]
+
+
+@pytest.mark.parametrize("N", [5000, 40000])
+@pytest.mark.parametrize("tiling", [None, (1, 24), (2, 48), (2, 16), (4, 48)])
+def test_resident_f32_records_every_probe(tiling, N):
+    """The resident tiles are cut elsewhere than the one-block tiles, and no
+    FP32 tile of theirs records more than two probes."""
+    K, S = tiling or (4, 32)
+    for spec in _probe_sims(N, 64 * K - 2 * S):
+        on, a = _run([spec], "f32", True, tiling=tiling)
+        off, b = _run([spec], "f32", False, tiling=tiling)
+        cells = [p[0] for p in spec.probes]
+        for k, (x, y) in enumerate(zip(a[0]["probes"], b[0]["probes"])):
+            same, seen = np.array_equal(x, y), np.abs(y).max() > 0
+            assert same and seen, (tiling, on, cells, k)
+
+
+@pytest.mark.parametrize("tiling", [(1, 24), (2, 48), (2, 16)])
+def test_blocks_f32_record_every_probe(tiling):
+    # (three probes in one of the one-block tiles would take the whole batch off the block launches)
+    tile = 64 * tiling[0] - 2 * tiling[1]
+    specs = [_phys(65536, 1601) for _ in range(12)]
+    specs += [s for s in _probe_sims(40000, tile) if len({p[0] // tile for p in s.probes}) > 1]
+    on, a = _run(specs, "f32", True, tiling=tiling)
+    off, b = _run(specs, "f32", False, tiling=tiling)
+    assert not on
+    for spec, x, y in zip(specs, a, b):
+        same = np.array_equal(x["probes"], y["probes"])
+        assert same, (tiling, [p[0] for p in spec.probes])
