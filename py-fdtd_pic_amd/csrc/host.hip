@@ -860,9 +860,10 @@ static bool res_sim(const fdtd_ctx* c, int i, ResSim& q) {
             q.probe.push_back(d.probe_cell[p]);
         }
         std::sort(q.probe.begin(), q.probe.end());
-        // the one-block tiles whose vacuum cells are emulated (tile_body)
+        // the one-block tiles whose vacuum cells are emulated (tile_body; with
+        // snapshots they run the general class, which emulates none)
         const int L = 64 * c->K, S0 = c->S_run;
-        if (d.slab_kind == SLAB_KERR_E && (float)d.ke0 == (float)d.kD && (float)d.jD == 1.0f)
+        if (d.slab_kind == SLAB_KERR_E && d.snap_interval == 0 && (float)d.ke0 == (float)d.kD && (float)d.jD == 1.0f)
             for (int t = std::max(0, (d.F - L) / U0); t * U0 <= d.N && t * U0 - S0 < d.R; ++t) {
                 const int t0 = t * U0 - S0, t1 = t0 + L;
                 if (t1 <= d.F || (t0 >= d.F && t1 <= d.R)) continue;              // no slab, or only slab

@@ -582,7 +582,7 @@ __device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, cons
 // without source or probe has a class of its own, probe rows are written
 // without a branch (lanes that hold no probe write a spare word of their own)
 // and go out after the loop, and one chunk of source values needs no
-// rotation.
+// rotation.  odd: the n steps begin at an odd step of their block (psi_next).
 constexpr int kResMaxS = 60;
 
 // Every vector store this wave has issued is in memory (and the compiler moves
@@ -593,7 +593,7 @@ __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)
 
 template <typename R, int K, bool KAHAN, int KIND, int MODE>
 __device__ __forceinline__ void res_steps(TILE_PARAMS, const TileCtx<R>& c, const SimDev<R>& sd,
-                                          const SrcChunk<R>& src, R* spare, const int n) {
+                                          const SrcChunk<R>& src, R* spare, const int n, const bool odd) {
     constexpr bool SLAB_CODE = (MODE & (M_PURE_SLAB | M_MIXED)) != 0 && KIND >= SLAB_LINEAR;
     constexpr bool STRIP = (MODE & M_STRIP) != 0;
     constexpr bool SRC = (MODE & M_SRC) != 0;
@@ -669,6 +669,9 @@ __device__ __forceinline__ void res_steps(TILE_PARAMS, const TileCtx<R>& c, cons
         }
     };
     int s = 0;
+    // (after an odd cut the first step here is an odd one of its block)
+    if constexpr (STRIP && sizeof(R) == 4)
+        if (odd) step(s++, std::integral_constant<int, 0>{});
     for (; s + 1 < n; s += 2) {
         step(s, std::integral_constant<int, 1>{});
         step(s + 1, std::integral_constant<int, 0>{});
@@ -995,7 +998,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
             // A block is cut at its snapshot steps: the lean loops run up to
             // and including a snapshot step, then the row is stored from
             // registers (t = 0 takes none).
-            const int kend = min(k0 + S, total);
+            const int kbeg = k0, kend = min(k0 + S, total);
             bool fresh = true;
             while (k0 < kend) {
                 int k1 = kend;
@@ -1015,29 +1018,31 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
                     __shared__ R spare_rows[kTileWaves][2][64];
                     R* sp = &spare_rows[wvi][0][0];
                     const int n = c.s_hi;
+                    const bool odd = (k0 - kbeg) & 1;
                     const bool srcs = tile_src || tile_tf, prb = c.npr > 0, ends = srcs || prb;
                     if constexpr (K == 4)      // light tiles: plain cells only
-                        res_steps<R, K, KAHAN, KIND, 0>(TILE_ARGS, c, sd, sc, sp, n);
+                        res_steps<R, K, KAHAN, KIND, 0>(TILE_ARGS, c, sd, sc, sp, n, odd);
                     else if (sizeof(R) == 8 && gen) {
                         run(&sc);
                         stores_done();
                     }
                     else if ((pure_slab || emu_tile) && !extras)
-                        res_steps<R, K, KAHAN, KIND, M_PURE_SLAB>(TILE_ARGS, c, sd, sc, sp, n);
+                        res_steps<R, K, KAHAN, KIND, M_PURE_SLAB>(TILE_ARGS, c, sd, sc, sp, n, odd);
                     else if (!any_slab && !extras)
-                        res_steps<R, K, KAHAN, KIND, 0>(TILE_ARGS, c, sd, sc, sp, n);
+                        res_steps<R, K, KAHAN, KIND, 0>(TILE_ARGS, c, sd, sc, sp, n, odd);
                     else if (!any_slab && !ends)
-                        res_steps<R, K, KAHAN, KIND, M_STRIP>(TILE_ARGS, c, sd, sc, sp, n);
+                        res_steps<R, K, KAHAN, KIND, M_STRIP>(TILE_ARGS, c, sd, sc, sp, n, odd);
                     else if (!any_slab && !prb)
-                        res_steps<R, K, KAHAN, KIND, M_STRIP | M_SRC>(TILE_ARGS, c, sd, sc, sp, n);
+                        res_steps<R, K, KAHAN, KIND, M_STRIP | M_SRC>(TILE_ARGS, c, sd, sc, sp, n, odd);
                     else if (!any_slab && !srcs)
-                        res_steps<R, K, KAHAN, KIND, M_STRIP | M_PROBE>(TILE_ARGS, c, sd, sc, sp, n);
+                        res_steps<R, K, KAHAN, KIND, M_STRIP | M_PROBE>(TILE_ARGS, c, sd, sc, sp, n, odd);
                     else if (!any_slab)
-                        res_steps<R, K, KAHAN, KIND, M_STRIP | M_SRC | M_PROBE>(TILE_ARGS, c, sd, sc, sp, n);
+                        res_steps<R, K, KAHAN, KIND, M_STRIP | M_SRC | M_PROBE>(TILE_ARGS, c, sd, sc, sp, n, odd);
                     else if (!ends)
-                        res_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP>(TILE_ARGS, c, sd, sc, sp, n);
+                        res_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP>(TILE_ARGS, c, sd, sc, sp, n, odd);
                     else
-                        res_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP | M_SRC | M_PROBE>(TILE_ARGS, c, sd, sc, sp, n);
+                        res_steps<R, K, KAHAN, KIND, M_MIXED | M_STRIP | M_SRC | M_PROBE>(TILE_ARGS, c, sd, sc, sp, n,
+                                                                                          odd);
                 }
                 if (row) {
                     R* o = c.snap + (long long)((t0s + k1 - 1) / snap_interval) * (N + 1) + c.base;

@@ -198,3 +198,26 @@ def test_blocks_f32_record_every_probe(tiling):
     for spec, x, y in zip(specs, a, b):
         same = np.array_equal(x["probes"], y["probes"])
         assert same, (tiling, [p[0] for p in spec.probes])
+
+
+@pytest.mark.parametrize("slab,tiling", [("kerr", None), ("linear", None), ("none", None), ("kerr", (2, 48)),
+                                         ("kerr", (2, 16)), ("kerr", (1, 24))])
+@pytest.mark.parametrize("interval", [1, 7, 13, 48, 50, 1000])
+def test_resident_f32_snapshots(slab, tiling, interval):
+    """A snapshot step cuts a block, and FP32 rounding depends on a step's place
+    in its block and on the class that a one-block tile with snapshots runs."""
+    specs = []
+    for n, kw in ((5003, {}), (2100, {}), (25013, dict(src_cell=4000))):
+        s = _phys(n, 611, slab, **kw)
+        s.snap_interval, s.snap_rows = interval, min(611 // interval + 1, 40)
+        specs.append(s)
+    _same(specs, "f32", f"snapshots every {interval}, {slab} {tiling}", cuts=(5, 96), tiling=tiling)
+
+
+@pytest.mark.parametrize("interval", [2000, 2001])
+def test_resident_f32_snapshots_long(interval):
+    for n in (25013, 24007, 23011, 9001, 5003):
+        F = n // 2
+        s = _phys(n, 24001, "kerr", F=F, R=F + 400 + n % 100, src_cell=100, probes=[60, n - 42])
+        s.snap_interval, s.snap_rows = interval, 13
+        _same([s], "f32", f"long, snapshots every {interval}, {n}")
