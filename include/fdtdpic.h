@@ -164,6 +164,14 @@ int fdtd_set_pic_lds_rows(fdtd_ctx *ctx, int rows);
 int fdtd_set_resident(fdtd_ctx *ctx, int on, int64_t max_wait_us);
 /* *active = 1 when the next fdtd_run uses resident launches. */
 int fdtd_resident_active(fdtd_ctx *ctx, int *active);
+/* What became of the context's resident launches so far: launches queued,
+ * launches whose steps were run again after a give-up, and launches not yet
+ * known to have finished.  Any pointer may be NULL. */
+int fdtd_resident_counts(fdtd_ctx *ctx, int64_t *launches, int64_t *again, int64_t *queued);
+/* Takes the nth resident launch from now on (1: the next; 0: none) for one
+ * that gave up: the device leaves it, and those behind it, undone, and their
+ * steps are run again.  For tests of that path. */
+int fdtd_resident_fail(fdtd_ctx *ctx, int nth);
 /* Request for persistent launches (on = 1) under the conditions of uniform
  * tiles with S <= 64K - 2S, one slab kind and no beam: fdtd_persistent_active
  * tells whether the next fdtd_run keeps its tiles on the device between

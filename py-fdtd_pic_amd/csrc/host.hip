@@ -329,6 +329,7 @@ static int resolve_resident(fdtd_ctx* c) {
         c->sims[x.id]->launches = x.launches;
     }
     c->dirty = true;
+    c->res_again += (long long)(pend.size() - k);
     long long again = 0;
     for (; k < pend.size(); ++k) again += pend[k].nsteps;
     return run_steps_host(c, again, false);
@@ -1382,6 +1383,11 @@ static int run_resident_t(fdtd_ctx* c, int64_t n, bool* taken) {
     ra.err = c->d_rerr;
     ra.herr = c->h_rerr;
     ra.max_polls = c->res_polls;
+    if (c->res_fail > 0 && --c->res_fail == 0) {
+        // the flags as the kernel leaves them; the launch finds its own ordinal and returns at once
+        HIPCHK(hipMemsetD32Async((hipDeviceptr_t)c->d_rerr, ra.ordinal, 1, c->st));
+        __atomic_store_n(c->h_rerr, ra.ordinal, __ATOMIC_RELEASE);
+    }
     EvPair* ev = nullptr;
     const int blocks = (int)((n + c->S_run - 1) / c->S_run);
     if (c->profile > 0) {
@@ -1802,6 +1808,21 @@ int fdtd_resident_active(fdtd_ctx* c, int* active) {
         if (rc) return rc;
     }
     *active = c->res_ok ? 1 : 0;
+    return FDTD_OK;
+}
+
+int fdtd_resident_counts(fdtd_ctx* c, int64_t* launches, int64_t* again, int64_t* queued) {
+    if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
+    if (launches) *launches = c->res_ordinal;
+    if (again) *again = c->res_again;
+    if (queued) *queued = (int64_t)c->res_pending.size();
+    return FDTD_OK;
+}
+
+int fdtd_resident_fail(fdtd_ctx* c, int nth) {
+    if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
+    if (nth < 0) return fdtd_fail(FDTD_E_ARG, "nth must be 0 (none) or more");
+    c->res_fail = nth;
     return FDTD_OK;
 }
 

@@ -148,6 +148,8 @@ struct fdtd_ctx {
     int res_ordinal = 0;
     std::vector<ResPending> res_pending;     // resident launches not yet known to have finished
     hipEvent_t res_ev = nullptr;             // recorded after the last resident launch
+    long long res_again = 0;                 // launches that gave up or were queued behind one that did
+    int res_fail = 0;                        // fdtd_resident_fail: launches until one is taken for a give-up
     int cu_count = 0;
     int lds_max = 0;            // shared memory a workgroup may use (bytes; 0: unknown)
     int pc_rows = 0;            // forced LDS rows per cell of the one-cell PIC kernel (0: chosen per launch)

@@ -73,6 +73,8 @@ SIGNATURES = {
     "fdtd_persistent_active": (C.c_int, [_vp, C.POINTER(C.c_int)]),
     "fdtd_set_resident": (C.c_int, [_vp, C.c_int, C.c_int64]),
     "fdtd_resident_active": (C.c_int, [_vp, C.POINTER(C.c_int)]),
+    "fdtd_resident_counts": (C.c_int, [_vp, C.POINTER(C.c_int64), C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
+    "fdtd_resident_fail": (C.c_int, [_vp, C.c_int]),
     "fdtd_set_halo_exchange": (C.c_int, [_vp, C.c_int]),
     "fdtd_halo_exchange_active": (C.c_int, [_vp, C.POINTER(C.c_int)]),
     "fdtd_add_sim": (C.c_int, [_vp, C.POINTER(SimDesc), C.POINTER(C.c_int)]),

@@ -230,6 +230,18 @@ class Context:
         check(self.lib.fdtd_resident_active(self.h, C.byref(v)))
         return bool(v.value)
 
+    def resident_counts(self):
+        """(queued so far, run again after a give-up, not yet known to have
+        finished) of the resident launches."""
+        v = [C.c_int64() for _ in range(3)]
+        check(self.lib.fdtd_resident_counts(self.h, *[C.byref(x) for x in v]))
+        return tuple(x.value for x in v)
+
+    def resident_fail(self, nth=1):
+        """Take the nth resident launch from now on for one that gave up
+        (0: none); for tests of that path."""
+        check(self.lib.fdtd_resident_fail(self.h, int(nth)))
+
     def set_halo_exchange(self, h=8):
         """Workgroup halo exchange every h steps between the four adjacent
         windows of a field workgroup (0: off); declined where it does not apply."""

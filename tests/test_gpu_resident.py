@@ -221,3 +221,44 @@ def test_resident_f32_snapshots_long(interval):
         s = _phys(n, 24001, "kerr", F=F, R=F + 400 + n % 100, src_cell=100, probes=[60, n - 42])
         s.snap_interval, s.snap_rows = interval, 13
         _same([s], "f32", f"long, snapshots every {interval}, {n}")
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("nth", [1, 2, 3])
+def test_resident_give_up_is_run_again(prec, nth):
+    """A give-up forced from the host, in the first, a middle and the last of
+    three launches: that one and those behind it are run again, once."""
+    from fdtd_pic_amd import engine
+    specs = [_phys(9000, 900), _phys(2000, 333, "none")]
+    S = 16
+    with engine.Context(prec) as c:
+        c.set_tiling(2, S)
+        sims = [c.add(s) for s in specs]
+        assert c.resident_active() and c.resident_counts() == (0, 0, 0)
+        c.resident_fail(nth)
+        for n in (6 * S, 2 * S, 5 * S):
+            c.run(n)
+        assert c.resident_counts() == (3, 0, 3)
+        got = [{f: s.read(f) for f in ("E", "H", "PSIE", "PSIH")} | {"probes": s.probes()} for s in sims]
+        assert c.resident_counts() == (3, 4 - nth, 0)
+    with engine.Context(prec) as c:
+        c.set_tiling(2, S)
+        c.set_resident(False)
+        sims = [c.add(s) for s in specs]
+        c.run(13 * S)
+        for s, g in zip(sims, got):
+            for f in g:
+                assert np.array_equal(g[f], s.probes() if f == "probes" else s.read(f)), f
+
+
+def test_resident_errors():
+    from fdtd_pic_amd import _capi, engine
+    with engine.Context("f64") as c:
+        for on, wait in ((2, 0), (-1, 0), (1, -1), (1, 60000001)):
+            with pytest.raises(_capi.FdtdError):
+                _capi.check(c.lib.fdtd_set_resident(c.h, on, wait))
+        with pytest.raises(_capi.FdtdError):
+            c.resident_fail(-1)
+        assert c.lib.fdtd_set_resident(None, 1, 0) and c.lib.fdtd_resident_fail(None, 1)
+        assert c.lib.fdtd_resident_active(None, None) and c.lib.fdtd_resident_counts(None, None, None, None)
+        assert c.lib.fdtd_resident_counts(c.h, None, None, None) == 0
