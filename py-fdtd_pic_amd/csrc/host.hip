@@ -307,7 +307,8 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident);
 // Waits for the queued resident launches and, if one gave up (a neighbour
 // wait passed its bound: its tiles were not all resident), takes the counters
 // back to where it began and runs its steps, and those of the launches behind
-// it, which returned at once, with one-block launches.
+// it, which returned at once, with one-block launches.  A simulation that was
+// added behind them stays out of those, and begins where the counters then are.
 static int resolve_resident(fdtd_ctx* c) {
     if (c->res_pending.empty()) return FDTD_OK;
     HIPCHK(hipStreamSynchronize(c->st));
@@ -328,11 +329,22 @@ static int resolve_resident(fdtd_ctx* c) {
         c->sims[x.id]->steps_done = x.steps_done;
         c->sims[x.id]->launches = x.launches;
     }
+    std::vector<SimHost*> late;
+    for (SimHost* s : c->sims)
+        if (s && s->t_begin > c->gstep) late.push_back(s);
+    for (SimHost* s : late) s->held = true;
     c->dirty = true;
     c->res_again += (long long)(pend.size() - k);
     long long again = 0;
     for (; k < pend.size(); ++k) again += pend[k].nsteps;
-    return run_steps_host(c, again, false);
+    const int rc = run_steps_host(c, again, false);
+    for (SimHost* s : late) {
+        s->held = false;
+        s->launch_begin = c->launch_idx;
+        s->t_begin = c->gstep;
+    }
+    if (!late.empty()) c->dirty = true;
+    return rc;
 }
 
 // Everything queued on the context's stream has finished.
@@ -427,6 +439,7 @@ int fdtd_set_tiling_mixed(fdtd_ctx* c, int K, int K_slab, int S) {
     if (S < 1 || S > 255 || 64 * K_slab - 2 - S < 1)
         return fdtd_fail(FDTD_E_ARG, "S must satisfy 1 <= S <= min(255, 64*K_slab-3)");
     if ((int64_t)c->sims.size() >= (1 << 24)) return fdtd_fail(FDTD_E_ARG, "too many simulations");
+    if (int rc = resolve_resident(c)) return rc;      // FP32: steps that are run again keep their tiling
     c->K = K; c->K_slab = K_slab; c->S = S; c->dirty = true;
     return FDTD_OK;
 }
@@ -1048,7 +1061,8 @@ static int rebuild_t(fdtd_ctx* c) {
     // a coupled beam forces one step per launch: tiles then carry a 1-cell halo
     bool pic = false;
     for (int i = 0; i < nsim; ++i)
-        if (c->sims[i] && c->sims[i]->steps_done < c->sims[i]->d.steps && i < (int)c->beams.size() && c->beams[i])
+        if (c->sims[i] && !c->sims[i]->held && c->sims[i]->steps_done < c->sims[i]->d.steps &&
+            i < (int)c->beams.size() && c->beams[i])
             pic = true;
     c->S_run = pic ? 1 : c->S;
     const int U = 64 * c->K - 2 * c->S_run;              // plain tiles
@@ -1074,7 +1088,7 @@ static int rebuild_t(fdtd_ctx* c) {
             devs[i].pS = (const double*)(bb + bh.off[BO_S]);
             for (int k = 0; k < 2; ++k) devs[i].prange[k] = (const int32_t*)(bb + bh.off[BO_RANGE + k]);
         }
-        if (s->steps_done >= s->d.steps) continue;
+        if (s->held || s->steps_done >= s->d.steps) continue;
         c->tile_sims.push_back(i);
     }
     // resident launches, or blocks with the same tiles, which need no other list
@@ -1767,6 +1781,7 @@ int fdtd_read_energy(fdtd_ctx* c, int id, double* values, int64_t* steps, int64_
 int fdtd_set_persistent(fdtd_ctx* c, int on) {
     if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
     if (on != 0 && on != 1) return fdtd_fail(FDTD_E_ARG, "persistent flag must be 0 or 1");
+    if (int rc = resolve_resident(c)) return rc;
     c->persist = on != 0;
     c->dirty = true;
     return FDTD_OK;
@@ -1837,6 +1852,7 @@ int fdtd_set_pic_lds_rows(fdtd_ctx* c, int rows) {
 int fdtd_set_halo_exchange(fdtd_ctx* c, int h) {
     if (!c) return fdtd_fail(FDTD_E_ARG, "null ctx");
     if (h < 0 || h > 32) return fdtd_fail(FDTD_E_ARG, "halo exchange period must be 0 (off) .. 32");
+    if (int rc = resolve_resident(c)) return rc;
     c->halo = h;
     c->dirty = true;
     return FDTD_OK;

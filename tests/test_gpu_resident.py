@@ -262,3 +262,83 @@ def test_resident_errors():
         assert c.lib.fdtd_set_resident(None, 1, 0) and c.lib.fdtd_resident_fail(None, 1)
         assert c.lib.fdtd_resident_active(None, None) and c.lib.fdtd_resident_counts(None, None, None, None)
         assert c.lib.fdtd_resident_counts(c.h, None, None, None) == 0
+
+
+def _beam_spec(N, steps):
+    from fdtd_pic_amd import configs, engine
+    rng = np.random.default_rng(N)
+    spec = engine.physical_spec(configs.base(N, steps, slab_start=60, slab_stop=90, src_cell=200, probes=[150, N - 60],
+                                             src_t0=5e-15, src_tau=2e-15, src_amp=1e6))
+    return spec, engine.Beam(300 + rng.uniform(0.0, 80, 2000), rng.normal(0.0, 0.15, (2000, 3)), -configs.E_CHARGE,
+                             configs.M_ELECTRON, 1e9, configs.DT, configs.DZ)
+
+
+def _play(prec, resident, script, fail=0):
+    """Runs the script's calls on one context: ("run", n), ("add", spec),
+    ("beam", spec, beam), ("write", sim), ("reset", sim), ("tiling", K, S),
+    ("halo", h), ("read",).  The state of every simulation at the end, and the
+    launches run again."""
+    from fdtd_pic_amd import engine
+    with engine.Context(prec) as c:
+        c.set_tiling(2, 16)
+        c.set_resident(resident)
+        if resident:
+            c.resident_fail(fail)
+        sims, out = [], []
+        for what, *a in script + [("read",)]:
+            if what == "run":
+                c.run(a[0])
+            elif what == "add":
+                sims.append(c.add(a[0]))
+            elif what == "beam":
+                sims.append(c.add(a[0], beam=a[1]))
+            elif what == "write":
+                x = np.arange(sims[a[0]].spec.N + 1)
+                sims[a[0]].write("E", 1e6 * np.exp(-((x - 300.0) / 40.0) ** 2))
+            elif what == "reset":
+                sims[a[0]].reset()
+            elif what == "tiling":
+                c.set_tiling(*a)
+            elif what == "halo":
+                c.set_halo_exchange(*a)
+            else:
+                for s in sims:
+                    out.append({f: s.read(f) for f in ("E", "H", "PSIE", "PSIH") + (("D", "P") if s.spec.R > s.spec.F
+                                                                                   else ())})
+                    out[-1]["probes"], out[-1]["progress"] = s.probes(), s.progress()
+                    if s.beam_n:
+                        out[-1]["x"], out[-1]["u"], _ = s.particles()
+        return out, c.resident_counts()[1]
+
+
+def _plays_the_same(prec, script, fail=1, again=None):
+    got, n = _play(prec, True, script, fail)
+    want, _ = _play(prec, False, script)
+    assert n > 0 if again is None else n == again
+    for k, (x, y) in enumerate(zip(got, want)):
+        assert np.abs(y["E"]).max() > 0 or y["progress"] == 0
+        for f in y:
+            same = np.array_equal(x[f], y[f])
+            assert same, (k, f)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("kind", ["add", "add and read", "write", "two", "beam", "beam, no run"])
+def test_simulation_added_behind_a_launch_that_gives_up(prec, kind):
+    """A simulation that is added while a resident launch is under way has no
+    part in that launch's steps, also where they are run again."""
+    a, b = ("add", _phys(5000, 500)), ("add", _phys(3000, 400, "none"))
+    beam = ("beam", *_beam_spec(700, 200))
+    run = ("run", 96)
+    _plays_the_same(prec, {"add": [a, run, b, run], "add and read": [a, run, b, ("read",), run, ("read",), run],
+                           "write": [a, run, b, ("write", 1), run, run],
+                           "two": [a, run, b, ("add", _phys(801, 300)), run, run],
+                           "beam": [a, run, beam, ("run", 32), ("read",), ("run", 7)],
+                           "beam, no run": [a, run, beam]}[kind])
+
+
+@pytest.mark.parametrize("change", [("tiling", 1, 24), ("tiling", 4, 32), ("tiling", 2, 32), ("halo", 8)])
+def test_tiling_changed_behind_a_launch_that_gives_up(change):
+    # FP32 rounding depends on the tiling: the steps before the change keep the old one
+    a = ("add", _phys(5000, 500))
+    _plays_the_same("f32", [a, ("run", 96), change, ("run", 96)])
