@@ -307,7 +307,8 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident);
 // Waits for the queued resident launches and, if one gave up (a neighbour
 // wait passed its bound: its tiles were not all resident), takes the counters
 // back to where it began and runs its steps, and those of the launches behind
-// it, which returned at once, with one-block launches.  A simulation that was
+// it, which returned at once, with one-block launches: one launch's after the
+// other, since FP32 rounding depends on where a block begins.  A simulation that was
 // added behind them stays out of those, and begins where the counters then are.
 static int resolve_resident(fdtd_ctx* c) {
     if (c->res_pending.empty()) return FDTD_OK;
@@ -335,9 +336,8 @@ static int resolve_resident(fdtd_ctx* c) {
     for (SimHost* s : late) s->held = true;
     c->dirty = true;
     c->res_again += (long long)(pend.size() - k);
-    long long again = 0;
-    for (; k < pend.size(); ++k) again += pend[k].nsteps;
-    const int rc = run_steps_host(c, again, false);
+    int rc = FDTD_OK;
+    for (; k < pend.size() && rc == FDTD_OK; ++k) rc = run_steps_host(c, pend[k].nsteps, false);
     for (SimHost* s : late) {
         s->held = false;
         s->launch_begin = c->launch_idx;
@@ -1454,7 +1454,8 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
         }
         if (c->ntiles == 0) break;
         if (c->res_ok && allow_resident) {
-            const int64_t n = std::min<int64_t>(remaining, kResMaxSteps);
+            // whole blocks of the one-block launches, unless the run ends
+            const int64_t n = std::min<int64_t>(remaining, kResMaxSteps / c->S_run * c->S_run);
             int rc = close_bracket(c);
             if (rc) return rc;
             bool taken = false;

@@ -342,3 +342,20 @@ def test_tiling_changed_behind_a_launch_that_gives_up(change):
     # FP32 rounding depends on the tiling: the steps before the change keep the old one
     a = ("add", _phys(5000, 500))
     _plays_the_same("f32", [a, ("run", 96), change, ("run", 96)])
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("cuts", [(5, 192), (37, 1, 192, 23), (96, 21, 17)])
+def test_runs_keep_their_pieces_when_run_again(prec, cuts):
+    """Several queued runs, none a whole number of blocks: FP32 rounding depends
+    on where a block begins."""
+    a, b = ("add", _phys(5000, 900)), ("add", _phys(3000, 400, "none"))
+    _plays_the_same(prec, [a, b] + [("run", n) for n in cuts], again=len(cuts))
+
+
+@pytest.mark.parametrize("tiling", [(2, 21), (4, 48)])
+def test_resident_f32_very_long_run(tiling):
+    # more steps than one launch takes: the cut falls between blocks
+    spec = _phys(700, (1 << 20) + 300, "none", probes=[200])
+    spec.srcE = 1e8 * np.sin(0.3 * np.arange(spec.steps))
+    _same([spec], "f32", f"1,048,876 steps at {tiling}", tiling=tiling)
