@@ -1878,8 +1878,10 @@ int fdtd_busy(fdtd_ctx* c, int* busy) {
     const hipError_t e = hipStreamQuery(c->st);
     if (e == hipErrorNotReady) { *busy = 1; return FDTD_OK; }
     if (e != hipSuccess) return fdtd_fail(FDTD_E_HIP, std::string("hipStreamQuery: ") + hipGetErrorString(e));
-    *busy = 0;
-    return resolve_resident(c);
+    const long long again = c->res_again;
+    if (int rc = resolve_resident(c)) return rc;
+    *busy = c->res_again != again;       // a launch gave up: its steps are queued again
+    return FDTD_OK;
 }
 
 int fdtd_kernel_timing(fdtd_ctx* c, int kind, double* ms, int64_t* launches) {

@@ -359,3 +359,17 @@ def test_resident_f32_very_long_run(tiling):
     spec = _phys(700, (1 << 20) + 300, "none", probes=[200])
     spec.srcE = 1e8 * np.sin(0.3 * np.arange(spec.steps))
     _same([spec], "f32", f"1,048,876 steps at {tiling}", tiling=tiling)
+
+
+def test_busy_behind_a_give_up():
+    # steps that are queued again are work: no "idle" before they have run
+    from fdtd_pic_amd import engine
+    with engine.Context("f64") as c:
+        c.add(_phys(65536, 20000))
+        c.resident_fail(1)
+        c.run_all()
+        seen = []
+        while len(seen) < 200 or seen[-1]:
+            seen.append(c.busy())
+        assert True in seen and seen == sorted(seen, reverse=True)
+        assert c.resident_counts() == (1, 1, 0)
