@@ -156,7 +156,8 @@ int fdtd_set_pic_lds_rows(fdtd_ctx *ctx, int rows);
  * neighbour is bounded (max_wait_us; 0: 50 ms): a launch that passes the bound
  * because something else holds the device leaves its starting state as it
  * was, and the next call on the context runs its steps again with one launch
- * per S steps.  Where the tiles do not fit (and no simulation records
+ * per S steps; so do the runs of the second after it (doubled, up to 64 s,
+ * with each give-up in a row).  Where the tiles do not fit (and no simulation records
  * snapshots), the same tiles run S steps per launch.  No counterpart in the
  * reference; it replaces the relaunch every S steps of this library's own loop
  * (the `for counts in range(P.timeSteps)` bodies of

@@ -304,6 +304,11 @@ static void res_release(fdtd_ctx* c) {
 
 static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident);
 
+// The plan is resident, and no give-up is so recent that none is tried.
+static bool res_now(const fdtd_ctx* c) {
+    return c->res_ok && (c->res_strikes == 0 || std::chrono::steady_clock::now() >= c->res_after);
+}
+
 // Waits for the queued resident launches and, if one gave up (a neighbour
 // wait passed its bound: its tiles were not all resident), takes the counters
 // back to where it began and runs its steps, and those of the launches behind
@@ -317,8 +322,14 @@ static int resolve_resident(fdtd_ctx* c) {
     std::vector<ResPending> pend;
     pend.swap(c->res_pending);
     const int32_t bad = __atomic_load_n(c->h_rerr, __ATOMIC_ACQUIRE);
-    if (bad == 0) return FDTD_OK;
+    if (bad == 0) {
+        c->res_strikes = 0;
+        return FDTD_OK;
+    }
     __atomic_store_n(c->h_rerr, 0, __ATOMIC_RELEASE);
+    c->res_after = std::chrono::steady_clock::now() +
+                   std::chrono::seconds(std::min(kResPauseS << std::min(c->res_strikes, 16), kResPauseMostS));
+    c->res_strikes++;
     HIPCHK(hipMemsetAsync(c->d_rerr, 0, sizeof(int32_t), c->st));
     c->box_stale = true;
     size_t k = 0;
@@ -1453,7 +1464,7 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
             if (rc) return rc;
         }
         if (c->ntiles == 0) break;
-        if (c->res_ok && allow_resident) {
+        if (allow_resident && res_now(c)) {
             // whole blocks of the one-block launches, unless the run ends
             const int64_t n = std::min<int64_t>(remaining, kResMaxSteps / c->S_run * c->S_run);
             int rc = close_bracket(c);
@@ -1798,7 +1809,7 @@ int fdtd_persistent_active(fdtd_ctx* c, int* active) {
         rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
         if (rc) return rc;
     }
-    *active = c->persist_ok ? 1 : 0;
+    *active = c->persist_ok && res_now(c) ? 1 : 0;
     return FDTD_OK;
 }
 
@@ -1808,6 +1819,7 @@ int fdtd_set_resident(fdtd_ctx* c, int on, int64_t max_wait_us) {
         return fdtd_fail(FDTD_E_ARG, "resident flag must be 0 or 1, the wait 0 (default) .. 60 s");
     if (int rc = resolve_resident(c)) return rc;
     c->res_mode = on;
+    c->res_strikes = 0;
     c->res_polls = max_wait_us > 0 ? (int)(2 * max_wait_us) : kResMaxPolls;
     c->dirty = true;
     return FDTD_OK;
@@ -1823,7 +1835,7 @@ int fdtd_resident_active(fdtd_ctx* c, int* active) {
         rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
         if (rc) return rc;
     }
-    *active = c->res_ok ? 1 : 0;
+    *active = res_now(c) ? 1 : 0;
     return FDTD_OK;
 }
 

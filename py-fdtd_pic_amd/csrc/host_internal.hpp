@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <string>
 #include <cstdint>
 #include <utility>
@@ -77,6 +78,11 @@ struct ResPending {
 constexpr int kResMaxPolls = 100000;
 constexpr long long kResMaxSteps = 1 << 20;
 
+// Pause after a give-up, doubled with each one in a row: what holds the device
+// (another process, say) would let every run wait for its bound and then run
+// its steps again.
+constexpr int kResPauseS = 1, kResPauseMostS = 64;
+
 struct fdtd_ctx {
     int prec = FDTD_F64;
     int device = 0;                          // HIP device current at fdtd_ctx_create
@@ -150,6 +156,8 @@ struct fdtd_ctx {
     std::vector<ResPending> res_pending;     // resident launches not yet known to have finished
     hipEvent_t res_ev = nullptr;             // recorded after the last resident launch
     long long res_again = 0;                 // launches that gave up or were queued behind one that did
+    int res_strikes = 0;                     // give-ups since a resident launch last finished
+    std::chrono::steady_clock::time_point res_after;   // none is tried before, after a give-up
     int res_fail = 0;                        // fdtd_resident_fail: launches until one is taken for a give-up
     int cu_count = 0;
     int lds_max = 0;            // shared memory a workgroup may use (bytes; 0: unknown)

@@ -373,3 +373,36 @@ def test_busy_behind_a_give_up():
             seen.append(c.busy())
         assert True in seen and seen == sorted(seen, reverse=True)
         assert c.resident_counts() == (1, 1, 0)
+
+
+def test_resident_pauses_after_a_give_up():
+    """Something else holds the device: the runs after a give-up do not each
+    wait for their bound again, until a second has passed."""
+    import time
+    from fdtd_pic_amd import engine
+    with engine.Context("f64") as c:
+        c.add(_phys(5000, 2000))
+        c.resident_fail(1)
+        for _ in range(5):
+            c.run(100)
+            c.sync()
+        assert c.resident_counts() == (1, 1, 0) and not c.resident_active()
+        time.sleep(1.1)
+        assert c.resident_active()
+        c.resident_fail(1)
+        for _ in range(3):
+            c.run(100)
+            c.sync()
+        time.sleep(1.1)                       # the second time it is two
+        assert c.resident_counts() == (2, 2, 0) and not c.resident_active()
+        time.sleep(1.0)
+        for _ in range(3):
+            c.run(100)
+            c.sync()
+        assert c.resident_counts() == (5, 2, 0)
+        c.resident_fail(1)
+        c.run(100)
+        c.sync()
+        assert not c.resident_active()
+        c.set_resident(True)                  # asked for: at once
+        assert c.resident_active()
