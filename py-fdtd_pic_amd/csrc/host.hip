@@ -1474,6 +1474,16 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
             if (rc) return rc;
             if (taken) {
                 remaining -= n;
+                rc = throttle(c);
+                if (rc) return rc;
+                if (c->res_pending.size() >= kResMostQueued) {
+                    // all but the last kThrottleEvery * (kThrottleDepth + 1) have finished
+                    std::vector<ResPending>& q = c->res_pending;
+                    if (__atomic_load_n(c->h_rerr, __ATOMIC_ACQUIRE) == 0)
+                        q.erase(q.begin(), q.end() - kThrottleEvery * (kThrottleDepth + 1));
+                    else if ((rc = resolve_resident(c)))
+                        return rc;
+                }
                 continue;
             }
         }

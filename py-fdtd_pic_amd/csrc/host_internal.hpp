@@ -192,6 +192,9 @@ constexpr int kFuseMaxTiles = 8192;
 
 constexpr int kThrottleEvery = 128;
 constexpr size_t kThrottleDepth = 4;
+// Resident launches that the host keeps track of before it forgets those that
+// the throttle has seen finish.
+constexpr size_t kResMostQueued = 2 * kThrottleEvery * kThrottleDepth;
 
 // Default steps per launch for K cells per lane: the tile keeps 75% of its
 // cells as output (U = 64K - 2S = 48K).

@@ -406,3 +406,28 @@ def test_resident_pauses_after_a_give_up():
         assert not c.resident_active()
         c.set_resident(True)                  # asked for: at once
         assert c.resident_active()
+
+
+@pytest.mark.parametrize("fail", [0, 1, 700, 2900])
+def test_resident_queue_is_bounded(fail):
+    """A loop of single steps: the host keeps track of so many launches only,
+    and of the right ones when one of them gives up."""
+    from fdtd_pic_amd import engine
+    spec = _phys(2000, 3000)
+    with engine.Context("f64") as c:
+        s = c.add(spec)
+        c.resident_fail(fail)
+        most = 0
+        for _ in range(3000):
+            c.run(1)
+            most = max(most, c.resident_counts()[2])
+        got = {f: s.read(f) for f in ("E", "H", "D", "P")} | {"probes": s.probes()}
+        assert s.progress() == 3000 and (c.resident_counts()[1] > 0) == (fail > 0)
+    assert most <= 1024
+    with engine.Context("f64") as c:
+        c.set_resident(False)
+        s = c.add(spec)
+        c.run_all()
+        for f in got:
+            same = np.array_equal(got[f], s.probes() if f == "probes" else s.read(f))
+            assert same, f
