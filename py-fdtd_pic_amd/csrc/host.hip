@@ -313,8 +313,9 @@ static bool res_now(const fdtd_ctx* c) {
 // wait passed its bound: its tiles were not all resident), takes the counters
 // back to where it began and runs its steps, and those of the launches behind
 // it, which returned at once, with one-block launches: one launch's after the
-// other, since FP32 rounding depends on where a block begins.  A simulation that was
-// added behind them stays out of those, and begins where the counters then are.
+// other, since FP32 rounding depends on where a block begins.  A simulation
+// whose life (since it was added or reset) began behind the failed launch
+// comes in at the launch before which it began, or after all of them.
 static int resolve_resident(fdtd_ctx* c) {
     if (c->res_pending.empty()) return FDTD_OK;
     HIPCHK(hipStreamSynchronize(c->st));
@@ -337,24 +338,36 @@ static int resolve_resident(fdtd_ctx* c) {
     if (k == pend.size()) return fdtd_fail(FDTD_E_STATE, "resident launch: unknown ordinal in the give-up flag");
     c->launch_idx = pend[k].launch_idx;
     c->gstep = pend[k].gstep;
-    for (const ResPending::Sim& x : pend[k].sims) {
-        c->sims[x.id]->steps_done = x.steps_done;
-        c->sims[x.id]->launches = x.launches;
-    }
+    c->dirty = true;
+    c->res_again += (long long)(pend.size() - k);
+    // the counters before each simulation's first launch of these
+    for (size_t j = pend.size(); j-- > k;)
+        for (const ResPending::Sim& x : pend[j].sims) {
+            SimHost* s = c->sims[x.id];
+            if (!s || s->t_begin > pend[j].gstep) continue;      // a former life
+            s->steps_done = x.steps_done;
+            s->launches = x.launches;
+        }
     std::vector<SimHost*> late;
     for (SimHost* s : c->sims)
         if (s && s->t_begin > c->gstep) late.push_back(s);
     for (SimHost* s : late) s->held = true;
-    c->dirty = true;
-    c->res_again += (long long)(pend.size() - k);
+    auto begin_now = [&](long long gstep) {       // those whose life began at this step or before
+        const auto rest = std::partition(late.begin(), late.end(), [&](SimHost* s) { return s->t_begin > gstep; });
+        for (auto it = rest; it != late.end(); ++it) {
+            (*it)->held = false;
+            (*it)->launch_begin = c->launch_idx;
+            (*it)->t_begin = c->gstep;
+            c->dirty = true;
+        }
+        late.erase(rest, late.end());
+    };
     int rc = FDTD_OK;
-    for (; k < pend.size() && rc == FDTD_OK; ++k) rc = run_steps_host(c, pend[k].nsteps, false);
-    for (SimHost* s : late) {
-        s->held = false;
-        s->launch_begin = c->launch_idx;
-        s->t_begin = c->gstep;
+    for (; k < pend.size() && rc == FDTD_OK; ++k) {
+        begin_now(pend[k].gstep);
+        rc = run_steps_host(c, pend[k].nsteps, false);
     }
-    if (!late.empty()) c->dirty = true;
+    begin_now(INT64_MAX);
     return rc;
 }
 
@@ -499,7 +512,6 @@ int fdtd_remove_sim(fdtd_ctx* c, int id) {
 
 int fdtd_reset_sim(fdtd_ctx* c, int id) {
     if (!c || id < 0 || id >= (int)c->sims.size() || !c->sims[id]) return fdtd_fail(FDTD_E_ARG, "bad sim id");
-    if (int rc = resolve_resident(c)) return rc;
     SimHost* s = c->sims[id];
     const size_t state0 = s->lay_off[14];   // first state sub-array (after coefficients and sources)
     HIPCHK(hipMemsetAsync((char*)s->block + state0, 0, s->bytes - state0, c->st));
@@ -556,15 +568,17 @@ static int staged_upload(fdtd_ctx* c, const std::vector<Upload>& ups) {
         c->stage_pending = false;
     }
     if (total > c->stage_cap) {
-        if (c->stage) HIPCHK(hipHostFree(c->stage));
-        c->stage = nullptr;
-        c->stage_cap = 0;
-        // the first words are the resident launches' give-up flag (resolved
-        // before a rebuild, so none is in flight here)
-        HIPCHK(hipHostMalloc(&c->stage, kStageHead + total * 2, hipHostMallocDefault));
+        // the first words are the resident launches' give-up flag: none may be
+        // in flight, and what one of them left there is kept
+        HIPCHK(hipStreamSynchronize(c->st));
+        const int32_t gave_up = c->h_rerr ? __atomic_load_n(c->h_rerr, __ATOMIC_ACQUIRE) : 0;
+        void* grown = nullptr;
+        HIPCHK(hipHostMalloc(&grown, kStageHead + total * 2, hipHostMallocDefault));
+        if (c->stage) (void)hipHostFree(c->stage);
+        c->stage = grown;
         c->stage_cap = total * 2;
         c->h_rerr = (int32_t*)c->stage;
-        *c->h_rerr = 0;
+        __atomic_store_n(c->h_rerr, gave_up, __ATOMIC_RELEASE);
     }
     if (grow) HIPCHK(hipStreamSynchronize(c->st));
     size_t off = 0;
@@ -1381,13 +1395,14 @@ static int run_resident_t(fdtd_ctx* c, int64_t n, bool* taken) {
     std::lock_guard<std::mutex> lock(g_res_mu);
     std::vector<ResUse>& use = g_res_use[c->device];
     const double share = (double)((nt + kTileWavesHost - 1) / kTileWavesHost) / (c->res_cap / kTileWavesHost);
-    double held = 0.0;
+    double held = 0.0, own = 0.0;
     for (size_t k = 0; k < use.size();) {
-        if (use[k].c == c) { use.erase(use.begin() + k); continue; }     // this stream runs its launches in turn
         const hipError_t e = hipEventQuery(use[k].done);
         if (e == hipSuccess) { use.erase(use.begin() + k); continue; }
         if (e == hipErrorNotReady) (void)hipGetLastError();
-        held += use[k].share;
+        // this stream runs its launches in turn, the largest share of them at most
+        if (use[k].c == c) own = use[k].share;
+        else held += use[k].share;
         ++k;
     }
     if (held + share > 1.0) return FDTD_OK;
@@ -1426,7 +1441,8 @@ static int run_resident_t(fdtd_ctx* c, int64_t n, bool* taken) {
     if (e != hipSuccess) return fdtd_fail(FDTD_E_HIP, std::string("resident launch: ") + hipGetErrorString(e));
     if (ev) HIPCHK(hipEventRecord(ev->second, c->st));
     HIPCHK(hipEventRecord(c->res_ev, c->st));
-    use.push_back({c, c->res_ev, share});
+    use.erase(std::remove_if(use.begin(), use.end(), [&](const ResUse& x) { return x.c == c; }), use.end());
+    use.push_back({c, c->res_ev, std::max(share, own)});
     *taken = true;
     c->box_set ^= 1;
     ResPending p{ra.ordinal, c->launch_idx, c->gstep, n, {}};
@@ -1458,8 +1474,6 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
         if (c->dirty) {
             int rc = close_bracket(c);
             if (rc) return rc;
-            rc = resolve_resident(c);
-            if (rc) return rc;
             rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
             if (rc) return rc;
         }
@@ -1487,7 +1501,9 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
                 continue;
             }
         }
+        // other launches follow the resident ones only when those have finished
         if (int rc = resolve_resident(c)) return rc;
+        if (c->dirty) continue;
         // steps this launch: S, bounded by the remaining request; one step when
         // a beam is coupled (the deposit feeds every E update)
         int n = (int)std::min<int64_t>(remaining, c->S_run);
@@ -1812,9 +1828,7 @@ int fdtd_set_persistent(fdtd_ctx* c, int on) {
 int fdtd_persistent_active(fdtd_ctx* c, int* active) {
     if (!c || !active) return fdtd_fail(FDTD_E_ARG, "null argument");
     if (c->dirty) {
-        int rc = resolve_resident(c);
-        if (rc) return rc;
-        rc = close_bracket(c);
+        int rc = close_bracket(c);
         if (rc) return rc;
         rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
         if (rc) return rc;
@@ -1838,9 +1852,7 @@ int fdtd_set_resident(fdtd_ctx* c, int on, int64_t max_wait_us) {
 int fdtd_resident_active(fdtd_ctx* c, int* active) {
     if (!c || !active) return fdtd_fail(FDTD_E_ARG, "null argument");
     if (c->dirty) {
-        int rc = resolve_resident(c);
-        if (rc) return rc;
-        rc = close_bracket(c);
+        int rc = close_bracket(c);
         if (rc) return rc;
         rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
         if (rc) return rc;
@@ -1884,9 +1896,7 @@ int fdtd_set_halo_exchange(fdtd_ctx* c, int h) {
 int fdtd_halo_exchange_active(fdtd_ctx* c, int* active) {
     if (!c || !active) return fdtd_fail(FDTD_E_ARG, "null argument");
     if (c->dirty) {
-        int rc = resolve_resident(c);
-        if (rc) return rc;
-        rc = close_bracket(c);
+        int rc = close_bracket(c);
         if (rc) return rc;
         rc = c->prec == FDTD_F64 ? rebuild_t<double>(c) : rebuild_t<float>(c);
         if (rc) return rc;

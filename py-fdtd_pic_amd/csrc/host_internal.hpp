@@ -20,7 +20,7 @@ struct SimHost {
     long long launch_begin = 0; // context launch index at admission (ping-pong parity base)
     long long t_begin = 0;      // context global step at admission
     long long steps_done = 0;
-    bool held = false;          // no part in the launches: its life began behind the ones that are run again
+    bool held = false;          // no part in the launches that are run again: its life begins behind them
     long long launches = 0;     // launches this simulation took part in
     // energy accumulator (fdtd_set_energy): H' before a launch's last H update
     // (N+1 FP64) then the recorded W values (rows FP64), one allocation

@@ -431,3 +431,46 @@ def test_resident_queue_is_bounded(fail):
         for f in got:
             same = np.array_equal(got[f], s.probes() if f == "probes" else s.read(f))
             assert same, f
+
+
+def test_reset_add_and_run_wait_for_nothing():
+    from fdtd_pic_amd import engine
+    with engine.Context("f64") as c:
+        a = c.add(_phys(65536, 40000))
+        b = c.add(_phys(2000, 40000, "none"))
+        c.run(10)
+        a.reset()
+        b.reset()
+        c.run(10)                             # the arrays that grow have grown
+        c.sync()
+        c.run(20000)
+        a.reset()
+        c.run(20000)
+        c.add(_phys(1000, 2000))
+        b.reset()
+        c.run(100)
+        assert c.resident_active() and c.resident_counts()[2] == 3 and c.busy()
+        c.sync()
+        assert c.resident_counts()[1:] == (0, 0)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("fail", [1, 2, 3, 4])
+@pytest.mark.parametrize("kind", ["reset", "all reset", "reset twice", "reset and add", "short", "blocks behind",
+                                  "beam behind"])
+def test_reset_and_add_between_runs_that_give_up(prec, fail, kind):
+    """Each of several queued runs has other simulations, or the same ones begun
+    anew: the ones that are run again have those that they had."""
+    a, b, s = ("add", _phys(5000, 500)), ("add", _phys(3000, 400, "none")), ("add", _phys(801, 120))
+    r = ("run", 64)
+    script = {
+        "reset": [a, b, r, ("reset", 0), r, r, ("reset", 1), ("run", 37)],
+        "all reset": [a, b, r, ("reset", 0), ("reset", 1), ("run", 32), ("reset", 0), ("reset", 1), r, ("run", 5)],
+        "reset twice": [a, b, r, ("reset", 0), ("reset", 0), r, ("reset", 0), r, ("run", 16)],
+        "reset and add": [a, r, b, r, ("reset", 0), s, r, ("reset", 2), ("run", 70)],
+        # simulations that end inside a run, before others begin
+        "short": [s, ("run", 300), a, ("run", 300), ("reset", 0), ("run", 300), b, ("run", 450)],
+        "blocks behind": [a, b, r, ("reset", 0), r, r, ("halo", 8), r, ("halo", 0), ("reset", 1), r],
+        "beam behind": [a, b, r, ("reset", 0), r, r, ("beam", *_beam_spec(700, 200)), ("run", 33), ("read",), ("run", 9)],
+    }[kind]
+    _plays_the_same(prec, script, fail=fail, again=None if fail < 4 else 0 if kind == "beam behind" else 1)
