@@ -474,3 +474,55 @@ def test_reset_and_add_between_runs_that_give_up(prec, fail, kind):
         "beam behind": [a, b, r, ("reset", 0), r, r, ("beam", *_beam_spec(700, 200)), ("run", 33), ("read",), ("run", 9)],
     }[kind]
     _plays_the_same(prec, script, fail=fail, again=None if fail < 4 else 0 if kind == "beam behind" else 1)
+
+
+@pytest.mark.parametrize("threads", [False, True])
+def test_resident_contexts_share_the_device(threads):
+    """A launch is taken while the tiles of all contexts' launches fit on the
+    device together; the others run one block per launch.  Same bits."""
+    from concurrent.futures import ThreadPoolExecutor
+    from fdtd_pic_amd import engine
+    big, small = _phys(65536, 30000), _phys(2000, 3000)
+    with engine.Context("f64") as a, engine.Context("f64") as b, engine.Context("f32") as d, engine.Context("f64") as e:
+        sims = [a.add(big), b.add(big), d.add(small), e.add(small)]
+        for c in (a, b, d, e):
+            assert c.resident_active()
+        if threads:
+            def go(c):
+                for _ in range(30):
+                    c.run(c is a and 1000 or 100)
+                    c.sync()
+            with ThreadPoolExecutor(4) as ex:
+                list(ex.map(go, (a, b, d, e)))
+            b.run(27000)
+        else:
+            a.run_all()
+            assert a.busy()
+            b.run(100)                        # while a's launch holds the device
+            assert b.resident_counts()[0] == 0
+            for c in (d, e):
+                c.run(100)
+            for c in (a, b, d, e):
+                c.sync()
+            b.run(100)                        # and after it
+            d.run(2900)
+            e.run(2900)
+            b.run(29800)
+            assert b.resident_counts()[0] > 0
+        got = [{f: s.read(f) for f in ("E", "H", "D", "P")} | {"probes": s.probes()} for s in sims]
+    for k, (prec, spec) in enumerate((("f64", big), ("f64", big), ("f32", small), ("f64", small))):
+        if k == 1:
+            continue
+        with engine.Context(prec) as c:
+            c.set_resident(False)
+            s = c.add(spec)
+            if prec == "f32" and threads:
+                for _ in range(30):
+                    c.run(100)
+            elif prec == "f32":
+                c.run(100)
+            c.run_all()
+            for f in got[k]:
+                want = s.probes() if f == "probes" else s.read(f)
+                same = np.array_equal(got[k][f], want) and (k > 0 or np.array_equal(got[1][f], want))
+                assert same, (k, f)
