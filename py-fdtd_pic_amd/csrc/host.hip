@@ -733,21 +733,20 @@ static int attach_t(fdtd_ctx* c, int id, SimHost& s, const fdtd_beam_desc_t* bd)
     b->range0[0] = b->cell0.front();
     b->range0[1] = b->cell0.back();
     // Cells per push/count group; the kernels loop over the groups of the live
-    // range in a grid stride.  G fixes the order of the deposit's sums, so it
-    // depends on the beam alone.  Dense beams take one-cell groups (the
-    // scalar-carry path), sparser ones groups of about 1,024 particles, which
-    // amortise the per-group work of the multi-cell path (config 4's 2,048
-    // beams: push/count 1.17 ms per step at ~96 particles per group, 0.85 ms
-    // with this rule).  FP32 from 96 particles per occupied cell (config 3,
-    // 100 per cell: 13.0 us at one cell per group, 16.9 us at four).  FP64 from
-    // 40: us per step, one cell per group against groups of 1,024, 45 per cell:
-    // 1 beam 10.8 / 16, 24 beams 38 / 57, 200 beams 328 / 286; 57 per cell: 1
-    // beam 11.2 / 16, 64 beams 70 / 88, 200 beams 233 / 234; below 40 it loses
-    // from 24 beams on (27 per cell 48.5 / 47).
+    // range in a grid stride.  G fixes the order of the deposit's sums and what
+    // a checkpoint holds, so it depends on the beam alone, and in one way.
+    // Dense beams (from 96 particles per occupied cell) take one-cell groups
+    // (the scalar-carry path), sparser ones groups of about 1,024 particles,
+    // which amortise the per-group work of the multi-cell path (config 4's
+    // 2,048 beams: push/count 1.17 ms per step at ~96 particles per group, 0.85
+    // ms with this rule; config 3, 100 per cell: 13.0 us at one cell per group,
+    // 16.9 us at four).  FP64 from 40 per cell on was tried: us per step, one
+    // cell per group against groups of 1,024, 45 per cell: 1 beam 10.8 / 16, 24
+    // beams 38 / 57, but 200 beams 328 / 286.
     int G = bd->group;
     if (G <= 0) {
         const double per_cell = occupied ? (double)n / occupied : 1.0;
-        G = per_cell >= kOneCellDensity<R> ? 1 : (int)std::lround(1024.0 / per_cell);
+        G = per_cell >= 96.0 ? 1 : (int)std::lround(1024.0 / per_cell);
     }
     b->G = std::min(std::max(G, 1), kPicGMax);
     const int span = b->range0[1] - b->range0[0] + 3;

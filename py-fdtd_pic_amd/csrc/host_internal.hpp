@@ -172,11 +172,6 @@ struct fdtd_ctx {
 
 int fdtd_fail(int code, const std::string& msg);
 
-// Particles per occupied cell from which a beam takes one-cell groups (see
-// attach_t).
-template <typename R>
-constexpr double kOneCellDensity = sizeof(R) == 4 ? 96.0 : 40.0;
-
 // Groups per CU up to which a launch's multi-cell beams take pic_push_group
 // (a workgroup per group) rather than pic_push_count (a wave per group): two
 // workgroups of it fit on a CU in FP32, one in FP64.  us per step, group

@@ -322,3 +322,39 @@ def test_plain_and_slab_beams_share_a_launch(prec):
         assert np.abs(x["J"]).max() > 0
         for k in x:
             assert np.array_equal(x[k], y[k]), k
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("per_cell", [30, 45, 60, 90])
+def test_checkpoint_of_a_beam_of_middling_density(prec, per_cell):
+    """A beam of fewer than 96 particles per occupied cell takes groups of about
+    1,024 particles, at any load: that fixes the order of the deposit's sums and
+    what a checkpoint holds, so one that was taken with such groups loads and
+    goes on with the same bits."""
+    from fdtd_pic_amd import configs, engine
+    rng = np.random.default_rng(per_cell)
+    cells, steps = 60, 80
+    x = 200.0 + np.repeat(np.arange(cells), per_cell) + rng.uniform(0.0, 1.0, cells * per_cell)
+    u = rng.normal(0.0, 0.15, (x.size, 3))
+    spec = engine.physical_spec(configs.base(700, steps, slab_start=60, slab_stop=90, src_cell=200, probes=[150, 640],
+                                             src_t0=5e-15, src_tau=2e-15, src_amp=1e6))
+
+    def start(c, group):
+        return c.add(spec, beam=engine.Beam(x, u, -configs.E_CHARGE, configs.M_ELECTRON, 1e9, configs.DT, configs.DZ,
+                                            group=group))
+
+    out = []
+    with engine.Context(prec, K=1, S=1) as c:
+        s = start(c, round(1024.0 / per_cell))
+        c.run(40)
+        blob = s.save_state()
+        c.run(40)
+        out.append([s.read("E"), s.read("J"), s.particles()[1]])
+    with engine.Context(prec, K=1, S=1) as c:
+        s = start(c, 0)
+        s.load_state(blob)
+        c.run(40)
+        out.append([s.read("E"), s.read("J"), s.particles()[1]])
+    assert np.abs(out[0][1]).max() > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
