@@ -306,14 +306,13 @@ __device__ __forceinline__ void e_pure_slab(TILE_PARAMS, const TileCtx<R>& c, co
     if constexpr (KIND == SLAB_KERR_E) kerr_fixup<R, K>(E, x, z, ied, c.chi3);
 }
 
-// psi' = b psi + c d of the CPML.  FP64 fuses b psi.  FP32 rounds as the
-// compiler fused the one-block loops: FORM < 0 leaves it to the compiler (the
-// one-block kernels themselves); a resident tile writes the fused product out:
-// b psi (0), or, where FORM is 1 and the cell is not a lane's first one in
-// the one-block tiles, c d.  Those loops fuse c d in the E half of a lane's
-// later cells at the even steps of a launch, and b psi everywhere else (read
-// from the compiled loops of K = 1, 2 and 4; the tests hold resident FP32 runs
-// to the one-block runs bit for bit).
+// psi' = b psi + c d of the CPML.  FP64 fuses b psi.  FP32 fuses it too (FORM 0),
+// except in the E half of the even steps of a block (FORM 1): there the cells
+// that are not a lane's first one in the one-block tiles fuse c d.  That is how
+// the one-block loops were first compiled; one-block and resident tiles both
+// write it out, so that a result does not depend on which of them ran (the
+// tests hold them to the same bits).  FORM < 0 leaves the choice to the
+// compiler: the halo-exchange instance, which stands alone.
 template <int FORM, typename R>
 __device__ __forceinline__ R psi_next(R b, R psi, R c, R d, bool first) {
     if constexpr (FORM < 0 || sizeof(R) == 8) {
@@ -427,7 +426,8 @@ __device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, cons
     }
     // the step body, called twice per loop trip: with two copies the
     // loop-carried registers alternate instead of being moved back each step
-    auto step = [&](const int s) {
+    auto step = [&](const int s, auto form) {
+        constexpr int FORM = decltype(form)::value;
         const int ix = s - c.s_lo;
         R Jv[K];
 #pragma unroll
@@ -458,14 +458,14 @@ __device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, cons
         if constexpr (SLAB_CODE && (MODE & M_PURE_SLAB) && !STRIP) {
             e_pure_slab<R, K, KAHAN, KIND, GEN>(TILE_ARGS, c, sd, dH, Jv);
         } else if constexpr (SLAB_CODE) {
-            e_mixed<R, K, KAHAN, KIND, STRIP, GEN>(TILE_ARGS, c, sd, dH, Jv);
+            e_mixed<R, K, KAHAN, KIND, STRIP, GEN, FORM>(TILE_ARGS, c, sd, dH, Jv);
         } else {
 #pragma unroll
             for (int j = 0; j < K; ++j) {
                 const R a = dH[j] - Jv[j];
                 if (KAHAN) kahan_fma(E[j], cE[j], a, ke[j]); else E[j] = fmr(a, ke[j], E[j]);
                 if (STRIP) {
-                    psE[j] = fmr(bE[j], psE[j], cEc[j] * dH[j]);
+                    psE[j] = psi_next<FORM>(bE[j], psE[j], cEc[j], dH[j], (c.first_mask >> j) & 1u);
                     E[j] = fmr(-CbE[j], psE[j], E[j]);
                 }
             }
@@ -494,7 +494,7 @@ __device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, cons
             const R dE = ((j == K - 1) ? Er : E[j + 1]) - E[j];
             if (KAHAN) kahan_fma(H[j], cH[j], dE, kh[j]); else H[j] = fmr(dE, kh[j], H[j]);
             if (STRIP) {
-                psH[j] = fmr(bH[j], psH[j], cHc[j] * dE);
+                psH[j] = psi_next<GROUP ? -1 : 0>(bH[j], psH[j], cHc[j], dE, true);
                 H[j] = fmr(C2H[j], psH[j], H[j]);
             }
         }
@@ -566,12 +566,14 @@ __device__ __forceinline__ void run_steps(TILE_PARAMS, const TileCtx<R>& c, cons
             }
         }
     };
+    using Even = std::integral_constant<int, GROUP ? -1 : 1>;
+    using Odd = std::integral_constant<int, GROUP ? -1 : 0>;
     int s = c.s_lo;
     for (; s + 1 < c.s_hi; s += 2) {
-        step(s);
-        step(s + 1);
+        step(s, Even{});
+        step(s + 1, Odd{});
     }
-    if (s < c.s_hi) step(s);
+    if (s < c.s_hi) step(s, Even{});
 }
 
 // Steps of a resident tile: the arithmetic of run_steps, cell by cell
@@ -754,7 +756,7 @@ __device__ __forceinline__ void tile_body(const SimDev<R>& sd, int out0_, long l
     c.wv = wv;
     c.hx = hx;
     c.emu_mask = 0;
-    c.first_mask = 0;
+    c.first_mask = RES ? 0 : 1;
     c.base = c.t0 + lane * K;
     c.N = N;
     c.T = sd.T;
