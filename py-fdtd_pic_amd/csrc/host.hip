@@ -1289,9 +1289,10 @@ static EvPair* next_event(fdtd_ctx* c, int kind) {
 // ev (profiling): ev->first is stamped at the start of the first group's
 // kernel, ev->second at the end of the last one.  With fused, the last group
 // runs in one launch with the particle scatter (stamped by fev instead).
+// block: the resident plan's tiles, n <= res_S steps.
 static int launch_once(fdtd_ctx* c, int n, EvPair* ev, hipStream_t st, bool fused = false,
-                       EvPair* fev = nullptr) {
-    if (c->blk_ok) {
+                       EvPair* fev = nullptr, bool block = false) {
+    if (c->blk_ok || block) {
         if (n > c->res_S) return fdtd_fail(FDTD_E_STATE, "a block launch of more than S steps");
         ResArgs ra{};
         ra.nsteps = n;
@@ -1477,7 +1478,20 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
             if (rc) return rc;
         }
         if (c->ntiles == 0) break;
-        if (allow_resident && res_now(c)) {
+        // A run of one block hands nothing over, so it needs no mailbox, no
+        // event and no record (where no launch ahead of it may give up): the
+        // resident tiles in a block launch, or in FP64 at K <= 2 the one-block
+        // tiles, whose kernel has less to set up.  us per run, queued, with one
+        // launch of either kind, and as a resident launch: FP64, K = 2,
+        // S = 16, 65,536 cells, 1 step 7.4 / 4.8 / 11.1, 16 steps 9.4 / 7.3 /
+        // 13.1, 32 steps 11.7 / 14.6 (two launches) / 15.4; 2,000 cells, 1 step
+        // 5.8 / 4.6 / 9.1.  FP32, K = 4, S = 32: 65,536 cells, 1 step 7.3 /
+        // 14.7 / 11.1, 32 steps 11.8 / 23.6 / 15.5; 2,000 cells, 1 step 7.1 /
+        // 9.1 / 10.7.
+        const bool resident = allow_resident && res_now(c);
+        const bool alone = resident && remaining <= c->res_S && c->res_pending.empty();
+        const bool block = alone && !(c->prec == FDTD_F64 && c->K <= 2 && remaining <= c->S_run);
+        if (resident && !alone) {
             // whole blocks of the one-block launches, unless the run ends
             const int64_t n = std::min<int64_t>(remaining, kResMaxSteps / c->S_run * c->S_run);
             int rc = close_bracket(c);
@@ -1505,7 +1519,7 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
         if (c->dirty) continue;
         // steps this launch: S, bounded by the remaining request; one step when
         // a beam is coupled (the deposit feeds every E update)
-        int n = (int)std::min<int64_t>(remaining, c->S_run);
+        int n = (int)(block ? remaining : std::min<int64_t>(remaining, c->S_run));
         // profiling samples every profile-th launch (events cost host time)
         const bool prof = c->profile > 0 && (c->launches % c->profile) == 0;
         // event handles are copied out at once: next_event may grow (move) the vector
@@ -1557,7 +1571,7 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
                 HIPCHK(hipEventRecord(b->first, c->st));
                 c->bracket = (long long)(b - c->events.data());
             }
-            rc = launch_once(c, n, nullptr, c->st);
+            rc = launch_once(c, n, nullptr, c->st, false, nullptr, block);
             if (rc) return rc;
             if (++c->events[(size_t)c->bracket].launches == c->profile) {
                 rc = close_bracket(c);
@@ -1568,7 +1582,7 @@ static int run_steps_host(fdtd_ctx* c, int64_t nsteps, bool allow_resident) {
             EvPair* ev = (prof && !(fused && c->groups.size() == 1)) ? next_event(c, FDTD_KERNEL_STENCIL) : nullptr;
             if (prof && !ev && !(fused && c->groups.size() == 1)) return FDTD_E_HIP;
             EvPair fev{e2, e3, FDTD_KERNEL_FIELD_SORT, 1};
-            rc = launch_once(c, n, ev, c->st, fused, prof ? &fev : nullptr);
+            rc = launch_once(c, n, ev, c->st, fused, prof ? &fev : nullptr, block);
             if (rc) return rc;
         }
         if (c->has_pic && !fused) {

@@ -345,7 +345,7 @@ def test_tiling_changed_behind_a_launch_that_gives_up(change):
 
 
 @pytest.mark.parametrize("prec", ["f32", "f64"])
-@pytest.mark.parametrize("cuts", [(5, 192), (37, 1, 192, 23), (96, 21, 17)])
+@pytest.mark.parametrize("cuts", [(101, 192), (69, 1, 192, 23), (96, 21, 17)])
 def test_runs_keep_their_pieces_when_run_again(prec, cuts):
     """Several queued runs, none a whole number of blocks: FP32 rounding depends
     on where a block begins."""
@@ -410,19 +410,19 @@ def test_resident_pauses_after_a_give_up():
 
 @pytest.mark.parametrize("fail", [0, 1, 700, 2900])
 def test_resident_queue_is_bounded(fail):
-    """A loop of single steps: the host keeps track of so many launches only,
+    """A loop of short runs: the host keeps track of so many launches only,
     and of the right ones when one of them gives up."""
     from fdtd_pic_amd import engine
-    spec = _phys(2000, 3000)
+    spec = _phys(2000, 300000)
     with engine.Context("f64") as c:
         s = c.add(spec)
         c.resident_fail(fail)
         most = 0
         for _ in range(3000):
-            c.run(1)
+            c.run(100)
             most = max(most, c.resident_counts()[2])
         got = {f: s.read(f) for f in ("E", "H", "D", "P")} | {"probes": s.probes()}
-        assert s.progress() == 3000 and (c.resident_counts()[1] > 0) == (fail > 0)
+        assert s.progress() == 300000 and (c.resident_counts()[1] > 0) == (fail > 0)
     assert most <= 1024
     with engine.Context("f64") as c:
         c.set_resident(False)
@@ -526,3 +526,31 @@ def test_resident_contexts_share_the_device(threads):
                 want = s.probes() if f == "probes" else s.read(f)
                 same = np.array_equal(got[k][f], want) and (k > 0 or np.array_equal(got[1][f], want))
                 assert same, (k, f)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("tiling", [None, (2, 16), (4, 48), (1, 24)])
+@pytest.mark.parametrize("fail", [0, 1])
+def test_runs_of_one_block(prec, tiling, fail):
+    """Runs that end within a block, alone and behind resident launches, one
+    of which gives up."""
+    a, b = _phys(5000, 900), _phys(3000, 400, "none")
+    b.snap_interval, b.snap_rows = 7, 40
+    script = [("tiling", *tiling)] if tiling else []
+    script += [("add", a), ("add", b)] + [("run", n) for n in (1, 1, 5, 16, 150, 1, 3, 24, 110)] + [("read",)]
+    script += [("run", n) for n in (7, 2)] + [("reset", 0), ("run", 9), ("read",), ("run", 130), ("run", 4)]
+    _plays_the_same(prec, script, fail=fail, again=None if fail else 0)
+
+
+def test_short_runs_are_no_resident_launches():
+    from fdtd_pic_amd import engine
+    for prec in ("f32", "f64"):
+        with engine.Context(prec) as c:
+            c.add(_phys(5000, 2000))
+            assert c.resident_active()
+            for _ in range(20):
+                c.run(1)
+                c.run(16)
+            assert c.resident_counts() == (0, 0, 0)
+            c.run(500)
+            assert c.resident_counts() == (1, 0, 1)
