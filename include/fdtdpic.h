@@ -125,9 +125,10 @@ int fdtd_set_tiling(fdtd_ctx *ctx, int K, int S);
  * costly slab cells then get more lanes while plain cells use fewer waves. */
 int fdtd_set_tiling_mixed(fdtd_ctx *ctx, int K, int K_slab, int S);
 /* PIC step launches: with on = 1 (the default) the particle scatter runs in
- * the same launch as the field step when that launch is small (K = 1 or 2
- * and at most 2,048 tiles; with several slab kinds in one context, the last
- * kind's launch), so a step is two launches instead of three.  A larger
+ * the same launch as the field step when that launch is not large (K = 1 or 2
+ * and at most 8,192 tiles; tiles without a Lorentz/Kerr slab join those of one
+ * slab kind, and with several kinds in one context it is the last kind's
+ * launch), so a step is two launches instead of three or four.  A larger
  * field launch keeps its own, since the fused kernel's register count (the
  * field tile's) would cut the scatter's occupancy.  0 always launches them
  * one after the other.  Results are bitwise the same either way.  No
@@ -173,11 +174,12 @@ int fdtd_resident_counts(fdtd_ctx *ctx, int64_t *launches, int64_t *again, int64
  * that gave up: the device leaves it, and those behind it, undone, and their
  * steps are run again.  For tests of that path. */
 int fdtd_resident_fail(fdtd_ctx *ctx, int nth);
-/* Request for persistent launches (on = 1) under the conditions of uniform
- * tiles with S <= 64K - 2S, one slab kind and no beam: fdtd_persistent_active
- * tells whether the next fdtd_run keeps its tiles on the device between
- * blocks of S steps under them.  Resident launches do so with or without
- * this request; the results are the same bits. */
+/* Request for persistent launches (on = 1), which have no kernel of their own:
+ * fdtd_persistent_active tells whether the next fdtd_run is resident and the
+ * tiling is uniform with S <= 64K - 2S, one slab kind and no beam (FP32 runs
+ * are resident up to S = 60 and K = 4 only, and none is with fdtd_set_resident
+ * off).  Runs are resident with or without this request, with the same bits;
+ * all it changes is that the workgroup halo exchange is off. */
 int fdtd_set_persistent(fdtd_ctx *ctx, int on);
 /* *active = 1 when the request holds for the next fdtd_run. */
 int fdtd_persistent_active(fdtd_ctx *ctx, int *active);

@@ -207,12 +207,13 @@ class Context:
         check(self.lib.fdtd_set_pic_lds_rows(self.h, int(rows)))
 
     def set_persistent(self, on=True):
-        """Persistent field launches: many blocks of S steps per launch when
-        every tile fits on the device at once (bitwise the same results)."""
+        """A request that persistent_active answers; runs are resident with or
+        without it (it only switches the halo exchange off)."""
         check(self.lib.fdtd_set_persistent(self.h, 1 if on else 0))
 
     def persistent_active(self):
-        """True when the next run() uses persistent launches."""
+        """True when the next run() is resident under uniform tiles with
+        S <= 64K - 2S and one slab kind."""
         v = C.c_int()
         check(self.lib.fdtd_persistent_active(self.h, C.byref(v)))
         return bool(v.value)
@@ -221,7 +222,8 @@ class Context:
         """Resident field launches (default on): a whole run() in one launch
         when every tile fits on the device at once (bitwise the same results).
         max_wait_us bounds one wait for a neighbour (0: 50 ms); a launch that
-        passes it is run again with one launch per S steps."""
+        passes it is run again with one launch per S steps, as are the runs of
+        the next second."""
         check(self.lib.fdtd_set_resident(self.h, 1 if on else 0, int(max_wait_us)))
 
     def resident_active(self):

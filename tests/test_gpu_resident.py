@@ -554,3 +554,25 @@ def test_short_runs_are_no_resident_launches():
             assert c.resident_counts() == (0, 0, 0)
             c.run(500)
             assert c.resident_counts() == (1, 0, 1)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_simulation_removed_behind_a_launch_that_gives_up(prec):
+    from fdtd_pic_amd import engine
+    specs = [_phys(5000, 900), _phys(3000, 400, "none"), _phys(801, 300)]
+    out = []
+    for resident in (True, False):
+        with engine.Context(prec) as c:
+            c.set_tiling(2, 16)
+            c.set_resident(resident)
+            c.resident_fail(2 if resident else 0)
+            sims = [c.add(s) for s in specs[:2]]
+            c.run(96)
+            c.run(64)
+            sims[0].remove()
+            assert c.resident_counts()[1] == (1 if resident else 0)
+            sims.append(c.add(specs[2]))
+            c.run(80)
+            out.append([s.read(f) for s in sims[1:] for f in ("E", "H", "PSIE")] + [s.probes() for s in sims[1:]])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
