@@ -436,16 +436,16 @@ def test_resident_queue_is_bounded(fail):
 def test_reset_add_and_run_wait_for_nothing():
     from fdtd_pic_amd import engine
     with engine.Context("f64") as c:
-        a = c.add(_phys(65536, 40000))
-        b = c.add(_phys(2000, 40000, "none"))
+        a = c.add(_phys(65536, 120000))
+        b = c.add(_phys(2000, 120000, "none"))
         c.run(10)
         a.reset()
         b.reset()
         c.run(10)                             # the arrays that grow have grown
         c.sync()
-        c.run(20000)
+        c.run(60000)
         a.reset()
-        c.run(20000)
+        c.run(60000)
         c.add(_phys(1000, 2000))
         b.reset()
         c.run(100)
